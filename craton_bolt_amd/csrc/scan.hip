@@ -122,41 +122,72 @@ static int scan_prepare(ScanScratch& sc, int64_t n_tiles, hipStream_t s) {
   return BOLT_OK;
 }
 
-// Gather: dst[i] = src[rows[i]].  The validity bitmap is rebuilt a wave at a
-// time (64 bits -> 8 bytes, written by the wave's first lane), so it needs no
-// clearing; a row id out of range sets *err and gathers zero.
-__global__ __launch_bounds__(256) void take_kernel(const uint8_t* __restrict__ src, const uint8_t* __restrict__ sval,
-                                                   int64_t src_len, int width, const uint32_t* __restrict__ rows,
-                                                   int64_t n, uint8_t* __restrict__ dst, uint8_t* __restrict__ dval,
+// Gather: dst[i] = src[rows[i]].  Bound by the row ids and the output streamed
+// past the random reads of src.  A workgroup covers kTakeItems stripes of 256
+// consecutive rows at a time: all row ids are loaded before the first is used
+// and all gathers before the first store, with clamped indexes instead of
+// branches, so a lane keeps kTakeItems random reads in flight.  The validity
+// bitmap is rebuilt a wave at a time (64 bits, lanes 0..7 write one byte
+// each), so it needs no clearing.  Row ids out of range and NULL row ids are
+// noted in a register and reported with one atomic per wave that saw one (an
+// atomic per such row, all on one word, took 3.55 ms for 2M NULL row ids
+// among 20M int32 rows; 0.10 ms now).
+constexpr int kTakeItems = 4;
+template <typename T>
+__global__ __launch_bounds__(256) void take_kernel(const T* __restrict__ src, const uint8_t* __restrict__ sval,
+                                                   int64_t src_len, const uint32_t* __restrict__ rows, int64_t n,
+                                                   T* __restrict__ dst, uint8_t* __restrict__ dval,
                                                    uint32_t* __restrict__ err) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t end = (n + 63) / 64 * 64;  // wave-uniform trip count for the ballot
+  constexpr int64_t kTile = 256 * kTakeItems;
+  const int lane = threadIdx.x & 63;
   const int64_t nbytes = (n + 7) / 8;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < end; i += stride) {
-    const bool in = i < n;
-    int64_t r = in ? (int64_t)rows[i] : 0;
-    const bool null_row = r == 0xFFFFFFFFll;  // the NULL index of an outer join
-    const bool ok = r < src_len && !null_row;
-    if (in && !ok) atomicOr(err, null_row ? (dval ? 0u : 2u) : 1u);
-    if (!ok) r = 0;
-    if (in) {
-      switch (width) {
-        case 1: dst[i] = ok ? src[r] : 0; break;
-        case 4: reinterpret_cast<uint32_t*>(dst)[i] = ok ? reinterpret_cast<const uint32_t*>(src)[r] : 0u; break;
-        case 8: reinterpret_cast<uint64_t*>(dst)[i] = ok ? reinterpret_cast<const uint64_t*>(src)[r] : 0ull; break;
-        case 16:
-          reinterpret_cast<uint4*>(dst)[i] = ok ? reinterpret_cast<const uint4*>(src)[r] : make_uint4(0u, 0u, 0u, 0u);
-          break;
-      }
+  uint32_t seen = 0;
+  for (int64_t base = (int64_t)blockIdx.x * kTile + threadIdx.x; base - threadIdx.x < n;
+       base += (int64_t)gridDim.x * kTile) {
+    uint32_t r[kTakeItems];
+    bool ok[kTakeItems];
+    T v[kTakeItems];
+#pragma unroll
+    for (int j = 0; j < kTakeItems; j++) {
+      const int64_t i = base + j * 256;
+      r[j] = __builtin_nontemporal_load(rows + (i < n ? i : n - 1));
+    }
+#pragma unroll
+    for (int j = 0; j < kTakeItems; j++) {
+      const bool in = base + j * 256 < n;
+      const bool null_row = r[j] == 0xFFFFFFFFu;  // the NULL index of an outer join
+      ok[j] = in && !null_row && (int64_t)r[j] < src_len;
+      if (in && !ok[j]) seen |= null_row ? (dval ? 0u : 2u) : 1u;
+      if (!ok[j]) r[j] = 0;
+    }
+    if (src_len > 0) {
+#pragma unroll
+      for (int j = 0; j < kTakeItems; j++) v[j] = src[r[j]];
+    }
+#pragma unroll
+    for (int j = 0; j < kTakeItems; j++) {
+      const int64_t i = base + j * 256;
+      if (i < n) dst[i] = ok[j] ? v[j] : T{};
     }
     if (dval) {
-      const uint64_t b = __ballot(in && ok && bit_valid(sval, r));
-      if ((threadIdx.x & 63) == 0) {
-        const int64_t b0 = i / 8;  // i is a multiple of 64 on the wave's first lane
-        for (int k = 0; k < 8 && b0 + k < nbytes; k++) dval[b0 + k] = (uint8_t)(b >> (8 * k));
+#pragma unroll
+      for (int j = 0; j < kTakeItems; j++) {
+        const uint64_t b = __ballot(ok[j] && bit_valid(sval, r[j]));
+        const int64_t byte = (base + j * 256 - lane) / 8 + lane;  // the wave's first row is a multiple of 64
+        if (lane < 8 && byte < nbytes) dval[byte] = (uint8_t)(b >> (8 * lane));
       }
     }
   }
+  const uint32_t w = (__ballot(seen & 1u) ? 1u : 0u) | (__ballot(seen & 2u) ? 2u : 0u);
+  if (w && lane == 0) atomicOr(err, w);
+}
+
+template <typename T>
+static void launch_take(const bolt_column_t* src, const uint32_t* rows, int64_t n, const bolt_column_t* dst,
+                        uint32_t* err, hipStream_t s) {
+  take_kernel<T><<<grid_for(n, 256, kTakeItems, 256 * 8), 256, 0, s>>>(
+      static_cast<const T*>(src->data), src->validity, src->length, rows, n,
+      static_cast<T*>(const_cast<void*>(dst->data)), const_cast<uint8_t*>(dst->validity), err);
 }
 
 }  // namespace bolt
@@ -268,10 +299,12 @@ extern "C" int bolt_take(bolt_stream_t stream, const bolt_column_t* src, const u
   DevBuf<uint32_t> err;
   BOLT_TRY(err.alloc(1, s));
   BOLT_TRY(fill_u32(err.ptr, 0, 1, s));
-  take_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(static_cast<const uint8_t*>(src->data), src->validity, src->length,
-                                                  width, rows, n, static_cast<uint8_t*>(const_cast<void*>(dst->data)),
-                                                  const_cast<uint8_t*>(dst->validity),
-                                                  err.ptr);
+  switch (width) {
+    case 1: launch_take<uint8_t>(src, rows, n, dst, err.ptr, s); break;
+    case 4: launch_take<uint32_t>(src, rows, n, dst, err.ptr, s); break;
+    case 8: launch_take<uint64_t>(src, rows, n, dst, err.ptr, s); break;
+    case 16: launch_take<uint4>(src, rows, n, dst, err.ptr, s); break;
+  }
   BOLT_HIP(hipGetLastError());
   uint32_t e = 0;
   BOLT_HIP(hipMemcpyAsync(&e, err.ptr, 4, hipMemcpyDeviceToHost, s));
