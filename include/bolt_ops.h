@@ -166,7 +166,8 @@ int bolt_aggregate_noalloc(bolt_stream_t stream, const bolt_column_t* inputs, in
  * *n_out (host) and synchronises the stream.  If more rows survive than the
  * smallest capacity, nothing beyond it is written, *n_out is the full count
  * and BOLT_DECLINE is returned (the capacity contract of bolt_join_probe).
- * Single pass: predicate, decoupled look-back scan and gather in one kernel.
+ * Two kernels: the predicate into one bit per row and survivor counts, then the
+ * gather, so every column is read once.
  * ------------------------------------------------------------------------ */
 int bolt_filter_compact(bolt_stream_t stream, const bolt_column_t* cols, int32_t n_cols,
                         const bolt_filter_t* filter, const uint8_t* mask, bolt_column_t* out,
