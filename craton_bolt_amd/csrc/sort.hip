@@ -13,8 +13,10 @@
 //     earlier tiles per digit for its global offsets (decoupled look-back,
 //     one digit per thread), reorders the tile by digit in LDS and writes
 //     runs of equal digits with coalesced stores;
+//   * up to 2^23 rows, and up to 2^25 where the top digits are uneven, the
+//     buckets come from a sample of the keys instead (sort_split.h);
 //   * passes whose digit is constant over the whole input are skipped;
-//   * for large inputs with three or more varying digits the sort is hybrid
+//   * for larger inputs with three or more varying digits the sort is hybrid
 //     (MSD-grouped, LSD-finished): only the two most significant varying
 //     digits get global onesweep passes; they leave up to 65536 contiguous
 //     buckets of ~n/65536 keys, which one workgroup each sorts by the
@@ -86,11 +88,17 @@ __global__ __launch_bounds__(kBins) void radix_scan_kernel(const uint32_t* __res
 
 // ---- one onesweep pass ------------------------------------------------------------
 
+// Where a pass finds a row's digit: 8 bits of the key, the low `shift` bits of
+// its 16-bit code (the code's other bits are then carried along, for the next
+// pass), or an 8-bit digit carried by the pass before.
+enum { kDigitKey = 0, kDigitCode = 1, kDigitByte = 2 };
+
+template <int SRC>
 __global__ __launch_bounds__(kSortBlock) void radix_pass_kernel(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin, uint64_t* __restrict__ kout,
     uint32_t* __restrict__ vout, int64_t n, int shift, const uint32_t* __restrict__ digit_base,
     uint32_t* __restrict__ status, uint32_t* __restrict__ ticket, uint32_t* __restrict__ err, uint64_t in_xor,
-    uint64_t out_xor) {
+    uint64_t out_xor, const void* __restrict__ din, uint8_t* __restrict__ dout) {
   __shared__ uint64_t sk[kSortTile];
   __shared__ uint32_t sv[kSortTile];
   __shared__ uint32_t wh[kSortWaves][kBins];  // per-wave digit counts, then per-wave prefixes
@@ -98,6 +106,7 @@ __global__ __launch_bounds__(kSortBlock) void radix_pass_kernel(
   __shared__ uint32_t gb[kBins];              // global base of each digit's run in this tile
   __shared__ uint32_t wtot[kSortWaves];
   __shared__ uint32_t sh_tile;
+  __shared__ uint16_t sd[SRC == kDigitKey ? 1 : kSortTile];
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (threadIdx.x == 0) sh_tile = atomicAdd(ticket, 1u);
@@ -110,6 +119,12 @@ __global__ __launch_bounds__(kSortBlock) void radix_pass_kernel(
   uint64_t key[kSortItems];
   uint32_t val[kSortItems];
   uint16_t rank[kSortItems];
+  uint16_t code[SRC == kDigitKey ? 1 : kSortItems];
+  const uint32_t dmask = SRC == kDigitCode ? (1u << shift) - 1 : kBins - 1;
+  auto digit = [&](int j) -> uint32_t {
+    if constexpr (SRC == kDigitKey) return (uint32_t)(key[j] >> shift) & (kBins - 1);
+    else return code[j] & dmask;
+  };
   // branch-free loads (clamped index) so all 2 x ITEMS loads are in flight at
   // once; out-of-range lanes become ~0 (last digit) and are never stored
 #pragma unroll
@@ -118,16 +133,19 @@ __global__ __launch_bounds__(kSortBlock) void radix_pass_kernel(
     const int64_t ic = i < n ? i : n - 1;
     key[j] = __builtin_nontemporal_load(kin + ic);
     val[j] = __builtin_nontemporal_load(vin + ic);
+    if constexpr (SRC == kDigitCode) code[j] = static_cast<const uint16_t*>(din)[ic];
+    if constexpr (SRC == kDigitByte) code[j] = static_cast<const uint8_t*>(din)[ic];
   }
 #pragma unroll
   for (int j = 0; j < kSortItems; j++) {
     const int64_t i = tbase + (int64_t)wave * 64 * kSortItems + j * 64 + lane;
     key[j] = i < n ? key[j] ^ in_xor : ~0ull;
+    if constexpr (SRC != kDigitKey) code[j] = i < n ? code[j] : (uint16_t)0xFFFF;
   }
   const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
   for (int j = 0; j < kSortItems; j++) {
-    const uint32_t d = (uint32_t)(key[j] >> shift) & (kBins - 1);
+    const uint32_t d = digit(j);
     uint64_t peers = ~0ull;
 #pragma unroll
     for (int b = 0; b < kRadixBits; b++) {
@@ -218,10 +236,11 @@ __global__ __launch_bounds__(kSortBlock) void radix_pass_kernel(
   for (int j = 0; j < kSortItems; j++) {
     int64_t i = tbase + (int64_t)wave * 64 * kSortItems + j * 64 + lane;
     if (i < n) {
-      const uint32_t d = (uint32_t)(key[j] >> shift) & (kBins - 1);
+      const uint32_t d = digit(j);
       const uint32_t pos = lex[d] + wh[wave][d] + rank[j];
       sk[pos] = key[j];
       sv[pos] = val[j];
+      if constexpr (SRC != kDigitKey) sd[pos] = code[j];
     }
   }
   __syncthreads();
@@ -231,10 +250,12 @@ __global__ __launch_bounds__(kSortBlock) void radix_pass_kernel(
     const int i = j * kSortBlock + threadIdx.x;
     if (i < valid) {
       const uint64_t k = sk[i];
-      const uint32_t d = (uint32_t)(k >> shift) & (kBins - 1);
+      const uint32_t d = SRC == kDigitKey ? (uint32_t)(k >> shift) & (kBins - 1) : sd[i] & dmask;
       const uint64_t dst = (uint64_t)gb[d] + (uint32_t)i - lex[d];
       kout[dst] = k ^ out_xor;
       vout[dst] = sv[i];
+      if constexpr (SRC == kDigitCode)
+        if (dout) dout[dst] = (uint8_t)(sd[i] >> shift);
     }
   }
 }
@@ -268,8 +289,8 @@ __device__ __forceinline__ uint32_t bucket_of(uint64_t k, int s1, int s2) {
 }
 
 // start[b] = first index whose bucket is >= b (b = 0 .. 65536); *max_size =
-// the largest bucket.  keys are sorted by bucket.
-__global__ void bucket_bounds_kernel(const uint64_t* __restrict__ keys, int64_t n, int s1, int s2,
+// the largest bucket.  keys ^ x are sorted by bucket.
+__global__ void bucket_bounds_kernel(const uint64_t* __restrict__ keys, int64_t n, uint64_t x, int s1, int s2,
                                      uint32_t* __restrict__ start, uint32_t* __restrict__ max_size) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b > kBuckets) return;
@@ -277,7 +298,7 @@ __global__ void bucket_bounds_kernel(const uint64_t* __restrict__ keys, int64_t 
     int64_t lo = 0, hi = n;
     while (lo < hi) {
       const int64_t mid = (lo + hi) >> 1;
-      if (bucket_of(keys[mid], s1, s2) < target) lo = mid + 1;
+      if (bucket_of(keys[mid] ^ x, s1, s2) < target) lo = mid + 1;
       else hi = mid;
     }
     return lo;
@@ -496,6 +517,88 @@ __global__ __launch_bounds__(kLocBlock) void local_sort_kernel(
   }
 }
 
+}  // namespace bolt
+
+#include "sort_split.h"
+
+namespace bolt {
+
+// The splitter sort of 2 <= n <= kSplitMax pairs.  *done = false when a bucket
+// of different keys exceeded the LDS sort (keys_out / vals_out then hold
+// nothing of use; the inputs are untouched).
+static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t* vals_in, int64_t n,
+                                uint64_t* keys_out, uint32_t* vals_out, uint64_t in_xor, uint64_t out_xor,
+                                bool* done) {
+  *done = true;
+  if (n <= kSplitWhole) {
+    split_whole_kernel<<<1, 1024, 0, s>>>(keys_in, vals_in, keys_out, vals_out, (int)n, in_xor, out_xor);
+    BOLT_HIP(hipGetLastError());
+    return BOLT_OK;
+  }
+  // Buckets of at most 384 rows on average (512 in one pass and above 3 << 23
+  // rows), most of which the first bucket kernel holds.
+  const bool one = n <= kSplitOnePass;
+  int cbits = one ? 6 : 9;  // 6: the splitters of one sorted list, no merge
+  while (((int64_t)(one ? 512 : 384) << cbits) < n && cbits < 16) cbits++;
+  const int C = 1 << cbits;
+  const int b1 = one ? 8 : cbits / 2;
+  const int S = cbits == 6 ? kSampleList : cbits <= 12 ? 4096 : 16384;
+  const int64_t tiles = (n + kSortTile - 1) / kSortTile;
+  DevBuf<uint64_t> sample, ktmp;
+  DevBuf<uint32_t> vtmp, words, start;
+  DevBuf<uint16_t> codes;
+  DevBuf<uint8_t> digits;
+  BOLT_TRY(sample.alloc((size_t)2 * S, s));
+  BOLT_TRY(codes.alloc((size_t)n, s));
+  // counts, scanned counts, tickets and error, then the look-back words of
+  // each pass: one fill
+  const size_t status_words = (size_t)tiles * kBins;
+  const size_t head = 512 + 514 + 6;
+  BOLT_TRY(words.alloc(head + status_words * (one ? 1 : 2), s));
+  BOLT_TRY(fill_u32(words.ptr, 0, head + status_words * (one ? 1 : 2), s));
+  uint32_t* hist = words.ptr;
+  uint32_t* offs = words.ptr + 512;
+  uint32_t* misc = offs + 514;
+  uint32_t* status = words.ptr + head;
+  const Splitters sp{S == kSampleList ? sample.ptr : sample.ptr + S, S, std::min(C, S), std::max(cbits - 14, 0)};
+  split_sample_kernel<<<S / kSampleList, kSampleList, 0, s>>>(keys_in, n, in_xor, S, sample.ptr);
+  if (S > 4096) split_merge_kernel<16><<<S / 64, 64, 0, s>>>(sample.ptr, sample.ptr + S);
+  else if (S > kSampleList) split_merge_kernel<4><<<S / 64, 64, 0, s>>>(sample.ptr, sample.ptr + S);
+  const size_t lds = (size_t)(sp.G + 1) * 8;
+  BOLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(split_code_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  split_code_kernel<<<grid_for(n, kCodeBlock, 4, sp.G > 8192 ? 256 : 512), kCodeBlock, lds, s>>>(
+      keys_in, n, in_xor, sp, b1, codes.ptr, hist);
+  split_scan_kernel<<<2, 256, 0, s>>>(hist, offs);
+  const uint32_t* starts = offs;
+  if (one) {
+    radix_pass_kernel<kDigitCode><<<(unsigned)tiles, kSortBlock, 0, s>>>(keys_in, vals_in, keys_out, vals_out, n, b1,
+                                                                        offs, status, misc, misc + 4, in_xor, out_xor,
+                                                                        codes.ptr, nullptr);
+  } else {
+    BOLT_TRY(ktmp.alloc((size_t)n, s));
+    BOLT_TRY(vtmp.alloc((size_t)n, s));
+    BOLT_TRY(digits.alloc((size_t)n, s));
+    BOLT_TRY(start.alloc((size_t)C + 1, s));
+    radix_pass_kernel<kDigitCode><<<(unsigned)tiles, kSortBlock, 0, s>>>(keys_in, vals_in, ktmp.ptr, vtmp.ptr, n, b1,
+                                                                        offs, status, misc, misc + 4, in_xor, 0,
+                                                                        codes.ptr, digits.ptr);
+    radix_pass_kernel<kDigitByte><<<(unsigned)tiles, kSortBlock, 0, s>>>(
+        ktmp.ptr, vtmp.ptr, keys_out, vals_out, n, 0, offs + 257, status + status_words, misc + 1, misc + 4, 0,
+        out_xor, digits.ptr, nullptr);
+    split_bounds_kernel<<<C / 256 + 1, 256, 0, s>>>(keys_out, n, out_xor, sp, C, start.ptr);
+    starts = start.ptr;
+  }
+  launch_bucket_sorts(keys_out, vals_out, starts, C, sp, out_xor, misc + 5, s);
+  BOLT_HIP(hipGetLastError());
+  uint32_t e[2] = {0, 0};
+  BOLT_HIP(hipMemcpyAsync(e, misc + 4, 8, hipMemcpyDeviceToHost, s));
+  BOLT_HIP(hipStreamSynchronize(s));
+  if (e[0]) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
+  *done = e[1] == 0;
+  return BOLT_OK;
+}
+
 // Sort (keys_in, vals_in) ascending by the low `key_bits` bits of
 // (key ^ in_xor), stable, writing (key image ^ out_xor, value) to keys_out /
 // vals_out.  Inputs are not modified and must not alias the outputs.
@@ -505,6 +608,22 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
   if (n >= (1ll << 30)) return set_error(BOLT_ERR_PLAN, "radix sort: %lld keys exceeds the 2^30 limit", (long long)n);
   const int passes = (key_bits + kRadixBits - 1) / kRadixBits;
   if (passes < 1 || passes > kMaxPasses) return set_error(BOLT_ERR_PLAN, "radix sort: bad key width %d", key_bits);
+  const bool grouped = getenv("BOLT_SORT_LSD") == nullptr;
+  bool split_tried = false;
+  auto split = [&](bool* done) -> int {
+    split_tried = true;
+    return split_sort_u64_pairs(s, keys_in, vals_in, n, keys_out, vals_out, in_xor, out_xor, done);
+  };
+  // Up to kSplitFirst rows the splitter sort costs no more than the digit
+  // histogram and its read-back; above, the histogram decides (30M uniform
+  // keys: 1.08 ms by digits, 1.84 ms by splitters; 1.75 ms before, with one
+  // large workgroup per bucket).
+  if (n <= kSplitFirst && grouped) {
+    bool done = false;
+    BOLT_TRY(split(&done));
+    if (done) return BOLT_OK;
+    // a bucket too large for LDS: LSD passes from the input
+  }
   DevBuf<uint32_t> hist, offs, misc;
   BOLT_TRY(hist.alloc((size_t)passes * kBins, s));
   BOLT_TRY(offs.alloc((size_t)passes * kBins, s));
@@ -538,9 +657,9 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
                   uint64_t ox) -> int {
     BOLT_TRY(fill_u32(status.ptr, 0, (size_t)tiles * kBins, s));
     BOLT_TRY(fill_u32(misc.ptr, 0, 4, s));
-    radix_pass_kernel<<<(unsigned)tiles, kSortBlock, 0, s>>>(ksrc, vsrc, kdst, vdst, n, p * kRadixBits,
-                                                             offs.ptr + (size_t)p * kBins, status.ptr, misc.ptr,
-                                                             misc.ptr + 1, ix, ox);
+    radix_pass_kernel<kDigitKey><<<(unsigned)tiles, kSortBlock, 0, s>>>(
+        ksrc, vsrc, kdst, vdst, n, p * kRadixBits, offs.ptr + (size_t)p * kBins, status.ptr, misc.ptr, misc.ptr + 1,
+        ix, ox, nullptr, nullptr);
     BOLT_HIP(hipGetLastError());
     return BOLT_OK;
   };
@@ -552,15 +671,43 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
     return BOLT_OK;
   };
   const int np = (int)todo.size();
+  if (n <= 2 * kSplitMax && grouped && !split_tried) {
+    // largest bucket of the top two varying digits if they were independent
+    double most = (double)n;
+    for (int q = np - 1; q >= 0 && q >= np - 2; q--)
+      most *= (double)*std::max_element(h.begin() + (size_t)todo[q] * kBins, h.begin() + (size_t)(todo[q] + 1) * kBins) /
+              (double)n;
+    if (np >= 3 && most <= 0.8 * kSplitMid) {
+      const int p1 = todo[np - 2], p2 = todo[np - 1];
+      BOLT_TRY(pass(keys_in, vals_in, ktmp.ptr, vtmp.ptr, p1, in_xor, 0));
+      BOLT_TRY(pass(ktmp.ptr, vtmp.ptr, keys_out, vals_out, p2, 0, out_xor));
+      DevBuf<uint32_t> starts;
+      BOLT_TRY(starts.alloc(kBuckets + 1, s));
+      BOLT_TRY(fill_u32(misc.ptr + 2, 0, 2, s));
+      bucket_bounds_kernel<<<(kBuckets + 1 + 255) / 256, 256, 0, s>>>(keys_out, n, out_xor, p1 * kRadixBits,
+                                                                    p2 * kRadixBits, starts.ptr, misc.ptr + 2);
+      BOLT_TRY(fill_u32(misc.ptr + 2, 0, 1, s));
+      launch_bucket_sorts(keys_out, vals_out, starts.ptr, kBuckets, Splitters{nullptr, 0, 0, 0}, out_xor, misc.ptr + 2, s);
+      BOLT_HIP(hipGetLastError());
+      uint32_t e[2] = {0, 0};
+      BOLT_HIP(hipMemcpyAsync(e, misc.ptr + 1, 8, hipMemcpyDeviceToHost, s));
+      BOLT_HIP(hipStreamSynchronize(s));
+      if (e[0]) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
+      if (e[1] == 0) return BOLT_OK;
+    }
+    bool done = false;
+    if (n <= kSplitMax) BOLT_TRY(split(&done));
+    if (done) return BOLT_OK;
+  }
   // hybrid: two global passes on the top varying digits, then LDS bucket sorts
-  if (np >= 3 && n >= (1 << 20) && getenv("BOLT_SORT_LSD") == nullptr) {
+  if (np >= 3 && n > kSplitMax && getenv("BOLT_SORT_LSD") == nullptr) {
     const int p1 = todo[np - 2], p2 = todo[np - 1];
     BOLT_TRY(pass(keys_in, vals_in, keys_out, vals_out, p1, in_xor, 0));
     BOLT_TRY(pass(keys_out, vals_out, ktmp.ptr, vtmp.ptr, p2, 0, 0));
     DevBuf<uint32_t> starts;
     BOLT_TRY(starts.alloc(kBuckets + 1, s));
     BOLT_TRY(fill_u32(misc.ptr + 2, 0, 2, s));
-    bucket_bounds_kernel<<<(kBuckets + 1 + 255) / 256, 256, 0, s>>>(ktmp.ptr, n, p1 * kRadixBits, p2 * kRadixBits,
+    bucket_bounds_kernel<<<(kBuckets + 1 + 255) / 256, 256, 0, s>>>(ktmp.ptr, n, 0, p1 * kRadixBits, p2 * kRadixBits,
                                                                   starts.ptr, misc.ptr + 2);
     BOLT_HIP(hipGetLastError());
     uint32_t mx[2] = {0, 0};
@@ -641,6 +788,159 @@ __global__ void order_key_kernel(const void* __restrict__ d, const uint8_t* __re
       if (bit_valid(valid, row))
         k = mode == 2 ? static_cast<const uint64_t*>(d)[2 * row + 1] ^ 0x8000000000000000ull : radix_image(d, dt, row);
       key[i] = (desc ? ~k : k) & mask;
+    }
+  }
+}
+
+// ---- multi-column ORDER BY as one sort ---------------------------------------------
+//
+// Every ORDER BY key is one or two fields (its NULL rank, its value; a
+// Decimal128 value is its signed high word, then its low word), each an
+// unsigned image that ascends along the order.  The fields' images, less their
+// smallest value, are packed most significant first into one 64-bit key, so a
+// single sort orders all columns: 0.76 ms for a nullable date and a float over
+// 5M rows, where one sort per field, each reading its column through the
+// permutation so far, took 1.25 ms (and 1.60 ms with LSD passes).  When the
+// fields need more than 64 bits the last one that fits is cut, and runs of rows
+// that agree on all 64 bits are put in order by the full columns afterwards.
+constexpr int kMaxFields = 16;
+enum { kFieldValue = 0, kFieldNull = 1, kFieldDecHigh = 2 };
+struct OrderField {
+  const void* d;
+  const uint8_t* v;
+  uint64_t min;      // smallest image of a valid row
+  int32_t dt, kind, bits, desc, nulls_first;
+  int32_t width;     // bits of the packed key
+  int32_t drop;      // low bits of the image left out of it
+};
+struct OrderFields {
+  OrderField f[kMaxFields];
+  int32_t n;
+};
+
+__device__ __forceinline__ uint64_t field_image(const OrderField& f, int64_t row) {
+  const uint64_t k = f.kind == kFieldDecHigh ? static_cast<const uint64_t*>(f.d)[2 * row + 1] ^ 0x8000000000000000ull
+                                             : radix_image(f.d, f.dt, row);
+  return (f.desc ? ~k : k) & (f.bits >= 64 ? ~0ull : (1ull << f.bits) - 1);
+}
+__device__ __forceinline__ uint64_t null_rank(const OrderField& f, int64_t row) {
+  return bit_valid(f.v, row) == (f.nulls_first != 0) ? 1 : 0;
+}
+
+// range[2 y], range[2 y + 1]: complement of the smallest image and the largest
+// image of field y's valid rows (both start at 0 and grow).
+__global__ __launch_bounds__(256) void field_range_kernel(OrderFields of, int64_t n,
+                                                          unsigned long long* __restrict__ range) {
+  const OrderField& f = of.f[blockIdx.y];
+  if (f.kind == kFieldNull) return;
+  uint64_t inv = 0, mx = 0;
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += 4 * stride) {
+    uint64_t k[4];
+    bool ok[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int64_t i = i0 + u * stride < n ? i0 + u * stride : i0;
+      ok[u] = bit_valid(f.v, i);
+      k[u] = field_image(f, i);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (ok[u]) {
+        inv = ~k[u] > inv ? ~k[u] : inv;
+        mx = k[u] > mx ? k[u] : mx;
+      }
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    const uint64_t a = __shfl_xor(inv, m), b = __shfl_xor(mx, m);
+    inv = a > inv ? a : inv;
+    mx = b > mx ? b : mx;
+  }
+  __shared__ uint64_t r[2][4];
+  if ((threadIdx.x & 63) == 0) {
+    r[0][threadIdx.x >> 6] = inv;
+    r[1][threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    uint64_t x = r[threadIdx.x][0];
+    for (int w = 1; w < 4; w++) x = r[threadIdx.x][w] > x ? r[threadIdx.x][w] : x;
+    if (x) atomicMax(&range[2 * blockIdx.y + threadIdx.x], (unsigned long long)x);
+  }
+}
+
+// key[i] = the packed fields of row i, rows[i] = i.
+__global__ __launch_bounds__(256) void pack_fields_kernel(OrderFields of, int64_t n, uint64_t* __restrict__ key,
+                                                          uint32_t* __restrict__ rows) {
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += 4 * stride) {
+    uint64_t k[4] = {0, 0, 0, 0};
+    for (int q = 0; q < of.n; q++) {
+      const OrderField& f = of.f[q];
+      if (f.width == 0) continue;  // constant, or beyond the packed bits
+      uint64_t x[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int64_t i = i0 + u * stride < n ? i0 + u * stride : i0;
+        x[u] = f.kind == kFieldNull ? null_rank(f, i)
+               : bit_valid(f.v, i)  ? (field_image(f, i) - f.min) >> f.drop
+                                    : 0ull;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) k[u] = f.width < 64 ? (k[u] << f.width) | x[u] : x[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int64_t i = i0 + u * stride;
+      if (i < n) {
+        key[i] = k[u];
+        rows[i] = (uint32_t)i;
+      }
+    }
+  }
+}
+
+// Rows that agree on the packed key, in row order: the first of each run sorts
+// it by the fields that the key does not hold whole (an insertion sort, which
+// keeps equal rows in row order).  A run above kTieRun rows sets *err.
+constexpr int kTieRun = 64;
+__device__ __forceinline__ int cmp_rows(const OrderFields& of, int first, uint32_t a, uint32_t b) {
+  for (int q = first; q < of.n; q++) {
+    const OrderField& f = of.f[q];
+    uint64_t x, y;
+    if (f.kind == kFieldNull) {
+      x = null_rank(f, a);
+      y = null_rank(f, b);
+    } else {
+      x = bit_valid(f.v, a) ? field_image(f, a) : f.min;
+      y = bit_valid(f.v, b) ? field_image(f, b) : f.min;
+    }
+    if (x != y) return x < y ? -1 : 1;
+  }
+  return 0;
+}
+__global__ __launch_bounds__(256) void tie_order_kernel(OrderFields of, int first, const uint64_t* __restrict__ key,
+                                                        int64_t n, uint32_t* __restrict__ rows,
+                                                        uint32_t* __restrict__ err) {
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i + 1 < n; i += stride) {
+    const uint64_t k = key[i];
+    if (key[i + 1] != k || (i > 0 && key[i - 1] == k)) continue;
+    int len = 2;
+    while (len <= kTieRun && i + len < n && key[i + len] == k) len++;
+    if (len > kTieRun) {
+      *err = 1u;
+      continue;
+    }
+    for (int x = 1; x < len; x++) {
+      const uint32_t r = rows[i + x];
+      int y = x - 1;
+      while (y >= 0 && cmp_rows(of, first, rows[i + y], r) > 0) {
+        rows[i + y + 1] = rows[i + y];
+        y--;
+      }
+      rows[i + y + 1] = r;
     }
   }
 }
@@ -969,6 +1269,92 @@ extern "C" int bolt_sort_pairs_i64(bolt_stream_t stream, const int64_t* keys_in,
   return BOLT_OK;
 }
 
+// ORDER BY as one sort of packed keys.  *done = false when it does not apply
+// (too many fields, or a long run of rows that agree on the packed bits only):
+// the caller then sorts field by field.
+static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys, const int32_t* descending,
+                       const int32_t* nulls_first, int64_t n, uint64_t* k0, uint64_t* k1, uint32_t* p0,
+                       uint32_t* out_rows, bool* done) {
+  OrderFields of;
+  memset(&of, 0, sizeof of);
+  int total = 0;
+  for (int k = 0; k < n_keys; k++) {
+    const bolt_column_t& c = keys[k];
+    if (of.n + 3 > kMaxFields) return BOLT_OK;
+    OrderField f;
+    memset(&f, 0, sizeof f);
+    f.d = c.data;
+    f.v = c.validity;
+    f.dt = c.dtype;
+    f.desc = descending ? descending[k] : 0;
+    f.nulls_first = nulls_first ? nulls_first[k] : 1;
+    if (c.validity) {
+      f.kind = kFieldNull;
+      f.width = f.bits = 1;
+      of.f[of.n++] = f;
+      total += 1;
+    }
+    f.bits = f.width = c.dtype == BOLT_BOOL ? 1 : c.dtype == BOLT_DEC128 ? 64 : dtype_size(c.dtype) * 8;
+    if (c.dtype == BOLT_DEC128) {
+      f.kind = kFieldDecHigh;
+      of.f[of.n++] = f;
+      total += 64;
+    }
+    f.kind = kFieldValue;
+    of.f[of.n++] = f;
+    total += f.width;
+  }
+  int cut = of.n;  // first field that the packed key does not hold whole
+  if (total > 64) {
+    // the fields' own ranges: a date, a count or the high word of a decimal
+    // needs far fewer bits than its type
+    DevBuf<unsigned long long> range;
+    unsigned long long h[2 * kMaxFields];
+    BOLT_TRY(range.alloc(2 * kMaxFields, s));
+    BOLT_TRY(fill_u32(range.ptr, 0, 4 * kMaxFields, s));
+    field_range_kernel<<<dim3(grid_for(n, 256, 4, 1024), of.n), 256, 0, s>>>(of, n, range.ptr);
+    BOLT_HIP(hipGetLastError());
+    BOLT_HIP(hipMemcpyAsync(h, range.ptr, sizeof h, hipMemcpyDeviceToHost, s));
+    BOLT_HIP(hipStreamSynchronize(s));
+    int left = 64;
+    total = 0;
+    for (int q = 0; q < of.n; q++) {
+      OrderField& f = of.f[q];
+      if (f.kind != kFieldNull) {
+        const uint64_t lo = ~(uint64_t)h[2 * q], hi = h[2 * q + 1];
+        f.min = lo <= hi ? lo : 0;  // no valid row: every image is skipped
+        const uint64_t r = lo <= hi ? hi - lo : 0;
+        f.width = r ? 64 - __builtin_clzll(r) : 0;
+      }
+      if (cut < of.n) {
+        f.width = 0;
+      } else if (f.width > left) {
+        cut = q;
+        f.drop = f.width - left;
+        f.width = left;
+      }
+      left -= f.width;
+      total += f.width;
+    }
+  }
+  pack_fields_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(of, n, k0, p0);
+  BOLT_HIP(hipGetLastError());
+  BOLT_TRY(radix_sort_u64_pairs(s, k0, p0, n, k1, out_rows, std::max(total, 1), 0, 0));
+  *done = true;
+  if (cut < of.n) {
+    DevBuf<uint32_t> err;
+    uint32_t e = 0;
+    BOLT_TRY(err.alloc(1, s));
+    BOLT_TRY(fill_u32(err.ptr, 0, 1, s));
+    tie_order_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(of, cut, k1, n, out_rows, err.ptr);
+    BOLT_HIP(hipGetLastError());
+    BOLT_HIP(hipMemcpyAsync(&e, err.ptr, 4, hipMemcpyDeviceToHost, s));
+    BOLT_HIP(hipStreamSynchronize(s));
+    *done = e == 0;
+  }
+  return BOLT_OK;
+}
+
 extern "C" int bolt_sort_indices(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys,
                                  const int32_t* descending, const int32_t* nulls_first, uint32_t* out_rows) {
   BOLT_CHECK_DEVICE();
@@ -990,6 +1376,13 @@ extern "C" int bolt_sort_indices(bolt_stream_t stream, const bolt_column_t* keys
   BOLT_TRY(k0.alloc((size_t)n, s));
   BOLT_TRY(k1.alloc((size_t)n, s));
   BOLT_TRY(p0.alloc((size_t)n, s));
+  bool done = false;
+  if (getenv("BOLT_SORT_LSD") == nullptr)
+    BOLT_TRY(sort_packed(s, keys, n_keys, descending, nulls_first, n, k0.ptr, k1.ptr, p0.ptr, out_rows, &done));
+  if (done) {
+    BOLT_HIP(hipStreamSynchronize(s));
+    return BOLT_OK;
+  }
   iota_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(out_rows, n);
   BOLT_HIP(hipGetLastError());
   // least significant key first; each step is a stable sort of the current
