@@ -239,6 +239,17 @@ struct JitCols {
   const unsigned char* v[kJitMaxCols];
 };
 
+// Key-partitioned copies of a GROUP BY's input (by value): the key columns, one
+// byte per row of key validity, and the aggregates' columns with one byte per
+// row of validity where they are nullable.
+struct GbCopies {
+  void* k0;
+  void* k1;
+  unsigned char* kv;
+  void* d[kJitMaxCols];
+  unsigned char* v[kJitMaxCols];
+};
+
 // 128-bit signed compare of (hi, lo) with (lhi, llo): -1, 0, 1
 __device__ __forceinline__ int cmp128(i64_t hi, u64_t lo, i64_t lhi, u64_t llo) {
   return hi < lhi ? -1 : hi > lhi ? 1 : (lo < llo ? -1 : lo > llo ? 1 : 0);

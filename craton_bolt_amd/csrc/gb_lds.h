@@ -23,7 +23,8 @@ struct PartOut {
   u64_t* words;         // [words][cap]
   i64_t cap;
   u64_t* count;
-  u32_t* spill;         // [grid][per] row ids: each workgroup spills into its own segment
+  u32_t* spill;         // [grid][per] row ids: each workgroup spills into its own segment; null: spilled rows
+                        // are only counted
   u64_t* spill_count;   // total spilled rows (one atomic per workgroup)
   u32_t* spill_seg;     // [grid] rows in each workgroup's segment
   i64_t per;            // segment capacity
@@ -144,13 +145,13 @@ __device__ __forceinline__ void gb_spill(bool spill, i64_t row, u64_t key, u32_t
     u32_t base = 0;
     if (lane == leader) base = atomicAdd(&sused[2], (u32_t)__popcll(m));
     base = __shfl(base, leader);
-    if (spill) {
+    if (spill && out.spill) {
       const u64_t below = lane == 0 ? 0ull : (m & (~0ull >> (64 - lane)));
       const i64_t at = (i64_t)blockIdx.x * out.per + base + (u32_t)__popcll(below);
       out.spill[at] = (u32_t)row;
       if (out.spill_key) out.spill_key[at] = key;
-      hll_add(shll, key);
     }
+    if (spill) hll_add(shll, key);
   }
 }
 
@@ -163,7 +164,7 @@ __device__ __forceinline__ void gb_lds_flush(const u64_t* skeys, const u64_t* sw
   const int SS = S + 2;
   __syncthreads();
   if (threadIdx.x == 0) {
-    out.spill_seg[blockIdx.x] = sused[2];
+    if (out.spill_seg) out.spill_seg[blockIdx.x] = sused[2];
     if (sused[2]) atomicAdd(out.spill_count, (u64_t)sused[2]);
   }
   for (int base = 0; base < SS; base += (int)blockDim.x) {

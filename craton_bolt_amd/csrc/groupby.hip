@@ -101,6 +101,148 @@ __global__ __launch_bounds__(kGbBlock) void gb_lds_kernel(KeySpec ks, DevFilter 
   gb_lds_flush(skeys, swords, S, P.words, shll, sused, out);
 }
 
+// ---- key partition: when the groups are too many for one LDS table -------------------
+//
+// Between what one workgroup's LDS table holds and what 256 of them hold, the
+// LDS tier alone spills most rows to global atomics on the table's words.
+// There the input is first copied, partitioned by the key's hash, and each of
+// 256 workgroups runs the LDS tier on one partition: no row spills, and every
+// group is complete in one workgroup.  A sample of the keys decides: it
+// estimates the group count, and a key frequent enough to leave its
+// partition's workgroup behind the others keeps the plain path, which
+// aggregates such keys in every workgroup.  10M rows of two int32 keys and two
+// float sums: 10,000 groups 1.41 -> 0.63 ms, 100,000 1.60 -> 0.96, 500,000 1.68
+// -> 1.02; 100M rows, 50,000 groups 8.6 -> 3.5 ms.  Below 2^21 rows the copy and
+// the sample's round trip cost what they save.
+
+constexpr int kGbSample = 4096;
+constexpr int kGbSampleSlots = 2 * kGbSample;
+constexpr int64_t kGbPartMinRows = (int64_t)1 << 21;
+
+// One workgroup: distinct keys among kGbSample stratified rows that pass the
+// filter.  out = {rows with a regular key, distinct keys, most frequent key's
+// rows}.
+__global__ __launch_bounds__(1024) void gb_sample_kernel(KeySpec ks, DevFilter f, int64_t n,
+                                                         uint32_t* __restrict__ out) {
+  __shared__ unsigned long long slot[kGbSampleSlots];
+  __shared__ uint32_t cnt[kGbSampleSlots];
+  __shared__ uint32_t res[3];
+  for (int i = threadIdx.x; i < kGbSampleSlots; i += 1024) {
+    slot[i] = kEmpty;
+    cnt[i] = 0;
+  }
+  if (threadIdx.x < 3) res[threadIdx.x] = 0;
+  __syncthreads();
+  uint64_t key[kGbSample / 1024];
+  int kind[kGbSample / 1024];
+#pragma unroll
+  for (int u = 0; u < kGbSample / 1024; u++) {
+    const int j = u * 1024 + threadIdx.x;
+    const int64_t lo = (int64_t)j * n / kGbSample, hi = (int64_t)(j + 1) * n / kGbSample;
+    const int64_t row = lo + (int64_t)(((uint64_t)((uint32_t)j * 0x9E3779B1u) * (uint64_t)(hi - lo)) >> 32);
+    key[u] = 0;
+    kind[u] = eval_filter(f, row) ? row_key(ks, row, &key[u]) : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < kGbSample / 1024; u++) {
+    if (kind[u] != 1 || key[u] == kEmpty) continue;
+    uint32_t s = (uint32_t)(mix64(key[u]) >> 32) & (kGbSampleSlots - 1);
+    for (;;) {  // at most half of the slots are ever taken
+      const unsigned long long prev = atomicCAS(&slot[s], kEmpty, (unsigned long long)key[u]);
+      if (prev == kEmpty || prev == key[u]) break;
+      s = (s + 1) & (kGbSampleSlots - 1);
+    }
+    atomicAdd(&cnt[s], 1u);
+  }
+  __syncthreads();
+  uint32_t rows = 0, keys = 0, most = 0;
+  for (int i = threadIdx.x; i < kGbSampleSlots; i += 1024) {
+    const uint32_t c = cnt[i];
+    rows += c;
+    keys += c ? 1u : 0u;
+    most = c > most ? c : most;
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    rows += __shfl_xor(rows, m);
+    keys += __shfl_xor(keys, m);
+    const uint32_t o = __shfl_xor(most, m);
+    most = o > most ? o : most;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(&res[0], rows);
+    atomicAdd(&res[1], keys);
+    atomicMax(&res[2], most);
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) out[threadIdx.x] = res[threadIdx.x];
+}
+
+// counts[c][p] -> first output row of chunk c's rows of partition p (rows of a
+// partition in chunk order), and ranges[p] = the partition's first row.  One
+// workgroup; thread (q, p) sums a quarter q of the chunks.
+__global__ __launch_bounds__(1024) void gb_part_offsets_kernel(uint32_t* __restrict__ counts, int chunks,
+                                                               uint32_t* __restrict__ ranges) {
+  constexpr int P = 1 << kGbPartBits;
+  static_assert(P == 256, "one thread per partition and quarter");
+  __shared__ uint32_t part[4][P];
+  __shared__ uint32_t start[P];
+  __shared__ uint32_t wtot[4];
+  const int p = threadIdx.x & (P - 1), q = threadIdx.x >> 8, lane = threadIdx.x & 63;
+  const int per = (chunks + 3) / 4;
+  const int c0 = q * per, c1 = c0 + per < chunks ? c0 + per : chunks;
+  uint32_t sum = 0;
+#pragma unroll 8
+  for (int c = c0; c < c1; c++) sum += counts[(int64_t)c * P + p];
+  part[q][p] = sum;
+  __syncthreads();
+  uint32_t tot = 0, inc = 0;
+  if (q == 0) {
+    for (int k = 0; k < 4; k++) tot += part[k][p];
+    inc = tot;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t v = __shfl_up(inc, d);
+      if (lane >= d) inc += v;
+    }
+    if (lane == 63) wtot[p >> 6] = inc;
+  }
+  __syncthreads();
+  if (q == 0) {
+    for (int w = 0; w < (p >> 6); w++) inc += wtot[w];
+    start[p] = inc - tot;
+    ranges[p] = inc - tot;
+    if (p == P - 1) ranges[P] = inc;
+  }
+  __syncthreads();
+  uint32_t at = start[p];
+  for (int k = 0; k < q; k++) at += part[k][p];
+#pragma unroll 8
+  for (int c = c0; c < c1; c++) {
+    const uint32_t v = counts[(int64_t)c * P + p];
+    counts[(int64_t)c * P + p] = at;
+    at += v;
+  }
+}
+
+// Extraction straight from the partial records, when every group has exactly
+// one: t.keys / t.words are the records (words `stride` apart).
+__global__ __launch_bounds__(256) void gb_extract_dense_kernel(GTable t, GPlan P, KeySpec ks, OutSpec o, int64_t n,
+                                                               size_t stride) {
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) {
+    const uint64_t key = t.keys[i];
+    o.packed[i] = key;
+    if (ks.n_keys == 1) {
+      write_key(o.key[0], i, key);
+    } else {
+      write_key(o.key[0], i, key >> 32);
+      write_key(o.key[1], i, key & 0xFFFFFFFFull);
+    }
+    for (int a = 0; a < P.n; a++) finalize_to(t, P.a[a], o.agg[a], stride, (uint64_t)i, (uint64_t)i);
+  }
+}
+
 // ---- pass B: global table ------------------------------------------------------------
 
 
@@ -393,19 +535,33 @@ int part_bits_delta(double est, int words) {
   return it == g_part_delta.end() ? 0 : it->second;
 }
 
-// Gather for the sorted output order: out[i] = in[perm[i]].
-__global__ void gather_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int width,
-                              const uint32_t* __restrict__ perm, int64_t n, const uint32_t* __restrict__ vsrc,
-                              uint32_t* __restrict__ vdst) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    int64_t p = perm[i];
-    switch (width) {
+// Columns of a result put in key order.  A count that only the device knows
+// is read there (n_dev), so the host need not wait for it between the
+// extraction and the ordering.
+struct OrderCols {
+  const uint8_t* src[kMaxAggs + 2];
+  uint8_t* dst[kMaxAggs + 2];
+  const uint32_t* vsrc[kMaxAggs + 2];
+  uint32_t* vdst[kMaxAggs + 2];  // zeroed bitmap words
+  int32_t width[kMaxAggs + 2];
+};
+
+// out[i] = in[perm[i]] for column blockIdx.y: all columns in one launch.
+__global__ __launch_bounds__(256) void gather_cols_kernel(OrderCols oc, const uint32_t* __restrict__ perm, int64_t n,
+                                                          const unsigned long long* __restrict__ n_dev) {
+  if (n_dev) n = (int64_t)*n_dev;
+  const int c = blockIdx.y;
+  const uint8_t* src = oc.src[c];
+  uint8_t* dst = oc.dst[c];
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
+    const int64_t p = perm[i];
+    switch (oc.width[c]) {
       case 4: reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(src)[p]; break;
       case 8: reinterpret_cast<uint64_t*>(dst)[i] = reinterpret_cast<const uint64_t*>(src)[p]; break;
       case 16: reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[p]; break;
     }
-    if (vsrc && ((vsrc[p >> 5] >> (p & 31)) & 1u)) atomicOr(&vdst[i >> 5], 1u << (i & 31));
+    if (oc.vsrc[c] && ((oc.vsrc[c][p >> 5] >> (p & 31)) & 1u)) atomicOr(&oc.vdst[c][i >> 5], 1u << (i & 31));
   }
 }
 
@@ -421,40 +577,50 @@ __global__ void flip_sign_kernel(const unsigned long long* __restrict__ in, uint
 
 // Ascending order of a few signed 64-bit keys (ties by position): the rank
 // of a key is the number of keys that precede it.  A workgroup ranks 64 keys;
-// its four waves count over interleaved quarters of all keys (staged through
-// LDS, read as broadcasts) and add their counts.  One launch and no host
-// round trip, where the radix sort needs a histogram read-back; O(n^2) work,
-// so only for small n.
-constexpr int kRankChunk = 2048;
-constexpr int64_t kRankSortMax = 4096;
-__global__ __launch_bounds__(256) void rank_sort_kernel(const unsigned long long* __restrict__ keys, int64_t n,
-                                                        uint32_t* __restrict__ perm) {
+// its 16 waves count over interleaved shares of all keys (staged through LDS,
+// read as broadcasts) and add their counts.  Keys before the workgroup's own
+// count when <=, those after when <, so only the 64 in between compare
+// positions.  One launch and no host round trip; O(n^2) work, bound by two
+// vector operations a pair, so only up to kRankSortMax keys (10,000 keys:
+// 28 us; the splitter sort's launches and read-back take about 95).
+constexpr int kRankChunk = 4096;
+constexpr int64_t kRankSortMax = 16384;
+__global__ __launch_bounds__(1024) void rank_sort_kernel(const unsigned long long* __restrict__ keys, int64_t n,
+                                                         const unsigned long long* __restrict__ n_dev,
+                                                         uint32_t* __restrict__ perm) {
   __shared__ long long sk[kRankChunk];
-  __shared__ uint32_t part[4][64];
+  __shared__ uint32_t part[16][64];
+  if (n_dev) n = (int64_t)*n_dev;
+  const int64_t i0 = (int64_t)blockIdx.x * 64;
+  if (i0 >= n) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
-  const long long ki = i < n ? (long long)keys[i] : 0;
-  uint32_t r0 = 0, r1 = 0;
+  const int64_t i = i0 + lane;
+  const long long ki = (long long)keys[i < n ? i : n - 1];
+  uint32_t r = 0;
   for (int64_t base = 0; base < n; base += kRankChunk) {
     const int m = (int)(n - base < kRankChunk ? n - base : kRankChunk);
     __syncthreads();
-    for (int j = threadIdx.x; j < m; j += 256) sk[j] = (long long)keys[base + j];
+    for (int j = threadIdx.x; j < m; j += 1024) sk[j] = (long long)keys[base + j];
     __syncthreads();
-    const int64_t li = i - base;  // position of key i relative to this chunk
-    int j = wave;
-    for (; j + 4 < m; j += 8) {
-      const long long a = sk[j], b = sk[j + 4];
-      r0 += (a < ki || (a == ki && j < li)) ? 1u : 0u;
-      r1 += (b < ki || (b == ki && j + 4 < li)) ? 1u : 0u;
-    }
-    if (j < m) {
+    const int64_t rel = i0 - base;  // the workgroup's first key in this chunk
+    const int own = rel < 0 ? 0 : (rel > m ? m : (int)rel);
+    const int after = rel < 0 ? 0 : (rel + 64 > m ? m : (int)rel + 64);
+#pragma unroll 8
+    for (int j = wave; j < own; j += 16) r += sk[j] <= ki ? 1u : 0u;
+    for (int j = own + wave; j < after; j += 16) {
       const long long a = sk[j];
-      r0 += (a < ki || (a == ki && j < li)) ? 1u : 0u;
+      r += (a < ki || (a == ki && j - (int)rel < lane)) ? 1u : 0u;
     }
+#pragma unroll 8
+    for (int j = after + wave; j < m; j += 16) r += sk[j] < ki ? 1u : 0u;
   }
-  part[wave][lane] = r0 + r1;
+  part[wave][lane] = r;
   __syncthreads();
-  if (wave == 0 && i < n) perm[part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]] = (uint32_t)i;
+  if (wave == 0 && i < n) {
+    uint32_t at = 0;
+    for (int w = 0; w < 16; w++) at += part[w][lane];
+    perm[at] = (uint32_t)i;
+  }
 }
 
 }  // namespace bolt
@@ -653,7 +819,138 @@ static int gb_jit_spec(const KeySpec& ks, const GPlan& P, const DevFilter& f, Gb
   return BOLT_OK;
 }
 
-static int lds_budget_bytes() {
+// The key-partitioned copy of an input and where its partitions start.
+struct GbPartCopy {
+  DevBuf<uint32_t> counts, ranges;
+  std::vector<DevBuf<uint8_t>> bufs;
+  KeySpec ks;          // the copied key (NULLs one byte per row)
+  GbJitSpec spec;      // the LDS tier's kernel over the copies
+  JitCols cols;
+};
+
+// Groups that a sample of m keys with d distinct ones stands for, if they are
+// about equally frequent: the G with G (1 - exp(-m / G)) = d.
+static double sample_groups(double m, double d) {
+  if (d >= m) return 1e18;
+  double lo = d, hi = 1e12;
+  for (int i = 0; i < 100; i++) {
+    const double g = std::sqrt(lo * hi);
+    if (g * -std::expm1(-m / g) < d) lo = g;
+    else hi = g;
+  }
+  return lo;
+}
+
+// Whether the input goes through the key partition (synchronises).
+static int gb_part_wanted(hipStream_t s, const KeySpec& ks, const DevFilter& f, int64_t n, int S, int part_S,
+                          bool* yes) {
+  *yes = false;
+  if (const char* e = getenv("BOLT_GB_KEY_PARTITION")) {  // testing: 0 never, 1 always
+    *yes = e[0] == '1';
+    return BOLT_OK;
+  }
+  if (n < kGbPartMinRows) return BOLT_OK;
+  DevBuf<uint32_t> out;
+  uint32_t h[3];
+  BOLT_TRY(out.alloc(4, s));
+  gb_sample_kernel<<<1, 1024, 0, s>>>(ks, f, n, out.ptr);
+  BOLT_HIP(hipGetLastError());
+  BOLT_HIP(hipMemcpyAsync(h, out.ptr, 12, hipMemcpyDeviceToHost, s));
+  BOLT_HIP(hipStreamSynchronize(s));
+  // few sampled rows pass the filter: the plain path; more groups than half
+  // of what the LDS tables hold together would spill; a key above 0.4% of the
+  // rows (its share of 1/256) would make one workgroup the last
+  const double est = sample_groups(h[0], h[1]);
+  *yes = h[0] >= kGbSample / 4 && est > 0.75 * S && est <= 0.5 * part_S * (1 << kGbPartBits) &&
+         h[2] <= 8 + h[0] / 256;
+  return BOLT_OK;
+}
+
+// Copies the rows that pass the filter, partitioned by key hash.
+static int gb_part_copy(hipStream_t s, const KeySpec& ks, const GPlan& P, const DevFilter& f, const GbJitSpec& gs,
+                        JitLits& lits, JitCols& cols, int64_t n, GbPartCopy* out, bool* ok) {
+  *ok = false;
+  std::vector<int> copied;
+  for (const GbJitSpec::Agg& a : gs.aggs)
+    if (a.col >= 0 && std::find(copied.begin(), copied.end(), a.col) == copied.end()) copied.push_back(a.col);
+  hipFunction_t fn = nullptr;
+  if (jit_get_keyed(gb_partition_jit_key(gs, copied), [&] { return jit_gb_partition_source(gs, copied); }, &fn) != BOLT_OK) {
+    clear_error();
+    return BOLT_OK;
+  }
+  const int64_t tiles = (n + kGbPartTile - 1) / kGbPartTile;
+  const int64_t per_tiles = (tiles + 511) / 512;
+  const int chunks = (int)((tiles + per_tiles - 1) / per_tiles);
+  long long per = per_tiles * kGbPartTile, nn = n;
+  const int np = 1 << kGbPartBits;
+  BOLT_TRY(out->counts.alloc((size_t)chunks * np, s));
+  BOLT_TRY(out->ranges.alloc(np + 1, s));
+  GbCopies dst;
+  memset(&dst, 0, sizeof dst);
+  auto buf = [&](size_t bytes, void** p) -> int {
+    out->bufs.emplace_back();
+    BOLT_TRY(out->bufs.back().alloc(bytes, s));
+    *p = out->bufs.back().ptr;
+    return BOLT_OK;
+  };
+  void* p = nullptr;
+  // the LDS tier over the copies: the same aggregates, no filter, and only
+  // the columns that the aggregates read
+  GbJitSpec& sp = out->spec;
+  sp = gs;
+  sp.terms.clear();
+  sp.cols.clear();
+  memset(&out->cols, 0, sizeof out->cols);
+  memset(&out->ks, 0, sizeof out->ks);
+  out->ks = ks;
+  out->ks.v0 = out->ks.v1 = nullptr;
+  const bool kv = ks.n_keys == 1 && ks.v0 != nullptr;
+  sp.kv0 = kv;
+  sp.kv1 = false;
+  if (sp.t0 == BOLT_DEC128) sp.t0 = BOLT_I64;
+  BOLT_TRY(buf((size_t)n * dtype_size(sp.t0), &p));
+  out->ks.d0 = dst.k0 = p;
+  if (ks.n_keys == 2) {
+    BOLT_TRY(buf((size_t)n * 4, &p));
+    out->ks.d1 = dst.k1 = p;
+  }
+  if (kv) {
+    BOLT_TRY(buf((size_t)n, &p));
+    dst.kv = static_cast<unsigned char*>(p);
+    out->ks.v0 = dst.kv;
+  }
+  bool any_valid = kv;
+  std::vector<int> at(gs.cols.size(), -1);
+  for (int c : copied) {
+    const JitSpec::Col& jc = gs.cols[c];
+    BOLT_TRY(buf((size_t)n * dtype_size(jc.dtype), &p));
+    dst.d[c] = p;
+    if (jc.has_valid) {
+      BOLT_TRY(buf((size_t)n, &p));
+      dst.v[c] = static_cast<unsigned char*>(p);
+      any_valid = true;
+    }
+    at[c] = (int)sp.cols.size();
+    out->cols.d[at[c]] = dst.d[c];
+    out->cols.v[at[c]] = dst.v[c];
+    sp.cols.push_back(jc);
+  }
+  for (GbJitSpec::Agg& a : sp.aggs)
+    if (a.col >= 0) a.col = at[a.col];
+  sp.vbytes = any_valid;
+  unsigned int* counts = out->counts.ptr;
+  for (int mode = 0; mode < 2; mode++) {
+    void* args[] = {&nn, &per, &mode, (void*)&ks.d0, (void*)&ks.v0, (void*)&ks.d1, (void*)&ks.v1, &lits, &cols,
+                    (void*)&counts, &dst};
+    BOLT_HIP(hipModuleLaunchKernel(fn, (unsigned)chunks, 1, 1, 1024, 1, 1, 0, s, args, nullptr));
+    if (mode == 0) gb_part_offsets_kernel<<<1, 1024, 0, s>>>(counts, chunks, out->ranges.ptr);
+  }
+  BOLT_HIP(hipGetLastError());
+  *ok = true;
+  return BOLT_OK;
+}
+
+static int lds_max_bytes() {
   static int cached = -1;
   if (cached < 0) {
     int dev = 0, v = 0;
@@ -662,6 +959,20 @@ static int lds_budget_bytes() {
       (void)hipGetLastError();
       v = 65536;
     }
+    cached = v;
+  }
+  return cached;
+}
+
+// Slots of an LDS table of W words in `budget` bytes, beside the sketch.
+static int lds_slots(int budget, int W, int most) {
+  return std::min(most, (int)((budget - (kHllRegs + 4) * 4) / (8 * (1 + W))) - 2);
+}
+
+static int lds_budget_bytes() {
+  static int cached = -1;
+  if (cached < 0) {
+    const int v = lds_max_bytes();
     int kb = 96;  // one 1024-thread workgroup per CU either way; BOLT_GB_LDS_KB overrides
     if (const char* e = getenv("BOLT_GB_LDS_KB")) {
       const int x = atoi(e);
@@ -672,9 +983,44 @@ static int lds_budget_bytes() {
   return cached;
 }
 
-extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys,
-                            const bolt_column_t* inputs, int32_t n_inputs, const bolt_agg_t* aggs, int32_t n_aggs,
-                            const bolt_filter_t* filter, uint32_t flags, bolt_table_t** out) {
+// Puts a result's columns in ascending packed-key order (src/exec/groupby.rs:800):
+// `n` groups, or at most n with the count at n_dev.  `cols` become the ordered
+// columns, owned by the table as well.
+static int order_groups(hipStream_t s, bolt_table* tbl, std::vector<bolt_column_t>& cols,
+                        const unsigned long long* packed, int64_t n, const unsigned long long* n_dev) {
+  if (n < 1) return BOLT_OK;
+  DevBuf<uint64_t> kin, kout;
+  DevBuf<uint32_t> vin, perm;
+  BOLT_TRY(perm.alloc((size_t)n, s));
+  if (n <= kRankSortMax + 2) {
+    rank_sort_kernel<<<(unsigned)((n + 63) / 64), 1024, 0, s>>>(packed, n, n_dev, perm.ptr);
+  } else {
+    BOLT_TRY(kin.alloc((size_t)n, s));
+    BOLT_TRY(kout.alloc((size_t)n, s));
+    BOLT_TRY(vin.alloc((size_t)n, s));
+    flip_sign_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(packed, kin.ptr, vin.ptr, n);
+    BOLT_TRY(radix_sort_u64_pairs(s, kin.ptr, vin.ptr, n, kout.ptr, perm.ptr, 64));
+  }
+  OrderCols oc;
+  memset(&oc, 0, sizeof oc);
+  for (size_t c = 0; c < cols.size(); c++) {
+    bolt_column_t out;
+    BOLT_TRY(table_alloc_col(tbl, cols[c].dtype, n, cols[c].validity != nullptr, s, &out));
+    oc.src[c] = static_cast<const uint8_t*>(cols[c].data);
+    oc.dst[c] = static_cast<uint8_t*>(out.data);
+    oc.vsrc[c] = reinterpret_cast<const uint32_t*>(cols[c].validity);
+    oc.vdst[c] = reinterpret_cast<uint32_t*>(const_cast<uint8_t*>(out.validity));
+    oc.width[c] = dtype_size(cols[c].dtype);
+    cols[c] = out;
+  }
+  gather_cols_kernel<<<dim3(grid_for(n, 256, 4), (unsigned)cols.size()), 256, 0, s>>>(oc, perm.ptr, n, n_dev);
+  BOLT_HIP(hipGetLastError());
+  return BOLT_OK;
+}
+
+static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys, const bolt_column_t* inputs,
+                       int32_t n_inputs, const bolt_agg_t* aggs, int32_t n_aggs, const bolt_filter_t* filter,
+                       uint32_t flags, bool try_partition, bolt_table_t** out) {
   BOLT_CHECK_DEVICE();
   clear_error();
   *out = nullptr;
@@ -729,12 +1075,14 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
 
   // ---- pass A ----
   const int W = P.words;
-  const int budget = lds_budget_bytes();
-  int S = (int)((budget - (kHllRegs + 4) * 4) / (8 * (1 + W))) - 2;
-  if (S > 4096) S = 4096;
+  int S = lds_slots(lds_budget_bytes(), W, 4096);
+  // a partition's table: as large as LDS allows, since every group of the
+  // input is in one of them
+  const int part_S = lds_slots(lds_max_bytes() - 1024, W, 8192);
   const bool use_lds = !(flags & BOLT_GROUPBY_FORCE_GLOBAL) && S >= 256 && n > 0;
   int64_t n_parts = 0, n_spill = 0;
   double est = 0;
+  bool key_parts = false;  // the input was partitioned by key
   DevBuf<unsigned long long> pkeys, pwords;
   DevBuf<uint8_t> ptag;
   DevBuf<uint32_t> spill, hll, spill_seg;
@@ -742,7 +1090,6 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
   unsigned grid = 0;
   int64_t spill_per = 0;
   if (use_lds) {
-    const size_t lds = (size_t)(S + 2) * 8 * (1 + W) + (kHllRegs + 4) * 4;
     // the per-query generated kernel when hipRTC is available, else the
     // precompiled one; rows_per_iter is what one workgroup iteration covers
     hipFunction_t gfn = nullptr;
@@ -753,24 +1100,48 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
         jit_get_keyed(gb_jit_key(gs), [&] { return jit_gb_lds_source(gs); }, &gfn) != BOLT_OK)
       gfn = nullptr;
     clear_error();
+    // more groups than one LDS table holds: the key partition first
+    GbPartCopy pc;
+    const KeySpec* pks = &ks;
+    JitCols* pcols = &gcols;
+    const uint32_t* ranges = nullptr;
+    if (gfn && try_partition) {
+      bool yes = false;
+      BOLT_TRY(gb_part_wanted(s, ks, f, n, S, part_S, &yes));
+      if (yes) BOLT_TRY(gb_part_copy(s, ks, P, f, gs, glits, gcols, n, &pc, &yes));
+      hipFunction_t pfn = nullptr;
+      if (yes && jit_get_keyed(gb_jit_key(pc.spec), [&] { return jit_gb_lds_source(pc.spec); }, &pfn) == BOLT_OK) {
+        gfn = pfn;
+        gs = pc.spec;
+        pks = &pc.ks;
+        pcols = &pc.cols;
+        ranges = pc.ranges.ptr;
+      }
+      clear_error();
+    }
+    key_parts = ranges != nullptr;
+    if (key_parts) S = part_S;
+    const size_t lds = (size_t)(S + 2) * 8 * (1 + W) + (kHllRegs + 4) * 4;
     const int64_t rows_per_iter = (int64_t)kGbBlock * (gfn ? gs.unroll : 1);
     if (!gfn)
       BOLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gb_lds_kernel),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    grid = grid_for(n, kGbBlock, 16, 256);
+    grid = key_parts ? 1u << kGbPartBits : grid_for(n, kGbBlock, 16, 256);
     const int64_t pcap = (int64_t)grid * (S + 2);
     // a workgroup handles at most ceil(n / (grid * rows_per_iter)) iterations
     spill_per = (n + (int64_t)grid * rows_per_iter - 1) / ((int64_t)grid * rows_per_iter) * rows_per_iter;
     BOLT_TRY(pkeys.alloc((size_t)pcap, s));
     BOLT_TRY(ptag.alloc((size_t)pcap, s));
     BOLT_TRY(pwords.alloc((size_t)pcap * (W > 0 ? W : 1), s));
-    BOLT_TRY(spill.alloc((size_t)grid * spill_per, s));
-    BOLT_TRY(spill_seg.alloc(grid, s));
+    if (!key_parts) {  // partitions do not spill; if one does after all, the plain path runs instead
+      BOLT_TRY(spill.alloc((size_t)grid * spill_per, s));
+      BOLT_TRY(spill_seg.alloc(grid, s));
+    }
     // inputs large enough for the partitioned tier: the spilled rows' keys are
     // captured beside the row ids (8 bytes more per spilled row, from a
     // register), so that tier's histogram and first scatter read them in
     // order instead of gathering them by row id
-    if (n > ((int64_t)1 << 25)) BOLT_TRY(spill_key.alloc((size_t)grid * spill_per, s));
+    if (n > ((int64_t)1 << 25) && !key_parts) BOLT_TRY(spill_key.alloc((size_t)grid * spill_per, s));
     // sketch registers and the two counters in one buffer: one read-back
     BOLT_TRY(hll.alloc(kHllRegs + 4, s));
     BOLT_TRY(fill_u32(hll.ptr, 0, kHllRegs + 4, s));
@@ -781,7 +1152,8 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
     if (gfn) {
       long long nn = n;
       int SSz = S;
-      void* args[] = {&nn, &SSz, (void*)&ks.d0, (void*)&ks.v0, (void*)&ks.d1, (void*)&ks.v1, &glits, &gcols, &po};
+      void* args[] = {&nn, &SSz, (void*)&pks->d0, (void*)&pks->v0, (void*)&pks->d1, (void*)&pks->v1, &glits, pcols, &po,
+                      (void*)&ranges};
       BOLT_HIP(hipModuleLaunchKernel(gfn, grid, 1, 1, kGbBlock, 1, 1, (unsigned)lds, s, args, nullptr));
     } else {
       gb_lds_kernel<<<grid, kGbBlock, lds, s>>>(ks, f, P, n, S, po);
@@ -796,6 +1168,8 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
     n_parts = (int64_t)hc[0];
     n_spill = (int64_t)hc[1];
     est = hll_estimate(regs.data());
+    if (key_parts && n_spill > 0)  // more groups than the sample promised
+      return groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags, false, out);
   } else {
     n_spill = n;  // every row goes to the global table
     est = (double)n;
@@ -845,17 +1219,29 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
   DevBuf<uint32_t> slot_of;
   int64_t n_groups = 0;
   int st = BOLT_OK;
+  const bool sorted = (flags & BOLT_GROUPBY_SORTED) != 0;
+  const bool clash = ks.null_group && (keys[0].dtype == BOLT_I64 || keys[0].dtype == BOLT_DEC128);
+  bool ordered = false;
+  // every group in exactly one partial record: no table, the records are the groups
+  const bool dense = key_parts && !ks.null_group && !has_var;
   for (int attempt = 0;; attempt++) {
-    BOLT_TRY(tkeys.alloc(cap, s));
-    BOLT_TRY(twords.alloc((cap + 2) * (W > 0 ? W : 1), s));
     BOLT_TRY(fill_u32(tmisc.ptr, 0, 8, s));
-    t.keys = tkeys.ptr;
-    t.words = twords.ptr;
     t.used_special = tmisc.ptr;
     t.err = tmisc.ptr + 4;
-    t.cap = cap;
-    gb_init_kernel<<<grid_for((int64_t)cap + 2, 256, 1), 256, 0, s>>>(t, P);
-    if (partitioned) {
+    if (dense) {
+      t.keys = pkeys.ptr;
+      t.words = pwords.ptr;
+      t.cap = (uint64_t)n_parts;
+    } else {
+      BOLT_TRY(tkeys.alloc(cap, s));
+      BOLT_TRY(twords.alloc((cap + 2) * (W > 0 ? W : 1), s));
+      t.keys = tkeys.ptr;
+      t.words = twords.ptr;
+      t.cap = cap;
+      gb_init_kernel<<<grid_for((int64_t)cap + 2, 256, 1), 256, 0, s>>>(t, P);
+    }
+    if (dense) {
+    } else if (partitioned) {
       BOLT_TRY(gb_part_reduce(s, t, P, parts, S));
     } else if (n_parts > 0) {
       if (est < 0.75 * (double)S && n_parts > 4096) {
@@ -866,7 +1252,7 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlds));
         gb_merge_lds_kernel<<<mgrid, kGbBlock, mlds, s>>>(t, P, pkeys.ptr, ptag.ptr, pwords.ptr,
                                                           (int64_t)pkeys.count, n_parts, S);
-      } else {
+      } else {  // also the key partition's records, one per group and workgroup
         gb_merge_parts_kernel<<<grid_for(n_parts, 256, 4), 256, 0, s>>>(t, P, pkeys.ptr, ptag.ptr, pwords.ptr,
                                                                         (int64_t)pkeys.count, n_parts);
       }
@@ -884,12 +1270,13 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
     if (has_var && n > 0) gb_m2_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(t, P, ks, f, n);
     BOLT_HIP(hipGetLastError());
 
-    const uint64_t total = cap + 2;
+    const uint64_t total = t.cap + 2;
     const int64_t out_cap = (int64_t)std::min<uint64_t>(total, (uint64_t)std::max<int64_t>(upper, 0) + 2);
     tbl = new bolt_table();
     tbl->stream = s;
     OutSpec o;
     memset(&o, 0, sizeof o);
+    ordered = false;
     for (int k = 0; k < n_keys && st == BOLT_OK; k++) {
       st = table_alloc_col(tbl, keys[k].dtype, out_cap, k == 0 && ks.null_group, s, &cols[k]);
       cols[k].scale = keys[k].scale;
@@ -910,6 +1297,8 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
     }
     o.packed = packed.ptr;
     o.slot_of = slot_of.ptr;
+    if (dense && n_parts > 0)
+      gb_extract_dense_kernel<<<grid_for(n_parts, 256, 1), 256, 0, s>>>(t, P, ks, o, n_parts, (size_t)pkeys.count);
     const bool small = total <= (1u << 20);
     const int64_t per_tile = (int64_t)kExBlock * (small ? 1 : kExItems);
     const int64_t tiles = (int64_t)((total + per_tile - 1) / per_tile);
@@ -921,12 +1310,23 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
       return st;
     }
     uint32_t* emisc = reinterpret_cast<uint32_t*>(status.ptr + tiles);
-    if (small)
+    if (dense) {
+    } else if (small)
       gb_extract_kernel<1><<<(unsigned)tiles, kExBlock, 0, s>>>(t, P, ks, o, status.ptr, emisc,
                                                                reinterpret_cast<unsigned long long*>(emisc + 2));
     else
       gb_extract_kernel<kExItems><<<(unsigned)tiles, kExBlock, 0, s>>>(
           t, P, ks, o, status.ptr, emisc, reinterpret_cast<unsigned long long*>(emisc + 2));
+    // A table small enough for the rank sort is put in order before the host
+    // learns the group count: one wait for both.
+    if (sorted && !clash && total <= (uint64_t)kRankSortMax) {
+      if ((st = order_groups(s, tbl, cols, packed.ptr, dense ? n_parts : (int64_t)total,
+                             dense ? nullptr : reinterpret_cast<const unsigned long long*>(emisc + 2))) != BOLT_OK) {
+        bolt_table_release(tbl);
+        return st;
+      }
+      ordered = true;
+    }
     hipError_t le = hipGetLastError();
     uint32_t eh[4] = {0, 0, 0, 0}, terr[4] = {0, 0, 0, 0};
     if (le == hipSuccess) le = hipMemcpyAsync(eh, emisc, 16, hipMemcpyDeviceToHost, s);
@@ -944,7 +1344,7 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
       cap *= 4;
       continue;
     }
-    n_groups = (int64_t)(((uint64_t)eh[3] << 32) | eh[2]);
+    n_groups = dense ? n_parts : (int64_t)(((uint64_t)eh[3] << 32) | eh[2]);
     if (terr[1]) {
       bolt_table_release(tbl);
       return set_error(BOLT_ERR_OTHER, "GROUP BY extraction look-back timed out");
@@ -960,7 +1360,7 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
     break;
   }
 
-  if (ks.null_group && (keys[0].dtype == BOLT_I64 || keys[0].dtype == BOLT_DEC128) && n_groups >= 2) {
+  if (clash && n_groups >= 2) {
     DevBuf<int64_t> clash;
     int64_t hc[2] = {-1, 0};
     st = clash.alloc(2, s);
@@ -994,32 +1394,8 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
   }
 
   // ---- ordering by packed key (src/exec/groupby.rs:800) ----
-  if ((flags & BOLT_GROUPBY_SORTED) && n_groups > 1) {
-    DevBuf<uint64_t> kin, kout;
-    DevBuf<uint32_t> vin, perm;
-    st = perm.alloc((size_t)n_groups, s);
-    if (st == BOLT_OK && n_groups > kRankSortMax) {
-      st = kin.alloc((size_t)n_groups, s);
-      if (st == BOLT_OK) st = kout.alloc((size_t)n_groups, s);
-      if (st == BOLT_OK) st = vin.alloc((size_t)n_groups, s);
-    }
-    if (st == BOLT_OK && n_groups <= kRankSortMax) {
-      rank_sort_kernel<<<(unsigned)((n_groups + 63) / 64), 256, 0, s>>>(packed.ptr, n_groups, perm.ptr);
-    } else if (st == BOLT_OK) {
-      flip_sign_kernel<<<grid_for(n_groups, 256, 4), 256, 0, s>>>(packed.ptr, kin.ptr, vin.ptr, n_groups);
-      st = radix_sort_u64_pairs(s, kin.ptr, vin.ptr, n_groups, kout.ptr, perm.ptr, 64);
-    }
-    for (size_t c = 0; c < cols.size() && st == BOLT_OK; c++) {
-      bolt_column_t sorted;
-      st = table_alloc_col(tbl, cols[c].dtype, n_groups, cols[c].validity != nullptr, s, &sorted);
-      if (st != BOLT_OK) break;
-      gather_kernel<<<grid_for(n_groups, 256, 4), 256, 0, s>>>(
-          static_cast<const uint8_t*>(cols[c].data), static_cast<uint8_t*>(sorted.data), dtype_size(cols[c].dtype),
-          perm.ptr, n_groups, reinterpret_cast<const uint32_t*>(cols[c].validity),
-          reinterpret_cast<uint32_t*>(const_cast<uint8_t*>(sorted.validity)));
-      cols[c] = sorted;
-    }
-    if (st == BOLT_OK && hipGetLastError() != hipSuccess) st = set_error(BOLT_ERR_DEVICE, "GROUP BY gather failed");
+  if (sorted && n_groups > 1 && !ordered) {
+    st = order_groups(s, tbl, cols, packed.ptr, n_groups, nullptr);
     if (st == BOLT_OK && hipStreamSynchronize(s) != hipSuccess) st = set_error(BOLT_ERR_DEVICE, "GROUP BY sort failed");
     if (st != BOLT_OK) {
       bolt_table_release(tbl);
@@ -1031,6 +1407,13 @@ extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int
   tbl->n_rows = n_groups;
   *out = tbl;
   return BOLT_OK;
+}
+
+extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys,
+                            const bolt_column_t* inputs, int32_t n_inputs, const bolt_agg_t* aggs, int32_t n_aggs,
+                            const bolt_filter_t* filter, uint32_t flags, bolt_table_t** out) {
+  return groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags,
+                     !(flags & BOLT_GROUPBY_FORCE_PARTITIONED), out);
 }
 
 extern "C" int bolt_groupby_last_plan(int32_t* tier, int64_t* spilled_rows, int64_t* partial_records,

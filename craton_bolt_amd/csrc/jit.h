@@ -51,6 +51,7 @@ struct GbJitSpec {
     int w, nw;  // first word, count word (-1 = none)
   };
   int unroll = 8;  // rows per lane per block iteration (1..8)
+  bool vbytes = false;  // validity is one byte per row (key-partitioned copies), not a bitmap
   int n_keys = 1;
   int t0 = 0, t1 = 0;
   bool kv0 = false, kv1 = false;
@@ -83,6 +84,11 @@ int jit_get(const std::string& src, hipFunction_t* fn);
 int jit_spec_from(const DevFilter& f, const AggList& aggs, bool probe, int key_dtype, bool key_valid, int carry_dtype,
                   JitSpec* sp, JitLits* lits, JitCols* cols);
 std::string jit_gb_lds_source(const GbJitSpec& sp);
+// Key partition of a GROUP BY's input: digit counts and the copy itself.
+constexpr int kGbPartBits = 8;
+constexpr int kGbPartTile = 4096;
+std::string jit_gb_partition_source(const GbJitSpec& sp, const std::vector<int>& copied);
+std::string gb_partition_jit_key(const GbJitSpec& sp, const std::vector<int>& copied);
 // Partitioned join: the filtered scatter of the probe side into per-partition
 // runs, and the region-ordered probe + aggregate over those runs.
 std::string jit_jp_scatter_source(const JpJitSpec& sp);

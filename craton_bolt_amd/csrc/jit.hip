@@ -354,7 +354,7 @@ std::string jit_row_agg_key(const JitSpec& sp) {
 
 std::string gb_jit_key(const GbJitSpec& sp) {
   std::ostringstream k;
-  k << "gb:" << sp.unroll << ':' << sp.n_keys << ':' << sp.t0 << ':' << sp.t1 << ':' << sp.kv0 << sp.kv1 << ':'
+  k << "gb:" << sp.vbytes << sp.unroll << ':' << sp.n_keys << ':' << sp.t0 << ':' << sp.t1 << ':' << sp.kv0 << sp.kv1 << ':'
     << sp.words << '|';
   for (unsigned long long v : sp.ident) k << v << ',';
   k << '|';
@@ -737,44 +737,36 @@ std::string jit_jp_probe_source(const JitSpec& sp, int runs) {
 // so R rows' HBM reads are in flight per lane instead of one.  Slot lookup,
 // spilling and the flush are the shared gb_lds.h helpers; the accumulator
 // updates are the same LDS atomics as update_slot, specialised to the plan.
-std::string jit_gb_lds_source(const GbJitSpec& sp) {
-  std::ostringstream o;
-  const int R = sp.unroll;
-  const int W = sp.words;
-  o << kJitPrelude << "\n";
-  o << "extern \"C\" __global__ void __launch_bounds__(1024) bolt_jit_kernel(\n"
-       "    long long n, int S, const void* __restrict__ k0p, const unsigned char* __restrict__ k0v,\n"
-       "    const void* __restrict__ k1p, const unsigned char* __restrict__ k1v, bolt::JitLits lits,\n"
-       "    bolt::JitCols cols, bolt::PartOut out) {\n"
-       "  using namespace bolt;\n"
-       "  extern __shared__ u64_t sm[];\n"
-       "  const int SS = S + 2;\n"
-       "  u64_t* skeys = sm;\n"
-       "  u64_t* swords = sm + SS;\n"
-       "  u32_t* shll = (u32_t*)(swords + (u64_t)" << W << " * SS);\n"
-       "  u32_t* sused = shll + kHllRegs;\n"
-       "  for (int i = threadIdx.x; i < SS; i += 1024) {\n"
-       "    skeys[i] = kEmpty;\n";
-  for (int w = 0; w < W; w++) o << "    swords[" << w << " * SS + i] = " << sp.ident[w] << "ull;\n";
-  o << "  }\n"
-       "  for (int i = threadIdx.x; i < kHllRegs; i += 1024) shll[i] = 0;\n"
-       "  if (threadIdx.x < 4) sused[threadIdx.x] = 0;\n"
-       "  __syncthreads();\n";
-  auto kty = [](int dt) { return dtype_size(dt) == 4 ? "u32_t" : "u64_t"; };
+namespace {
+
+// Validity of row `i` in a GROUP BY kernel: a bitmap, or a byte per row.
+std::string gb_valid(const GbJitSpec& sp, const std::string& v, const std::string& i) {
+  return sp.vbytes ? "(" + v + "[" + i + "] != 0)" : "vbit(" + v + ", " + i + ")";
+}
+
+const char* gb_key_type(int dt) { return dtype_size(dt) == 4 ? "u32_t" : "u64_t"; }
+
+// Typed pointers of the key columns (k0, k1) and the column set.
+void emit_gb_ptrs(std::ostringstream& o, const GbJitSpec& sp) {
+  o << "  const " << gb_key_type(sp.t0) << "* __restrict__ k0 = (const " << gb_key_type(sp.t0) << "*)k0p;\n";
+  if (sp.n_keys == 2)
+    o << "  const " << gb_key_type(sp.t1) << "* __restrict__ k1 = (const " << gb_key_type(sp.t1) << "*)k1p;\n";
+  emit_col_ptrs(o, sp.cols);
+}
+
+// Rows base + r * stride (r < R) below n: every load first, then each row's
+// predicate, canonical packed key (key<r>) and kind<r> (0 drop, 1 regular key,
+// 2 the NULL group).
+void emit_gb_rows(std::ostringstream& o, const GbJitSpec& sp, int R, int stride) {
+  auto kty = gb_key_type;
   auto kcanon = [](int dt, const std::string& v) -> std::string {
     if (dt == BOLT_F32) return "(u64_t)canon_f32_bits(" + v + ")";
     if (dt == BOLT_F64) return "canon_f64_bits(" + v + ")";
     return "(u64_t)" + v;
   };
-  o << "  const " << kty(sp.t0) << "* __restrict__ k0 = (const " << kty(sp.t0) << "*)k0p;\n";
-  if (sp.n_keys == 2) o << "  const " << kty(sp.t1) << "* __restrict__ k1 = (const " << kty(sp.t1) << "*)k1p;\n";
-  emit_col_ptrs(o, sp.cols);
-  o << "  const long long tile = 1024LL * " << R << ";\n"
-       "  const long long end = ((n + tile - 1) / tile) * tile;  // wave-uniform trip count\n"
-       "  for (long long base = (long long)blockIdx.x * tile + threadIdx.x; base < end; base += (long long)gridDim.x * tile) {\n";
   for (int r = 0; r < R; r++) {
     const std::string rs = std::to_string(r), i = "i" + rs, j = "j" + rs;
-    o << "    const long long " << i << " = base + " << 1024 * r << ";\n"
+    o << "    const long long " << i << " = base + " << stride * r << ";\n"
       << "    const bool in" << rs << " = " << i << " < n;\n"
       << "    const long long " << j << " = in" << rs << " ? " << i << " : n - 1;  // clamped: loads stay branch-free\n"
       << "    const " << kty(sp.t0) << " ka" << rs << " = __builtin_nontemporal_load(k0 + "
@@ -800,17 +792,54 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
     // 0 drop, 1 regular key, 2 the NULL group (single nullable key)
     if (sp.n_keys == 1) {
       o << "    const u64_t key" << rs << " = " << kcanon(sp.t0, "ka" + rs) << ";\n";
-      if (sp.kv0) o << "    const int kind" << rs << " = keep" << rs << " ? (vbit(k0v, " << i << ") ? 1 : 2) : 0;\n";
+      if (sp.kv0) o << "    const int kind" << rs << " = keep" << rs << " ? (" << gb_valid(sp, "k0v", i) << " ? 1 : 2) : 0;\n";
       else o << "    const int kind" << rs << " = keep" << rs << " ? 1 : 0;\n";
     } else {
       o << "    const u64_t key" << rs << " = (" << kcanon(sp.t0, "ka" + rs) << " << 32) | " << kcanon(sp.t1, "kb" + rs)
         << ";\n";
       std::string kv = "keep" + rs;
-      if (sp.kv0) kv += " && vbit(k0v, " + i + ")";
-      if (sp.kv1) kv += " && vbit(k1v, " + i + ")";
+      if (sp.kv0) kv += " && " + gb_valid(sp, "k0v", i);
+      if (sp.kv1) kv += " && " + gb_valid(sp, "k1v", i);
       o << "    const int kind" << rs << " = (" << kv << ") ? 1 : 0;\n";
     }
   }
+}
+
+}  // namespace
+
+std::string jit_gb_lds_source(const GbJitSpec& sp) {
+  std::ostringstream o;
+  const int R = sp.unroll;
+  const int W = sp.words;
+  o << kJitPrelude << "\n";
+  o << "extern \"C\" __global__ void __launch_bounds__(1024) bolt_jit_kernel(\n"
+       "    long long n, int S, const void* __restrict__ k0p, const unsigned char* __restrict__ k0v,\n"
+       "    const void* __restrict__ k1p, const unsigned char* __restrict__ k1v, bolt::JitLits lits,\n"
+       "    bolt::JitCols cols, bolt::PartOut out, const unsigned int* __restrict__ ranges) {\n"
+       "  using namespace bolt;\n"
+       "  extern __shared__ u64_t sm[];\n"
+       "  const int SS = S + 2;\n"
+       "  u64_t* skeys = sm;\n"
+       "  u64_t* swords = sm + SS;\n"
+       "  u32_t* shll = (u32_t*)(swords + (u64_t)" << W << " * SS);\n"
+       "  u32_t* sused = shll + kHllRegs;\n"
+       "  for (int i = threadIdx.x; i < SS; i += 1024) {\n"
+       "    skeys[i] = kEmpty;\n";
+  for (int w = 0; w < W; w++) o << "    swords[" << w << " * SS + i] = " << sp.ident[w] << "ull;\n";
+  o << "  }\n"
+       "  for (int i = threadIdx.x; i < kHllRegs; i += 1024) shll[i] = 0;\n"
+       "  if (threadIdx.x < 4) sused[threadIdx.x] = 0;\n"
+       "  __syncthreads();\n";
+  emit_gb_ptrs(o, sp);
+  // every row, the workgroups taking tiles in turn; or, with `ranges`, workgroup
+  // b the rows [ranges[b], ranges[b + 1])
+  o << "  const long long tile = 1024LL * " << R << ";\n"
+       "  const long long lo = ranges ? (long long)ranges[blockIdx.x] : 0;\n"
+       "  if (ranges) n = (long long)ranges[blockIdx.x + 1];\n"
+       "  const long long step = ranges ? tile : (long long)gridDim.x * tile;\n"
+       "  const long long end = lo + ((n - lo + tile - 1) / tile) * tile;  // wave-uniform trip count\n"
+       "  for (long long base = lo + (ranges ? 0 : (long long)blockIdx.x * tile) + threadIdx.x; base < end; base += step) {\n";
+  emit_gb_rows(o, sp, R, 1024);
   // home slots of all R rows read together (one LDS round trip); the rows
   // found at home, the common case once the table is warm, skip the probe loop
   for (int r = 0; r < R; r++) {
@@ -875,7 +904,8 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
             break;
         }
       }
-      if (sp.cols[g.col].has_valid) o << "        if (vbit(v" << g.col << ", " << i << ")) { " << u.str() << " }\n";
+      if (sp.cols[g.col].has_valid)
+        o << "        if (" << gb_valid(sp, "v" + std::to_string(g.col), i) << ") { " << u.str() << " }\n";
       else o << "        " << u.str() << "\n";
     }
     o << "      }\n"
@@ -902,6 +932,145 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
   o << "  gb_lds_flush(skeys, swords, S, " << W << ", shll, sused, out);\n"
        "}\n";
   return o.str();
+}
+
+// Key partition of a GROUP BY's input.  Workgroup c walks chunk c (rows
+// [c * per, (c + 1) * per)) in tiles of kGbPartTile rows; a row that passes the
+// filter goes to the partition of the top 8 bits of its key's hash (a row of
+// the NULL group to any, by its position).  mode 0: counts[c][p] = rows of the
+// chunk in partition p.  mode 1: `counts` holds where the chunk's rows of each
+// partition start, and the columns are copied there, in row order: a tile is
+// ranked per partition in LDS, and each column in turn is staged in LDS in
+// partition order and written as runs.  Bound by the copies' traffic: no
+// atomics outside LDS, no look-back, and the layout does not depend on timing.
+std::string jit_gb_partition_source(const GbJitSpec& sp, const std::vector<int>& copied) {
+  std::ostringstream o;
+  const int R = kGbPartTile / 1024;
+  const int P = 1 << kGbPartBits;
+  bool flags = sp.n_keys == 1 && sp.kv0;
+  for (int c : copied) flags |= sp.cols[c].has_valid;
+  o << kJitPrelude << "\n";
+  o << "extern \"C\" __global__ void __launch_bounds__(1024) bolt_jit_kernel(\n"
+       "    long long n, long long per, int mode, const void* __restrict__ k0p, const unsigned char* __restrict__ k0v,\n"
+       "    const void* __restrict__ k1p, const unsigned char* __restrict__ k1v, bolt::JitLits lits,\n"
+       "    bolt::JitCols cols, unsigned int* __restrict__ counts, bolt::GbCopies dst) {\n"
+       "  using namespace bolt;\n"
+       "  __shared__ u64_t st[" << kGbPartTile << "];\n"
+       "  __shared__ unsigned char sdig[" << kGbPartTile << "];\n"
+       "  __shared__ u32_t cnt[" << P << "], pre[" << P << "], off[" << P << "], run[" << P << "], wtot[" << P / 64 << "];\n"
+       "  const int t = threadIdx.x, lane = t & 63;\n";
+  emit_gb_ptrs(o, sp);
+  o << "  const long long lo = (long long)blockIdx.x * per;\n"
+       "  if (n > lo + per) n = lo + per;\n"
+       "  if (t < " << P << ") { cnt[t] = 0; off[t] = mode ? counts[(long long)blockIdx.x * " << P << " + t] : 0; }\n"
+       "  __syncthreads();\n"
+       "  for (long long t0 = lo; t0 < n; t0 += " << kGbPartTile << ") {\n"
+       "    const long long base = t0 + t;\n";
+  emit_gb_rows(o, sp, R, 1024);
+  for (int r = 0; r < R; r++) {
+    const std::string rs = std::to_string(r);
+    o << "    const int p" << rs << " = kind" << rs << " == 0 ? -1 : (int)((kind" << rs << " == 2 ? (u64_t)i" << rs
+      << " * 0x9E3779B97F4A7C15ull : fmix64(key" << rs << ")) >> " << 64 - kGbPartBits << ");\n";
+  }
+  o << "    if (mode == 0) {\n";
+  for (int r = 0; r < R; r++) o << "      if (p" << r << " >= 0) atomicAdd(&cnt[p" << r << "], 1u);\n";
+  o << "      continue;\n    }\n";
+  for (int r = 0; r < R; r++)
+    o << "    const u32_t rank" << r << " = p" << r << " >= 0 ? atomicAdd(&cnt[p" << r << "], 1u) : 0u;\n";
+  o << "    __syncthreads();\n"
+       "    u32_t c_ = 0, inc_ = 0;\n"
+       "    if (t < " << P << ") {\n"
+       "      c_ = inc_ = cnt[t];\n"
+       "      for (int d = 1; d < 64; d <<= 1) { const u32_t x_ = __shfl_up(inc_, d); if (lane >= d) inc_ += x_; }\n"
+       "      if (lane == 63) wtot[t >> 6] = inc_;\n"
+       "    }\n"
+       "    __syncthreads();\n"
+       "    if (t < " << P << ") {\n"
+       "      for (int w = 0; w < (t >> 6); w++) inc_ += wtot[w];\n"
+       "      pre[t] = inc_ - c_;\n"
+       "      run[t] = off[t] - (inc_ - c_);  // output row of tile position j in this partition: run + j\n"
+       "      off[t] += c_;\n"
+       "      cnt[t] = 0;\n"
+       "    }\n"
+       "    __syncthreads();\n"
+       "    u32_t total = 0;\n"
+       "    for (int w = 0; w < " << P / 64 << "; w++) total += wtot[w];\n";
+  for (int r = 0; r < R; r++)
+    o << "    const u32_t at" << r << " = p" << r << " >= 0 ? pre[p" << r << "] + rank" << r << " : 0u;\n"
+      << "    if (p" << r << " >= 0) sdig[at" << r << "] = (unsigned char)p" << r << ";\n";
+  // One staged column: values in, barrier, runs out.  The first one finds the
+  // output rows of this lane's tile positions, which the others share.
+  bool first = true;
+  auto column = [&](const std::function<std::string(int)>& val, const std::string& store) {
+    for (int r = 0; r < R; r++) o << "    if (p" << r << " >= 0) st[at" << r << "] = " << val(r) << ";\n";
+    o << "    __syncthreads();\n";
+    for (int r = 0; r < R; r++) {
+      const std::string j = "(t + " + std::to_string(1024 * r) + ")";
+      if (first) o << "    const u32_t to" << r << " = (u32_t)" << j << " < total ? run[sdig[" << j << "]] + " << j << " : 0u;\n";
+      std::string stmt = store;
+      for (size_t at; (at = stmt.find("$to")) != std::string::npos;) stmt.replace(at, 3, "to" + std::to_string(r));
+      for (size_t at; (at = stmt.find("$v")) != std::string::npos;) stmt.replace(at, 2, "st[" + j + "]");
+      o << "    if ((u32_t)" << j << " < total) { " << stmt << " }\n";
+    }
+    o << "    __syncthreads();\n";
+    first = false;
+  };
+  auto ptr = [](int dt) -> std::string {
+    return dtype_size(dt) == 1 ? "unsigned char" : dtype_size(dt) == 4 ? "u32_t" : "u64_t";
+  };
+  auto rr = [](int r) { return std::to_string(r); };
+  column([&](int r) { return "(u64_t)ka" + rr(r); }, "((" + ptr(sp.t0 == BOLT_DEC128 ? (int)BOLT_I64 : sp.t0) + "*)dst.k0)[$to] = (" +
+         ptr(sp.t0 == BOLT_DEC128 ? (int)BOLT_I64 : sp.t0) + ")$v;");
+  if (sp.n_keys == 2) column([&](int r) { return "(u64_t)kb" + rr(r); }, "((u32_t*)dst.k1)[$to] = (u32_t)$v;");
+  for (int c : copied) {
+    const int dt = sp.cols[c].dtype;
+    const std::string cs = std::to_string(c), d = "dst.d[" + cs + "]";
+    auto x = [&](int r) { return "x" + cs + "_" + rr(r); };
+    if (dt == BOLT_DEC128) {
+      column([&](int r) { return x(r) + "_lo"; }, "((u64_t*)" + d + ")[2 * (u64_t)$to] = $v;");
+      column([&](int r) { return x(r) + "_hi"; }, "((u64_t*)" + d + ")[2 * (u64_t)$to + 1] = $v;");
+    } else {
+      auto bits = [&](int r) -> std::string {
+        if (dt == BOLT_F64) return "(u64_t)__double_as_longlong(" + x(r) + ")";
+        if (dt == BOLT_F32) return "(u64_t)__float_as_uint(" + x(r) + ")";
+        return "(u64_t)" + x(r);
+      };
+      column(bits, "((" + ptr(dt) + "*)" + d + ")[$to] = (" + ptr(dt) + ")$v;");
+    }
+  }
+  if (flags) {  // every validity bit of a row in one staged word
+    auto bits = [&](int r) -> std::string {
+      std::string e = "0ull";
+      const std::string i = "i" + rr(r);
+      if (sp.n_keys == 1 && sp.kv0) e += " | (kind" + rr(r) + " == 1 ? 1ull : 0ull)";
+      for (int c : copied)
+        if (sp.cols[c].has_valid)
+          e += " | (" + gb_valid(sp, "v" + std::to_string(c), i) + " ? " + std::to_string(2ull << c) + "ull : 0ull)";
+      return e;
+    };
+    std::string store;
+    if (sp.n_keys == 1 && sp.kv0) store += "dst.kv[$to] = (unsigned char)($v & 1); ";
+    for (int c : copied)
+      if (sp.cols[c].has_valid)
+        store += "dst.v[" + std::to_string(c) + "][$to] = (unsigned char)(($v >> " + std::to_string(c + 1) + ") & 1); ";
+    column(bits, store);
+  }
+  o << "  }\n"
+       "  __syncthreads();\n"
+       "  if (mode == 0 && t < " << P << ") counts[(long long)blockIdx.x * " << P << " + t] = cnt[t];\n"
+       "}\n";
+  return o.str();
+}
+
+std::string gb_partition_jit_key(const GbJitSpec& sp, const std::vector<int>& copied) {
+  std::ostringstream k;
+  k << "gbp:" << sp.n_keys << ':' << sp.t0 << ':' << sp.t1 << ':' << sp.kv0 << sp.kv1 << '|';
+  for (const JitSpec::Col& c : sp.cols) k << c.dtype << (c.has_valid ? 'v' : 'n') << ',';
+  k << '|';
+  for (const JitSpec::Term& t : sp.terms) k << t.col << '.' << t.op << ',';
+  k << '|';
+  for (int c : copied) k << c << ',';
+  return k.str();
 }
 
 int jit_row_agg_col(const void* d, const uint8_t* v, int dt, std::vector<JitSpec::Col>* cols, JitCols* jc) {

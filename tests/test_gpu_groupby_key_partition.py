@@ -1,0 +1,104 @@
+"""GROUP BY through the key partition (BOLT_GB_KEY_PARTITION=1 takes it at any
+size): every key form, NULL keys and inputs, filters, every aggregate, row
+counts around the partition's tiles and chunks, and inputs with more groups
+than the partitions' LDS tables hold (the plain path runs instead), against
+the oracle with test_gpu_groupby's comparisons and tolerances."""
+import numpy as np
+import pytest
+
+from craton_bolt_amd import _native as N
+from craton_bolt_amd.ops import Term
+
+from gpu_util import dec_array
+from test_gpu_groupby import run_both
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def forced(monkeypatch):
+    monkeypatch.setenv("BOLT_JIT", "1")
+    monkeypatch.setenv("BOLT_GB_KEY_PARTITION", "1")
+
+
+def _key(kind, n, groups, rng):
+    g = rng.integers(0, groups, n)
+    if kind == "i64":
+        k = g * 0x9E3779B97F4A7 - 1  # the empty marker (-1) among them
+        return [(k.astype(np.int64), N.I64, None)], [N.I64]
+    if kind == "i32":
+        return [((g * 7919 - 1).astype(np.int32), N.I32, None)], [N.I32]
+    if kind == "date":
+        return [(g.astype(np.int32), N.DATE32, None)], [N.DATE32]
+    if kind == "f64":
+        k = g.astype(np.float64) - 3.0
+        k[g == 1] = np.nan
+        k[(g == 3) & (rng.random(n) < 0.5)] = -0.0
+        return [(k, N.F64, None)], [N.F64]
+    if kind == "f32":
+        return [(g.astype(np.float32), N.F32, None)], [N.F32]
+    if kind == "dec":
+        return [(dec_array([int(x) - 5 for x in g]), N.DEC128, None)], [N.DEC128]
+    if kind == "null_i32":
+        return [(g.astype(np.int32), N.I32, rng.random(n) > 0.3)], [N.I32]
+    a, b = (g % 50).astype(np.int32), (g // 50).astype(np.int32)
+    if kind == "null_pair":
+        return [(a, N.I32, rng.random(n) > 0.2), (b, N.I32, rng.random(n) > 0.2)], [N.I32, N.I32]
+    return [(a, N.I32, None), (b, N.I32, None)], [N.I32, N.I32]
+
+
+@pytest.mark.parametrize("n", [1, 4095, 4097, 100_003])
+@pytest.mark.parametrize("kind", ["i64", "i32", "date", "f64", "f32", "null_i32", "pair", "null_pair"])
+def test_key_forms(gpu, n, kind):
+    print(f"[case] key partition {kind} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    keys, kdt = _key(kind, n, max(2, n // 9), rng)
+    v = rng.integers(-1000, 1000, n).astype(np.int64)
+    x = rng.normal(size=n)
+    run_both(keys, [(v, N.I64, None), (x, N.F64, rng.random(n) > 0.2)],
+             [(N.SUM, 0), (N.COUNT_STAR, 0), (N.MIN, 0), (N.MAX, 1), (N.SUM, 1), (N.COUNT, 1)], kdt)
+
+
+@pytest.mark.parametrize("n", [60_001])
+def test_aggregates_and_filter(gpu, n):
+    rng = np.random.default_rng(5)
+    keys, kdt = _key("i32", n, 4000, rng)
+    i32 = rng.integers(-100, 100, n).astype(np.int32)
+    f32 = rng.normal(size=n).astype(np.float32)
+    dec = dec_array([int(x) for x in rng.integers(-10 ** 12, 10 ** 12, n)])
+    f64 = rng.normal(size=n) + 10.0
+    va = rng.random(n) > 0.1
+    ins = [(i32, N.I32, va), (f32, N.F32, None), (dec, N.DEC128, va), (f64, N.F64, va)]
+    print("[case] key partition aggregates", flush=True)
+    run_both(keys, ins, [(N.SUM, 0), (N.AVG, 0), (N.MAX, 1), (N.SUM, 2), (N.COUNT, 2), (N.MIN, 3), (N.COUNT_STAR, 0)],
+             kdt, terms=[Term(3, N.GT, 9.5), Term(0, N.LT, 50)])
+    print("[case] key partition variance", flush=True)
+    run_both(keys, [(f64, N.F64, va)], [(N.VAR_SAMP, 0), (N.STDDEV_POP, 0), (N.AVG, 0)], kdt)
+    print("[case] key partition keys only", flush=True)
+    run_both(keys, [(i32, N.I32, None)], [], kdt)
+
+
+def test_no_row_passes(gpu):
+    rng = np.random.default_rng(6)
+    keys, kdt = _key("i64", 10_000, 500, rng)
+    run_both(keys, [(np.ones(10_000), N.F64, None)], [(N.SUM, 0)], kdt, terms=[Term(0, N.GT, 2.0)])
+
+
+def test_more_groups_than_the_tables(gpu):
+    """Every row its own group: partitions overflow, the plain path takes over."""
+    n = 1_500_000
+    print("[case] key partition overflow", flush=True)
+    k = np.random.default_rng(7).permutation(n).astype(np.int64)
+    run_both([(k, N.I64, None)], [(k.astype(np.float64), N.F64, None)], [(N.SUM, 0), (N.COUNT_STAR, 0)], [N.I64])
+
+
+@pytest.mark.parametrize("groups", [9_000, 300_000])
+def test_chosen_by_the_sample(gpu, monkeypatch, groups):
+    """Large enough to be chosen without the switch: the same result."""
+    monkeypatch.delenv("BOLT_GB_KEY_PARTITION")
+    n = 2_500_000
+    print(f"[case] key partition sampled groups={groups}", flush=True)
+    rng = np.random.default_rng(groups)
+    k = rng.integers(0, groups, n).astype(np.int32)
+    v = rng.integers(0, 1000, n).astype(np.int64)
+    run_both([(k, N.I32, None)], [(v, N.I64, None)], [(N.SUM, 0), (N.MIN, 0)], [N.I32])
