@@ -513,8 +513,12 @@ static int bolt::aggregate_impl(hipStream_t s, const bolt_column_t* inputs, int3
     }
   }
   Acc host[kMaxAggs];
-  BOLT_HIP(hipMemcpyAsync(host, outs_p, sizeof(Acc) * n_aggs, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  if (scratch) {  // allocates nothing, host memory included
+    BOLT_HIP(hipMemcpyAsync(host, outs_p, sizeof(Acc) * n_aggs, hipMemcpyDeviceToHost, s));
+    BOLT_HIP(hipStreamSynchronize(s));
+  } else {
+    BOLT_TRY(read_back(s, {{host, outs_p, sizeof(Acc) * n_aggs}}));
+  }
   bolt_scalar_t res[kMaxAggs];
   for (int i = 0; i < n_aggs; i++) BOLT_TRY(acc_finalize(host[i], all.a[i].op, all.a[i].dtype, &res[i]));
   for (int gi = 0; gi < n_guards; gi++) {

@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <string>
 
 #include "../../include/bolt_ops.h"
@@ -92,6 +93,18 @@ struct DevBuf {
     return p;
   }
 };
+
+// Small results the host waits for: copies every part (whole 4-byte words of
+// device memory) and waits for the stream.  One kernel stores all parts into
+// page-locked memory that the calling thread keeps, so a read-back costs a
+// launch and one wait; each hipMemcpyAsync into ordinary memory blocks for a
+// staged copy of its own (about 20 us on the host).
+struct ReadPart {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+int read_back(hipStream_t s, std::initializer_list<ReadPart> parts);
 
 // Graph-capture-safe fill (a kernel, never hipMemsetAsync).
 int fill_u32(void* dst, uint32_t value, size_t n_words, hipStream_t s);

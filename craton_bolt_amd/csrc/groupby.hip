@@ -855,8 +855,7 @@ static int gb_part_wanted(hipStream_t s, const KeySpec& ks, const DevFilter& f, 
   BOLT_TRY(out.alloc(4, s));
   gb_sample_kernel<<<1, 1024, 0, s>>>(ks, f, n, out.ptr);
   BOLT_HIP(hipGetLastError());
-  BOLT_HIP(hipMemcpyAsync(h, out.ptr, 12, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{h, out.ptr, 12}}));
   // few sampled rows pass the filter: the plain path; more groups than half
   // of what the LDS tables hold together would spill; a key above 0.4% of the
   // rows (its share of 1/256) would make one workgroup the last
@@ -1067,8 +1066,7 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     dec_key_fit_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(static_cast<const uint64_t*>(keys[0].data),
                                                           keys[0].validity, n, err.ptr);
     BOLT_HIP(hipGetLastError());
-    BOLT_HIP(hipMemcpyAsync(&h, err.ptr, 4, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{&h, err.ptr, 4}}));
     if (h)
       return set_error(BOLT_DECLINE, "GROUP BY on a Decimal128 key with values beyond 64 bits (the host path takes it)");
   }
@@ -1161,8 +1159,7 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     prof_end(s);
     BOLT_HIP(hipGetLastError());
     std::vector<uint32_t> regs(kHllRegs + 4);
-    BOLT_HIP(hipMemcpyAsync(regs.data(), hll.ptr, (kHllRegs + 4) * 4, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{regs.data(), hll.ptr, (kHllRegs + 4) * 4}}));
     unsigned long long hc[2];
     memcpy(hc, regs.data() + kHllRegs, 16);
     n_parts = (int64_t)hc[0];
@@ -1329,10 +1326,8 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     }
     hipError_t le = hipGetLastError();
     uint32_t eh[4] = {0, 0, 0, 0}, terr[4] = {0, 0, 0, 0};
-    if (le == hipSuccess) le = hipMemcpyAsync(eh, emisc, 16, hipMemcpyDeviceToHost, s);
-    if (le == hipSuccess) le = hipMemcpyAsync(terr, t.err, 16, hipMemcpyDeviceToHost, s);
-    if (le == hipSuccess) le = hipStreamSynchronize(s);
-    if (le != hipSuccess) {
+    st = le == hipSuccess ? read_back(s, {{eh, emisc, 16}, {terr, t.err, 16}}) : BOLT_ERR_DEVICE;
+    if (st != BOLT_OK) {
       bolt_table_release(tbl);
       return set_error(BOLT_ERR_DEVICE, "GROUP BY extraction failed: %s", hipGetErrorString(le));
     }

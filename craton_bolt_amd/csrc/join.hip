@@ -890,9 +890,7 @@ extern "C" int bolt_join_probe_aggregate(bolt_stream_t stream, const bolt_join_t
   }
   Acc host[kMaxAggs];
   uint32_t fl[2];
-  BOLT_HIP(hipMemcpyAsync(host, outs.ptr, sizeof(Acc) * n_aggs, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipMemcpyAsync(fl, t->flags, 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{host, outs.ptr, sizeof(Acc) * n_aggs}, {fl, t->flags, 8}}));
   if (fl[1] != 0) return set_error(BOLT_ERR_OTHER, "hash join build lost %u rows (table full)", fl[1]);
   for (int i = 0; i < n_aggs; i++) BOLT_TRY(acc_finalize(host[i], all.a[i].op, all.a[i].dtype, &results[i]));
   return BOLT_OK;
@@ -945,10 +943,7 @@ static int probe_emit(hipStream_t s, const bolt_join_table_t* t, const bolt_colu
   }
   unsigned long long total = 0;
   uint32_t fl[2], hm[2];
-  BOLT_HIP(hipMemcpyAsync(&total, counter.ptr, 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipMemcpyAsync(fl, t->flags, 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipMemcpyAsync(hm, misc.ptr, 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{&total, counter.ptr, 8}, {fl, t->flags, 8}, {hm, misc.ptr, 8}}));
   if (fl[1] != 0) return set_error(BOLT_ERR_OTHER, "hash join build lost %u rows (table full)", fl[1]);
   if (hm[1] != 0) return set_error(BOLT_ERR_OTHER, "hash join probe: output offset look-back timed out");
   *total_out = (int64_t)total;

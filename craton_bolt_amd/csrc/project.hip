@@ -733,8 +733,7 @@ extern "C" int bolt_aggregate_expr(bolt_stream_t stream, const bolt_column_t* in
     BOLT_TRY(launch_finish(na, parts.ptr, (int)grid, n_aggs, first, agg_chunk(all, first, na), outs.ptr + first, s));
   }
   Acc host[kMaxAggs];
-  BOLT_HIP(hipMemcpyAsync(host, outs.ptr, sizeof(Acc) * n_aggs, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{host, outs.ptr, sizeof(Acc) * n_aggs}}));
   for (int i = 0; i < n_aggs; i++) BOLT_TRY(acc_finalize(host[i], all.a[i].op, all.a[i].dtype, &results[i]));
   return BOLT_OK;
 }

@@ -331,6 +331,94 @@ int dev_free(void* p, hipStream_t s) {
   return BOLT_OK;
 }
 
+// ---- read-backs -------------------------------------------------------------
+
+namespace {
+constexpr size_t kReadBackBytes = (size_t)72 << 10;
+constexpr int kReadBackParts = 4;
+struct ReadParts {
+  const uint32_t* src[kReadBackParts];
+  uint32_t words[kReadBackParts];
+  int n;
+};
+
+__global__ __launch_bounds__(256) void read_back_kernel(ReadParts p, uint32_t* __restrict__ host) {
+  for (int k = 0; k < p.n; k++) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < p.words[k]; i += gridDim.x * 256) host[i] = p.src[k][i];
+    host += p.words[k];
+  }
+}
+
+// Page-locked buffers of ended threads, for the next thread that needs one: at
+// most as many as threads that read back at the same time.  Never freed (a
+// thread may end after the HIP runtime).
+struct PinnedPool {
+  std::mutex mu;
+  std::vector<uint32_t*> idle;
+};
+PinnedPool& pinned_pool() {
+  static PinnedPool* p = new PinnedPool;
+  return *p;
+}
+struct PinnedBuffer {
+  uint32_t* p = nullptr;
+  ~PinnedBuffer() {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(pinned_pool().mu);
+    pinned_pool().idle.push_back(p);
+  }
+  uint32_t* get() {
+    if (p) return p;
+    {
+      std::lock_guard<std::mutex> lk(pinned_pool().mu);
+      if (!pinned_pool().idle.empty()) {
+        p = pinned_pool().idle.back();
+        pinned_pool().idle.pop_back();
+        return p;
+      }
+    }
+    void* m = nullptr;
+    if (hipHostMalloc(&m, kReadBackBytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    return p = static_cast<uint32_t*>(m);
+  }
+};
+thread_local PinnedBuffer t_pinned;
+}  // namespace
+
+int read_back(hipStream_t s, std::initializer_list<ReadPart> parts) {
+  size_t total = 0;
+  bool whole = parts.size() <= (size_t)kReadBackParts;
+  for (const ReadPart& r : parts) {
+    total += r.bytes;
+    whole = whole && (r.bytes & 3) == 0 && (reinterpret_cast<uintptr_t>(r.src) & 3) == 0;
+  }
+  uint32_t* host = whole && total <= kReadBackBytes ? t_pinned.get() : nullptr;
+  if (!host) {
+    for (const ReadPart& r : parts) BOLT_HIP(hipMemcpyAsync(r.dst, r.src, r.bytes, hipMemcpyDeviceToHost, s));
+    BOLT_HIP(hipStreamSynchronize(s));
+    return BOLT_OK;
+  }
+  ReadParts p;
+  memset(&p, 0, sizeof p);
+  for (const ReadPart& r : parts) {
+    p.src[p.n] = static_cast<const uint32_t*>(r.src);
+    p.words[p.n++] = (uint32_t)(r.bytes / 4);
+  }
+  read_back_kernel<<<grid_for((int64_t)total / 4, 256, 4, 64), 256, 0, s>>>(p, host);
+  BOLT_HIP(hipGetLastError());
+  BOLT_HIP(hipStreamSynchronize(s));
+  const uint32_t* h = host;
+  for (const ReadPart& r : parts) {
+    memcpy(r.dst, h, r.bytes);
+    h += r.bytes / 4;
+  }
+  return BOLT_OK;
+}
+
 // ---- fill kernels (graph-capture safe) ----------------------------------------
 
 __global__ void fill_u32_kernel(uint32_t* __restrict__ dst, uint32_t v, size_t n) {

@@ -491,8 +491,7 @@ extern "C" int bolt_filter_compact(bolt_stream_t stream, const bolt_column_t* co
                                                    sc.total());
   BOLT_HIP(hipGetLastError());
   unsigned long long total = 0;
-  BOLT_HIP(hipMemcpyAsync(&total, sc.total(), 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{&total, sc.total(), 8}}));
   *n_out = (int64_t)total;
   if (*n_out > gl.cap)
     return set_error(BOLT_DECLINE, "bolt_filter_compact: %lld rows survive, the outputs hold %lld",
@@ -519,8 +518,7 @@ extern "C" int bolt_prefix_scan_mask(bolt_stream_t stream, const uint8_t* mask, 
                                                    sc.total());
   BOLT_HIP(hipGetLastError());
   unsigned long long total = 0;
-  BOLT_HIP(hipMemcpyAsync(&total, sc.total(), 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{&total, sc.total(), 8}}));
   *total_out = (int64_t)total;
   return BOLT_OK;
 }
@@ -552,8 +550,7 @@ extern "C" int bolt_take(bolt_stream_t stream, const bolt_column_t* src, const u
   }
   BOLT_HIP(hipGetLastError());
   uint32_t e = 0;
-  BOLT_HIP(hipMemcpyAsync(&e, err.ptr, 4, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{&e, err.ptr, 4}}));
   if (e & 1u) return set_error(BOLT_ERR_PLAN, "bolt_take: a row id is out of range (source has %lld rows)",
                                (long long)src->length);
   if (e & 2u) return set_error(BOLT_ERR_PLAN, "bolt_take: a NULL row id needs a destination validity bitmap");

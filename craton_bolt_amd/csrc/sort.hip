@@ -592,8 +592,7 @@ static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const ui
   launch_bucket_sorts(keys_out, vals_out, starts, C, sp, out_xor, misc + 5, s);
   BOLT_HIP(hipGetLastError());
   uint32_t e[2] = {0, 0};
-  BOLT_HIP(hipMemcpyAsync(e, misc + 4, 8, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{e, misc + 4, 8}}));
   if (e[0]) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
   *done = e[1] == 0;
   return BOLT_OK;
@@ -633,8 +632,7 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
   radix_scan_kernel<<<passes, kBins, 0, s>>>(hist.ptr, offs.ptr);
   BOLT_HIP(hipGetLastError());
   std::vector<uint32_t> h((size_t)passes * kBins);
-  BOLT_HIP(hipMemcpyAsync(h.data(), hist.ptr, h.size() * 4, hipMemcpyDeviceToHost, s));
-  BOLT_HIP(hipStreamSynchronize(s));
+  BOLT_TRY(read_back(s, {{h.data(), hist.ptr, h.size() * 4}}));
   std::vector<int> todo;
   for (int p = 0; p < passes; p++) {
     bool trivial = false;
@@ -665,8 +663,7 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
   };
   auto check_lookback = [&]() -> int {
     uint32_t e = 0;
-    BOLT_HIP(hipMemcpyAsync(&e, misc.ptr + 1, 4, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{&e, misc.ptr + 1, 4}}));
     if (e) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
     return BOLT_OK;
   };
@@ -690,8 +687,7 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
       launch_bucket_sorts(keys_out, vals_out, starts.ptr, kBuckets, Splitters{nullptr, 0, 0, 0}, out_xor, misc.ptr + 2, s);
       BOLT_HIP(hipGetLastError());
       uint32_t e[2] = {0, 0};
-      BOLT_HIP(hipMemcpyAsync(e, misc.ptr + 1, 8, hipMemcpyDeviceToHost, s));
-      BOLT_HIP(hipStreamSynchronize(s));
+      BOLT_TRY(read_back(s, {{e, misc.ptr + 1, 8}}));
       if (e[0]) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
       if (e[1] == 0) return BOLT_OK;
     }
@@ -711,8 +707,7 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
                                                                   starts.ptr, misc.ptr + 2);
     BOLT_HIP(hipGetLastError());
     uint32_t mx[2] = {0, 0};
-    BOLT_HIP(hipMemcpyAsync(mx, misc.ptr + 1, 8, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{mx, misc.ptr + 1, 8}}));
     if (mx[0]) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
     if (mx[1] <= (uint32_t)kLocMax) {
       uint32_t byte_mask = 0;
@@ -722,8 +717,7 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
                                                        p1 * kRadixBits, byte_mask, out_xor, misc.ptr + 2);
       BOLT_HIP(hipGetLastError());
       uint32_t e2 = 0;
-      BOLT_HIP(hipMemcpyAsync(&e2, misc.ptr + 2, 4, hipMemcpyDeviceToHost, s));
-      BOLT_HIP(hipStreamSynchronize(s));
+      BOLT_TRY(read_back(s, {{&e2, misc.ptr + 2, 4}}));
       if (e2) return set_error(BOLT_ERR_OTHER, "radix sort: bucket larger than the LDS sort");
       return BOLT_OK;
     }
@@ -1314,8 +1308,7 @@ static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys,
     BOLT_TRY(fill_u32(range.ptr, 0, 4 * kMaxFields, s));
     field_range_kernel<<<dim3(grid_for(n, 256, 4, 1024), of.n), 256, 0, s>>>(of, n, range.ptr);
     BOLT_HIP(hipGetLastError());
-    BOLT_HIP(hipMemcpyAsync(h, range.ptr, sizeof h, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{h, range.ptr, sizeof h}}));
     int left = 64;
     total = 0;
     for (int q = 0; q < of.n; q++) {
@@ -1348,8 +1341,7 @@ static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys,
     BOLT_TRY(fill_u32(err.ptr, 0, 1, s));
     tie_order_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(of, cut, k1, n, out_rows, err.ptr);
     BOLT_HIP(hipGetLastError());
-    BOLT_HIP(hipMemcpyAsync(&e, err.ptr, 4, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{&e, err.ptr, 4}}));
     *done = e == 0;
   }
   return BOLT_OK;
@@ -1505,9 +1497,9 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
     topk_hist_sum_kernel<<<dim3((unsigned)(((1 << width) + 255) / 256), 32), 256, 0, s>>>(part.ptr, (int)hgrid,
                                                                                         1 << width, hist.ptr);
     BOLT_HIP(hipGetLastError());
-    BOLT_HIP(hipMemcpyAsync(h.data(), hist.ptr, (size_t)(1 << width) * 4, hipMemcpyDeviceToHost, s));
-    if (first_digit < 0) BOLT_HIP(hipMemcpyAsync(&spec_got, spec_cnt.ptr, 8, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    unsigned long long got_now = 0;
+    BOLT_TRY(read_back(s, {{h.data(), hist.ptr, (size_t)(1 << width) * 4}, {&got_now, spec_cnt.ptr, 8}}));
+    if (first_digit < 0) spec_got = got_now;
     int64_t cum = 0;
     int d = 0;
     for (; d < (1 << width); d++) {
@@ -1547,8 +1539,7 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
     }
     BOLT_HIP(hipGetLastError());
     unsigned long long got = 0;
-    BOLT_HIP(hipMemcpyAsync(&got, cnt.ptr, 8, hipMemcpyDeviceToHost, s));
-    BOLT_HIP(hipStreamSynchronize(s));
+    BOLT_TRY(read_back(s, {{&got, cnt.ptr, 8}}));
     if ((int64_t)got != Cx)
       return set_error(BOLT_ERR_OTHER, "bolt_sort_limit: collected %llu candidates, expected %lld", got, (long long)Cx);
     cptr = cand.ptr;
@@ -1573,8 +1564,7 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
         default: topk_cand_hist_kernel<8><<<cgrid, 256, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
       }
       BOLT_HIP(hipGetLastError());
-      BOLT_HIP(hipMemcpyAsync(h.data(), hist.ptr, (size_t)(1 << width) * 4, hipMemcpyDeviceToHost, s));
-      BOLT_HIP(hipStreamSynchronize(s));
+      BOLT_TRY(read_back(s, {{h.data(), hist.ptr, (size_t)(1 << width) * 4}}));
       int64_t cum = 0;
       int d = 0;
       for (; d < (1 << width); d++) {
@@ -1607,8 +1597,7 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
           default: topk_tie_hist_kernel<8><<<cgrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
         }
         BOLT_HIP(hipGetLastError());
-        BOLT_HIP(hipMemcpyAsync(h.data(), hist.ptr, (size_t)(1 << width) * 4, hipMemcpyDeviceToHost, s));
-        BOLT_HIP(hipStreamSynchronize(s));
+        BOLT_TRY(read_back(s, {{h.data(), hist.ptr, (size_t)(1 << width) * 4}}));
         int64_t cum = 0;
         int d = 0;
         for (; d < (1 << width); d++) {
@@ -1642,8 +1631,7 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
       }
       BOLT_HIP(hipGetLastError());
       unsigned long long got2 = 0;
-      BOLT_HIP(hipMemcpyAsync(&got2, cnt.ptr, 8, hipMemcpyDeviceToHost, s));
-      BOLT_HIP(hipStreamSynchronize(s));
+      BOLT_TRY(read_back(s, {{&got2, cnt.ptr, 8}}));
       if ((int64_t)got2 != C2)
         return set_error(BOLT_ERR_OTHER, "bolt_sort_limit: narrowed to %llu candidates, expected %lld", got2,
                          (long long)C2);
