@@ -158,13 +158,7 @@ int acc_finalize(const Acc& a, int op, int dt, bolt_scalar_t* r) {
 
 int launch_finish(int na, const Acc* parts, int n_parts, int stride, int first, const AggList& aggs, Acc* out,
                   hipStream_t s) {
-  switch (na) {
-    case 1: finish_partials_kernel<1><<<1, kReduceBlock, 0, s>>>(parts, n_parts, stride, first, aggs, out); break;
-    case 2: finish_partials_kernel<2><<<1, kReduceBlock, 0, s>>>(parts, n_parts, stride, first, aggs, out); break;
-    case 3: finish_partials_kernel<3><<<1, kReduceBlock, 0, s>>>(parts, n_parts, stride, first, aggs, out); break;
-    case 4: finish_partials_kernel<4><<<1, kReduceBlock, 0, s>>>(parts, n_parts, stride, first, aggs, out); break;
-    default: return set_error(BOLT_ERR_OTHER, "launch_finish: bad chunk size %d", na);
-  }
+  finish_partials_kernel<<<(unsigned)na, kReduceBlock, 0, s>>>(parts, n_parts, stride, first, aggs, out);
   BOLT_HIP(hipGetLastError());
   return BOLT_OK;
 }
@@ -177,6 +171,10 @@ int launch_finish(int na, const Acc* parts, int n_parts, int stride, int first, 
 // and each block writes one partial.  The row-to-thread mapping is fixed by
 // the grid, so float results are reproducible.
 constexpr int kAggUnroll = 4;
+// At most 1024 workgroups: a streaming read of 2 GiB measured 6.8-6.9 TB/s at
+// 1024 x 256 threads with nontemporal loads, 5.4-6.1 TB/s at 4096-16384.  Fewer
+// only where a workgroup would have less than one iteration of rows.
+constexpr int kAggMaxGrid = 1024;
 
 template <int NT, int NA>
 __global__ __launch_bounds__(kReduceBlock) void scalar_agg_kernel(DevFilter f, AggList aggs, int64_t n,
@@ -409,7 +407,7 @@ extern "C" int bolt_aggregate_noalloc(bolt_stream_t stream, const bolt_column_t*
   const int64_t n = n_inputs >= 1 && inputs ? inputs[0].length : 0;
   // room for the most the call can use: kMaxAggs accumulators (the caller's
   // and the hidden MIN / MAX of SUM(Int64)) per workgroup, in chunks of 4
-  const unsigned grid = grid_for(n, kReduceBlock, kAggUnroll * 4, 256 * 8);
+  const unsigned grid = grid_for(n, kReduceBlock, kAggUnroll, kAggMaxGrid);
   const size_t parts_b = align256((size_t)grid * kMaxAggs * sizeof(Acc));
   const size_t outs_b = align256((size_t)kMaxAggs * sizeof(Acc));
   const size_t pfx_b = (size_t)kPfxMaxGrid * sizeof(Pfx);
@@ -468,9 +466,7 @@ static int bolt::aggregate_impl(hipStream_t s, const bolt_column_t* inputs, int3
   AggList all;
   BOLT_TRY(make_agg_list(aggs, n_aggs, inputs, n_inputs, 0, &all));
 
-  // at most 1024 workgroups: a streaming read of 2 GiB measured 6.8-6.9 TB/s
-  // at 1024 x 256 threads with nontemporal loads, 5.4-6.1 TB/s at 4096-16384
-  unsigned grid = stream_grid(n, kReduceBlock, kAggUnroll * 4, 1024);
+  unsigned grid = stream_grid(n, kReduceBlock, kAggUnroll, kAggMaxGrid);
   DevBuf<Acc> parts, outs;
   Acc* outs_p = scratch ? scratch->outs : nullptr;
   if (!outs_p) {
@@ -489,10 +485,7 @@ static int bolt::aggregate_impl(hipStream_t s, const bolt_column_t* inputs, int3
       prof_begin(s);
       BOLT_TRY(jit_launch_row_agg(fn, grid, s, nullptr, 0, nullptr, n, nullptr, nullptr, lits, cols, parts.ptr, nullptr, 0));
       prof_end(s);
-      for (int first = 0; first < n_aggs; first += 4) {
-        int na = n_aggs - first < 4 ? n_aggs - first : 4;
-        BOLT_TRY(launch_finish(na, parts.ptr, (int)grid, n_aggs, first, agg_chunk(all, first, na), outs_p + first, s));
-      }
+      BOLT_TRY(launch_finish(n_aggs, parts.ptr, (int)grid, n_aggs, 0, all, outs_p, s));
       done = true;
     }
     clear_error();

@@ -208,22 +208,6 @@ __device__ __forceinline__ void wave_reduce_acc(Acc& a, int op, int dtype) {
   }
 }
 
-// Reduce across a block of `waves` wave64s through `sh` (>= waves entries of
-// LDS); thread 0 stores the block result to *out.  Must be called by every
-// thread of the block.
-__device__ __forceinline__ void block_reduce_acc(Acc a, int op, int dtype, Acc* sh, int waves, Acc* out) {
-  wave_reduce_acc(a, op, dtype);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) sh[wave] = a;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    Acc r = sh[0];
-    for (int w = 1; w < waves; w++) acc_merge(r, sh[w], op, dtype);
-    *out = r;
-  }
-  __syncthreads();
-}
-
 // Literal values of a generated kernel's predicate terms (passed by value, so
 // the generated code does not change with the literals).
 struct JitLits {

@@ -77,6 +77,8 @@ bool jit_enabled();
 // Device helpers every generated kernel starts with (device_acc.h, gb_lds.h).
 const char* jit_prelude_text();
 std::string jit_row_agg_source(const JitSpec& sp);
+// Block reduction and store of accumulators acc0.. (op, dtype of each).
+std::string jit_reduce_tail(const std::vector<std::pair<int, int>>& aggs);
 // Compact description of everything in `sp` that shapes jit_row_agg_source's
 // text, for jit_get_keyed.
 std::string jit_row_agg_key(const JitSpec& sp);

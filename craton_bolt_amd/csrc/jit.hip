@@ -475,6 +475,33 @@ std::string probe_chains(const JitSpec& sp, int R, const std::function<std::stri
 
 }  // namespace
 
+// The end of a row kernel of 256 threads: accumulators acc0.. reduced over the
+// workgroup and stored at parts[blockIdx.x][a].  All waves reduce all
+// accumulators first and meet once (a barrier pair per accumulator left a
+// small input's kernel waiting on ten reductions in turn); then one lane per
+// accumulator, on different waves, merges its four wave results in order.
+std::string jit_reduce_tail(const std::vector<std::pair<int, int>>& aggs) {
+  std::ostringstream o;
+  const int na = (int)aggs.size();
+  o << "  __shared__ Acc sh[" << 4 * na << "];\n  const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6;\n";
+  for (int a = 0; a < na; a++)
+    o << "  wave_reduce_acc(acc" << a << ", " << aggs[a].first << ", " << aggs[a].second << ");\n";
+  o << "  if (lane_ == 0) {\n";
+  for (int a = 0; a < na; a++) o << "    sh[" << 4 * a << " + wave_] = acc" << a << ";\n";
+  o << "  }\n  __syncthreads();\n";
+  for (int a = 0; a < na; a++)
+    o << "  if (threadIdx.x == " << (a % 4) * 64 + a / 4 << ") {\n    Acc r_ = sh[" << 4 * a << "];\n"
+      << "    for (int w = 1; w < 4; w++) acc_merge(r_, sh[" << 4 * a << " + w], " << aggs[a].first << ", "
+      << aggs[a].second << ");\n    parts[(long long)blockIdx.x * " << na << " + " << a << "] = r_;\n  }\n";
+  return o.str();
+}
+
+static std::vector<std::pair<int, int>> reduced(const JitSpec& sp) {
+  std::vector<std::pair<int, int>> v;
+  for (const JitSpec::Agg& g : sp.aggs) v.emplace_back(g.op, g.dtype);
+  return v;
+}
+
 std::string jit_row_agg_source(const JitSpec& sp) {
   std::ostringstream o;
   o << kJitPrelude << "\n";
@@ -541,11 +568,7 @@ std::string jit_row_agg_source(const JitSpec& sp) {
   } else {
     for (int r = 0; r < R; r++) o << "    if (keep" << r << ") {\n" << updates(r, "      ") << "    }\n";
   }
-  o << "  }\n  __shared__ Acc sh[4];\n";
-  for (int a = 0; a < na; a++)
-    o << "  block_reduce_acc(acc" << a << ", " << sp.aggs[a].op << ", " << sp.aggs[a].dtype << ", sh, 4, parts + (long long)blockIdx.x * "
-      << na << " + " << a << ");\n";
-  o << "}\n";
+  o << "  }\n" << jit_reduce_tail(reduced(sp)) << "}\n";
   return o.str();
 }
 
@@ -723,11 +746,7 @@ std::string jit_jp_probe_source(const JitSpec& sp, int runs) {
     o << "      unsigned long long s" << rs << " = fmix64((unsigned long long)k" << rs << ") & mask;\n";
   }
   o << probe_chains(sp, R, [](int r) { return "in" + std::to_string(r); }, "      ");
-  o << "    }\n  }\n  __shared__ Acc sh[4];\n";
-  for (int a = 0; a < na; a++)
-    o << "  block_reduce_acc(acc" << a << ", " << sp.aggs[a].op << ", " << sp.aggs[a].dtype
-      << ", sh, 4, parts + (long long)blockIdx.x * " << na << " + " << a << ");\n";
-  o << "}\n";
+  o << "    }\n  }\n" << jit_reduce_tail(reduced(sp)) << "}\n";
   return o.str();
 }
 

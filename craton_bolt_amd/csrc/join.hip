@@ -866,10 +866,7 @@ extern "C" int bolt_join_probe_aggregate(bolt_stream_t stream, const bolt_join_t
       BOLT_TRY(jit_launch_row_agg(fn, grid, s, t->tbl, t->mask, t->flags, key.length, key.data, key.validity, lits, cols,
                                   parts.ptr, t->bloom, t->bloom_mask));
       prof_end(s);
-      for (int first = 0; first < n_aggs; first += 4) {
-        int na = n_aggs - first < 4 ? n_aggs - first : 4;
-        BOLT_TRY(launch_finish(na, parts.ptr, (int)grid, n_aggs, first, agg_chunk(all, first, na), outs.ptr + first, s));
-      }
+      BOLT_TRY(launch_finish(n_aggs, parts.ptr, (int)grid, n_aggs, 0, all, outs.ptr, s));
       done = true;
     }
     clear_error();

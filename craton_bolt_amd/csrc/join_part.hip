@@ -486,10 +486,7 @@ int join_probe_aggregate_partitioned(hipStream_t s, const bolt_join_table_t* t, 
     void* args[] = {&tb, &m, &fl, &okeys.ptr, &PP, &GG, &counts.ptr, &base.ptr, &actual.ptr, &queue.ptr, &pcols,
                     &parts.ptr};
     BOLT_HIP(hipModuleLaunchKernel(jprobe, pgrid, 1, 1, kJpProbeBlock, 1, 1, 0, s, args, nullptr));
-    for (int first = 0; first < n_aggs; first += 4) {
-      const int na = n_aggs - first < 4 ? n_aggs - first : 4;
-      BOLT_TRY(launch_finish(na, parts.ptr, (int)pgrid, n_aggs, first, agg_chunk(all, first, na), outs + first, s));
-    }
+    BOLT_TRY(launch_finish(n_aggs, parts.ptr, (int)pgrid, n_aggs, 0, all, outs, s));
     prof_end(s);
     return BOLT_OK;
   }

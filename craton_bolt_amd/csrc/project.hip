@@ -599,11 +599,9 @@ int gen_agg_source(const bolt_column_t* in, int n_in, const bolt_expr_op_t* prog
     }
     s << "    }\n";
   }
-  s << "  }\n  __shared__ Acc sh[4];\n";
-  for (int a = 0; a < aggs.n; a++)
-    s << "  block_reduce_acc(acc" << a << ", " << aggs.a[a].op << ", " << aggs.a[a].dtype
-      << ", sh, 4, parts + (long long)blockIdx.x * " << aggs.n << " + " << a << ");\n";
-  s << "}\n";
+  std::vector<std::pair<int, int>> red;
+  for (int a = 0; a < aggs.n; a++) red.emplace_back(aggs.a[a].op, aggs.a[a].dtype);
+  s << "  }\n" << jit_reduce_tail(red) << "}\n";
   *src = s.str();
   return BOLT_OK;
 }
@@ -728,10 +726,7 @@ extern "C" int bolt_aggregate_expr(bolt_stream_t stream, const bolt_column_t* in
   prof_begin(s);
   BOLT_HIP(hipModuleLaunchKernel(fn, grid, 1, 1, 256, 1, 1, 0, s, args, nullptr));
   prof_end(s);
-  for (int first = 0; first < n_aggs; first += 4) {
-    const int na = n_aggs - first < 4 ? n_aggs - first : 4;
-    BOLT_TRY(launch_finish(na, parts.ptr, (int)grid, n_aggs, first, agg_chunk(all, first, na), outs.ptr + first, s));
-  }
+  BOLT_TRY(launch_finish(n_aggs, parts.ptr, (int)grid, n_aggs, 0, all, outs.ptr, s));
   Acc host[kMaxAggs];
   BOLT_TRY(read_back(s, {{host, outs.ptr, sizeof(Acc) * n_aggs}}));
   for (int i = 0; i < n_aggs; i++) BOLT_TRY(acc_finalize(host[i], all.a[i].op, all.a[i].dtype, &results[i]));
