@@ -995,6 +995,9 @@ __device__ __forceinline__ uint64_t coarse_of(const TopKey& k, uint64_t raw, boo
   return k.nulls_first ? (x >> 1) + 1 : x >> 1;
 }
 
+// Inputs whose leading key is read in about the time that the sample's kernels
+// take keep the counting pass.
+constexpr int64_t kTopSampleBytes = (int64_t)256 << 20;
 constexpr int kSelBits = 14;
 constexpr int kSelBins = 1 << kSelBits;  // 64 KB of LDS counters
 constexpr int kSelBlock = 1024;
@@ -1077,57 +1080,174 @@ __global__ __launch_bounds__(256) void topk_hist_sum_kernel(const uint32_t* __re
   if (t) atomicAdd(&hist[b], t);
 }
 
-// Appends (unordered) the rows whose image >> shift <= bound.
+// A bound from a sample: large inputs are read once, comparing each row's image
+// with a quantile of the sampled images a little above rank K, instead of
+// counting digits of every row in LDS (2 GiB of int64 keys: 0.57 ms to count
+// and guess, 0.43 to compare and collect; a plain read takes 0.33).  The
+// sample's images in sorted lists, as split_sample_kernel's.
+__global__ __launch_bounds__(kSampleList) void topk_sample_kernel(TopKey k, int64_t n, int S,
+                                                                  uint64_t* __restrict__ lists) {
+  __shared__ uint64_t key[kSampleList];
+  const int j = blockIdx.x * kSampleList + threadIdx.x;
+  const int64_t lo = (int64_t)j * n / S, hi = (int64_t)(j + 1) * n / S;
+  const uint32_t h = (uint32_t)j * 0x9E3779B1u;
+  const int64_t i = lo + (int64_t)(((uint64_t)h * (uint64_t)(hi - lo)) >> 32);
+  uint64_t raw;
+  switch (k.dt) {
+    case BOLT_BOOL: raw = load_raw<1>(k.d, i); break;
+    case BOLT_I32: case BOLT_F32: case BOLT_DATE32: raw = load_raw<4>(k.d, i); break;
+    case BOLT_DEC128: raw = load_raw<16>(k.d, i); break;
+    default: raw = load_raw<8>(k.d, i); break;
+  }
+  key[threadIdx.x] = coarse_of(k, raw, bit_valid(k.v, i));
+  __syncthreads();
+  lds_bitonic<kSampleList>(kSampleList, [&](int a, int b) {
+    const uint64_t x = key[a], y = key[b];
+    if (x > y) {
+      key[a] = y;
+      key[b] = x;
+    }
+  });
+  lists[j] = key[threadIdx.x];
+}
+
+// plan[0] = the sample's rank-r image (1-based); plan[1] = samples at or below
+// it (more than r where it is tied); one wave.
+__global__ __launch_bounds__(64) void topk_bound_kernel(const uint64_t* __restrict__ sorted, int S, int r,
+                                                        uint64_t* __restrict__ plan) {
+  const uint64_t b = sorted[r - 1];
+  int at = S;  // first sample above b
+  for (int base = r; base < S; base += 64) {
+    const int i = base + threadIdx.x;
+    const uint64_t m = __ballot(i < S && sorted[i] > b);
+    if (m) {
+      at = base + __builtin_ctzll(m);
+      break;
+    }
+  }
+  if (threadIdx.x == 0) {
+    plan[0] = b;
+    plan[1] = (uint64_t)at;
+  }
+}
+
+// Appends (unordered) the rows whose image >> shift <= bound.  With `plan`
+// the bound is the sample's, the kernel leaves *count at all ones at once when
+// the sample has more than max_ties rows at or below it, and the smallest image
+// appended goes to *min_out.
 template <int W>
 __global__ __launch_bounds__(256) void topk_collect_kernel(TopKey k, int64_t n, int shift, uint64_t bound,
                                                            uint32_t* __restrict__ out,
-                                                           unsigned long long* __restrict__ count, int64_t cap) {
+                                                           unsigned long long* __restrict__ count, int64_t cap,
+                                                           const uint64_t* __restrict__ plan = nullptr,
+                                                           uint64_t max_ties = 0,
+                                                           unsigned long long* __restrict__ min_out = nullptr) {
+  if (plan) {
+    bound = plan[0];
+    if (plan[1] > max_ties) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) *count = ~0ull;
+      return;
+    }
+  }
+  // Rows are gathered per wave in LDS and appended with one atomic per
+  // workgroup at the end (or per wave and kWaveBuf rows where many pass): an
+  // atomic per wave and row group, all on one word, took 15 ns each, 1.28 ms
+  // for 82,000 rows among 2^28.
+  constexpr int kWaveBuf = 1024;
+  __shared__ uint32_t buf[4][kWaveBuf];
+  __shared__ uint32_t wcnt[4];
+  __shared__ unsigned long long wbase[4];
   const int64_t stride = (int64_t)gridDim.x * 256;
   const int64_t end = (n + 255) / 256 * 256;  // block-uniform trip count for the ballot
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t have = 0;  // rows in buf[wave]
+  uint64_t least = ~0ull;
   for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < end; i0 += stride * kSelUnroll) {
     uint64_t x[kSelUnroll];
 #pragma unroll
     for (int u = 0; u < kSelUnroll; u++) {
       const int64_t i = i0 + u * stride;
-      x[u] = i < n ? load_raw<W>(k.d, i) : 0;
+      x[u] = load_raw<W>(k.d, i < n ? i : n - 1);
     }
     bool take[kSelUnroll];
 #pragma unroll
     for (int u = 0; u < kSelUnroll; u++) {
       const int64_t i = i0 + u * stride;
-      take[u] = i < n && (shift >= 64 ? 0ull : coarse_of(k, x[u], bit_valid(k.v, i)) >> shift) <= bound;
+      take[u] = false;
+      if (i < n) {  // the validity bit, too, is read only for rows that exist
+        const uint64_t c = shift >= 64 ? 0ull : coarse_of(k, x[u], bit_valid(k.v, i)) >> shift;
+        take[u] = c <= bound;
+        if (take[u] && c < least) least = c;
+      }
     }
 #pragma unroll
     for (int u = 0; u < kSelUnroll; u++) {
       const uint64_t m = __ballot(take[u]);
       if (m == 0) continue;
-      const int leader = __builtin_ctzll(m);
+      if (take[u]) buf[wave][have + __popcll(m & ((1ull << lane) - 1))] = (uint32_t)(i0 + u * stride);
+      have += (uint32_t)__popcll(m);
+    }
+    if (have > kWaveBuf - 64 * kSelUnroll) {  // no room for another iteration's rows
       unsigned long long base = 0;
-      if (lane == leader) base = atomicAdd(count, (unsigned long long)__popcll(m));
-      base = __shfl(base, leader);
-      if (take[u]) {
-        const int64_t pos = (int64_t)base + __popcll(m & ((1ull << lane) - 1));
-        if (pos < cap) out[pos] = (uint32_t)(i0 + u * stride);
-      }
+      if (lane == 0) base = atomicAdd(count, (unsigned long long)have);
+      base = __shfl(base, 0);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (uint32_t j = lane; j < have; j += 64)
+        if ((int64_t)(base + j) < cap) out[base + j] = buf[wave][j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      have = 0;
     }
   }
+  if (min_out) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const uint64_t o = __shfl_xor(least, m);
+      least = o < least ? o : least;
+    }
+    if (lane == 0) wbase[wave] = least;
+  }
+  if (lane == 0) wcnt[wave] = have;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (min_out) {
+      for (int w = 0; w < 4; w++) least = wbase[w] < least ? wbase[w] : least;
+      if (least != ~0ull) atomicMin(min_out, (unsigned long long)least);
+    }
+    const uint32_t total = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
+    unsigned long long base = total ? atomicAdd(count, (unsigned long long)total) : 0ull;
+    for (int w = 0; w < 4; w++) {
+      wbase[w] = base;
+      base += wcnt[w];
+    }
+  }
+  __syncthreads();
+  const unsigned long long base = wbase[wave];
+  for (uint32_t j = lane; j < have; j += 64)
+    if ((int64_t)(base + j) < cap) out[base + j] = buf[wave][j];
 }
 
 // ---- small final sets: narrowed over the candidates, sorted in one workgroup ----------
 constexpr int kSmallSort = 4096;  // (image, row) pairs sorted in LDS by one workgroup
 
-// hist[digit] over the candidates whose image >> (shift + width) == prefix
+// hist[digit] over the candidates whose image >> (shift + width) == prefix.
+// Counted in LDS first: candidates of neighbouring keys share their upper
+// digits, and an atomic each on one word would take 15 ns each.
 template <int W>
-__global__ __launch_bounds__(256) void topk_cand_hist_kernel(TopKey k, const uint32_t* __restrict__ cand, int64_t c,
-                                                             int shift, int width, uint64_t prefix,
-                                                             uint32_t* __restrict__ hist) {
-  const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (j >= c) return;
-  const uint64_t x = coarse_of(k, load_raw<W>(k.d, cand[j]), true);
+__global__ __launch_bounds__(kSelBlock) void topk_cand_hist_kernel(TopKey k, const uint32_t* __restrict__ cand,
+                                                                   int64_t c, int shift, int width, uint64_t prefix,
+                                                                   uint32_t* __restrict__ hist) {
+  __shared__ uint32_t sh[kSelBins];
+  const int nb = 1 << width;
+  for (int b = threadIdx.x; b < nb; b += kSelBlock) sh[b] = 0;
+  __syncthreads();
   const int hi = shift + width;
-  if (hi < 64 && (x >> hi) != prefix) return;
-  atomicAdd(&hist[(x >> shift) & ((1ull << width) - 1)], 1u);
+  for (int64_t j = (int64_t)blockIdx.x * kSelBlock + threadIdx.x; j < c; j += (int64_t)gridDim.x * kSelBlock) {
+    const uint64_t x = coarse_of(k, load_raw<W>(k.d, cand[j]), true);
+    if (hi >= 64 || (x >> hi) == prefix) atomicAdd(&sh[(x >> shift) & ((1ull << width) - 1)], 1u);
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < nb; b += kSelBlock)
+    if (sh[b]) atomicAdd(&hist[b], sh[b]);
 }
 
 // Candidates tied on the whole image `img`: histogram of their row ids'
@@ -1466,6 +1586,7 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
   int hi = tk.bits;  // every image is below 2^bits (coarse_of)
   int64_t below = 0, need = K, eq = n;
   const unsigned grid = grid_for(n, 256, kSelUnroll, 4096);
+  const unsigned cgrid = grid_for(n, 256, kSelUnroll, 1024);  // a streaming read's grid (see the aggregates)
   // Candidates guessed in the first pass: the rows whose first digit is at
   // most spec_bound, where the K-th row's digit lies when the keys are spread
   // (about K * 2^14 / n); capacity for twice the expected count.
@@ -1479,7 +1600,51 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
   BOLT_TRY(fill_u32(spec_cnt.ptr, 0, 2, s));
   unsigned long long spec_got = 0;
   int first_digit = -1;
-  while (hi > 0) {
+  DevBuf<uint32_t> cand;
+  DevBuf<unsigned long long> cnt;
+  BOLT_TRY(cnt.alloc(4, s));
+  BOLT_TRY(fill_u32(cnt.ptr, 0, 2, s));
+  int64_t sampled = -1;  // candidates collected below the sample's bound
+  int64_t sample_bytes = kTopSampleBytes;
+  if (const char* e = getenv("BOLT_TOPK_SAMPLE_BYTES")) sample_bytes = atoll(e);  // testing
+  if (n * kw >= sample_bytes && K <= n / 64) {
+    // rank of the bound: K's share of the sample and a few deviations more
+    constexpr int S = 8192;
+    const double share = (double)K * S / (double)n;
+    const int r = (int)std::min<double>(S, std::ceil(share + 4.0 * std::sqrt(share) + 4.0));
+    const int64_t expect = (int64_t)((double)r * (double)n / S);
+    const int64_t cap = 4 * expect + 65536;  // at r = 5 one sample in a hundred finds twice what is expected
+    DevBuf<uint64_t> samp;
+    BOLT_TRY(samp.alloc(2 * S + 4, s));
+    BOLT_TRY(cand.alloc((size_t)cap, s));
+    uint64_t* plan = samp.ptr + 2 * S;
+    unsigned long long* least = reinterpret_cast<unsigned long long*>(plan + 2);
+    BOLT_TRY(fill_u32(least, 0xFFFFFFFFu, 2, s));
+    topk_sample_kernel<<<S / kSampleList, kSampleList, 0, s>>>(tk, n, S, samp.ptr);
+    split_merge_kernel<S / kSampleList><<<S / 64, 64, 0, s>>>(samp.ptr, samp.ptr + S);
+    topk_bound_kernel<<<1, 64, 0, s>>>(samp.ptr + S, S, r, plan);
+    const uint64_t ties = (uint64_t)r + (uint64_t)r / 2 + 2;  // tied beyond that: more rows than `cap` are likely
+    switch (kw) {
+      case 1: topk_collect_kernel<1><<<cgrid, 256, 0, s>>>(tk, n, 0, 0, cand.ptr, cnt.ptr, cap, plan, ties, least); break;
+      case 4: topk_collect_kernel<4><<<cgrid, 256, 0, s>>>(tk, n, 0, 0, cand.ptr, cnt.ptr, cap, plan, ties, least); break;
+      case 8: topk_collect_kernel<8><<<cgrid, 256, 0, s>>>(tk, n, 0, 0, cand.ptr, cnt.ptr, cap, plan, ties, least); break;
+      default: topk_collect_kernel<16><<<cgrid, 256, 0, s>>>(tk, n, 0, 0, cand.ptr, cnt.ptr, cap, plan, ties, least); break;
+    }
+    BOLT_HIP(hipGetLastError());
+    unsigned long long got = 0;
+    uint64_t bound[3];  // the bound, its rank, the smallest image collected
+    BOLT_TRY(read_back(s, {{&got, cnt.ptr, 8}, {bound, plan, 24}}));
+    if (got >= (unsigned long long)K && got <= (unsigned long long)cap) {
+      // every row up to the bound, the K first among them; their images agree
+      // above bit hi
+      sampled = (int64_t)got;
+      hi = bound[0] != bound[2] ? 64 - __builtin_clzll(bound[0] ^ bound[2]) : 0;
+      prefix = hi < 64 ? bound[0] >> hi : 0;
+      eq = sampled;
+    }
+    BOLT_TRY(fill_u32(cnt.ptr, 0, 2, s));
+  }
+  while (hi > 0 && sampled < 0) {
     const int width = hi >= kSelBits ? kSelBits : hi;
     const int shift = hi - width;
     uint32_t* sp = first_digit < 0 ? spec.ptr : nullptr;
@@ -1517,16 +1682,15 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
   }
   const int64_t Cx = below + eq;  // rows whose image >> hi <= prefix
   if (Cx * 2 > n) return full_sort();  // the leading key ties too often to narrow the rows
-  DevBuf<uint32_t> cand;
-  DevBuf<unsigned long long> cnt;
-  BOLT_TRY(cnt.alloc(1, s));
-  BOLT_TRY(fill_u32(cnt.ptr, 0, 2, s));
   // The candidates: the first pass's guess when it holds every row of the
   // K-th row's first digit and below (a superset of the Cx rows, which the
   // steps below accept), else a collect pass for exactly the Cx rows.
   const uint32_t* cptr;
   int64_t C;
-  if (first_digit >= 0 && (uint64_t)first_digit <= spec_bound && (int64_t)spec_got <= spec_cap) {
+  if (sampled >= 0) {
+    cptr = cand.ptr;
+    C = sampled;
+  } else if (first_digit >= 0 && (uint64_t)first_digit <= spec_bound && (int64_t)spec_got <= spec_cap) {
     cptr = spec.ptr;
     C = (int64_t)spec_got;
   } else {
@@ -1553,15 +1717,16 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
     uint64_t p2 = prefix;
     int hi2 = hi;
     int64_t below2 = below, need2 = need, eq2 = eq;
-    const unsigned cgrid = (unsigned)((C + 255) / 256);
+    const unsigned ngrid = (unsigned)((C + 255) / 256);
+    const unsigned hcgrid = (unsigned)std::min<int64_t>(64, (C + kSelBlock - 1) / kSelBlock);
     while (hi2 > 0 && below2 + eq2 > kSmallSort) {
       const int width = hi2 >= kSelBits ? kSelBits : hi2;
       const int shift = hi2 - width;
       BOLT_TRY(fill_u32(hist.ptr, 0, (size_t)1 << width, s));
       switch (kw) {
-        case 1: topk_cand_hist_kernel<1><<<cgrid, 256, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
-        case 4: topk_cand_hist_kernel<4><<<cgrid, 256, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
-        default: topk_cand_hist_kernel<8><<<cgrid, 256, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
+        case 1: topk_cand_hist_kernel<1><<<hcgrid, kSelBlock, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
+        case 4: topk_cand_hist_kernel<4><<<hcgrid, kSelBlock, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
+        default: topk_cand_hist_kernel<8><<<hcgrid, kSelBlock, 0, s>>>(tk, cptr, C, shift, width, p2, hist.ptr); break;
       }
       BOLT_HIP(hipGetLastError());
       BOLT_TRY(read_back(s, {{h.data(), hist.ptr, (size_t)(1 << width) * 4}}));
@@ -1592,9 +1757,9 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
         const int shift = rhi - width;
         BOLT_TRY(fill_u32(hist.ptr, 0, (size_t)1 << width, s));
         switch (kw) {
-          case 1: topk_tie_hist_kernel<1><<<cgrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
-          case 4: topk_tie_hist_kernel<4><<<cgrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
-          default: topk_tie_hist_kernel<8><<<cgrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
+          case 1: topk_tie_hist_kernel<1><<<ngrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
+          case 4: topk_tie_hist_kernel<4><<<ngrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
+          default: topk_tie_hist_kernel<8><<<ngrid, 256, 0, s>>>(tk, cptr, C, p2, shift, width, rpre, hist.ptr); break;
         }
         BOLT_HIP(hipGetLastError());
         BOLT_TRY(read_back(s, {{h.data(), hist.ptr, (size_t)(1 << width) * 4}}));
@@ -1617,9 +1782,9 @@ extern "C" int bolt_sort_limit(bolt_stream_t stream, const bolt_column_t* keys, 
       BOLT_TRY(cand2.alloc((size_t)C2, s));
       BOLT_TRY(fill_u32(cnt.ptr, 0, 2, s));
       switch (kw) {
-        case 1: topk_cand_collect_kernel<1><<<cgrid, 256, 0, s>>>(tk, cptr, C, hi2, p2, cand2.ptr, cnt.ptr, C2, rmax); break;
-        case 4: topk_cand_collect_kernel<4><<<cgrid, 256, 0, s>>>(tk, cptr, C, hi2, p2, cand2.ptr, cnt.ptr, C2, rmax); break;
-        default: topk_cand_collect_kernel<8><<<cgrid, 256, 0, s>>>(tk, cptr, C, hi2, p2, cand2.ptr, cnt.ptr, C2, rmax); break;
+        case 1: topk_cand_collect_kernel<1><<<ngrid, 256, 0, s>>>(tk, cptr, C, hi2, p2, cand2.ptr, cnt.ptr, C2, rmax); break;
+        case 4: topk_cand_collect_kernel<4><<<ngrid, 256, 0, s>>>(tk, cptr, C, hi2, p2, cand2.ptr, cnt.ptr, C2, rmax); break;
+        default: topk_cand_collect_kernel<8><<<ngrid, 256, 0, s>>>(tk, cptr, C, hi2, p2, cand2.ptr, cnt.ptr, C2, rmax); break;
       }
       BOLT_HIP(hipGetLastError());
       int npow = 1;
