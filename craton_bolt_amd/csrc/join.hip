@@ -117,23 +117,36 @@ __global__ __launch_bounds__(kRegBlock) void join_region_hist_kernel(const void*
   for (int r = threadIdx.x; r < n_regions; r += kRegBlock) counts[(int64_t)blockIdx.x * n_regions + r] = sc[r];
 }
 
-// counts[b][r] becomes the rows of region r in chunks before b; totals[r] the region's rows
-__global__ __launch_bounds__(256) void join_region_offsets_kernel(uint32_t* __restrict__ counts, int blocks,
-                                                                  int n_regions, uint32_t* __restrict__ totals) {
-  const int r = blockIdx.x * 256 + threadIdx.x;
+// counts[b][r] becomes the rows of region r in chunks before b; totals[r] the
+// region's rows.  Sixteen chunks a thread, all loads in flight at once, and the
+// sixteen threads of a region meet in LDS (one thread a region over all 256
+// chunks was a chain of 16 batches: 14.4 us for 1024 regions, 3.1 now).
+constexpr int kRegParts = 16;
+constexpr int kRegOffRegions = 32;  // regions of a workgroup: a cache line of counts
+__global__ __launch_bounds__(kRegParts* kRegOffRegions) void join_region_offsets_kernel(uint32_t* __restrict__ counts,
+                                                                                      int n_regions,
+                                                                                      uint32_t* __restrict__ totals) {
+  constexpr int kPer = kRegGrid / kRegParts;
+  __shared__ uint32_t sum[kRegParts][kRegOffRegions];
+  const int l = threadIdx.x % kRegOffRegions, part = threadIdx.x / kRegOffRegions;
+  const int r = blockIdx.x * kRegOffRegions + l;
+  uint32_t* at = counts + (int64_t)part * kPer * n_regions + r;
+  uint32_t c[kPer], all = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; j++) c[j] = r < n_regions ? at[(int64_t)j * n_regions] : 0u;
+#pragma unroll
+  for (int j = 0; j < kPer; j++) all += c[j];
+  sum[part][l] = all;
+  __syncthreads();
   if (r >= n_regions) return;
   uint32_t run = 0;
-  for (int b0 = 0; b0 < blocks; b0 += 16) {  // 16 loads in flight per lane
-    uint32_t c[16];
+  for (int p = 0; p < part; p++) run += sum[p][l];
 #pragma unroll
-    for (int j = 0; j < 16; j++) c[j] = b0 + j < blocks ? counts[(int64_t)(b0 + j) * n_regions + r] : 0u;
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      if (b0 + j < blocks) counts[(int64_t)(b0 + j) * n_regions + r] = run;
-      run += c[j];
-    }
+  for (int j = 0; j < kPer; j++) {
+    at[(int64_t)j * n_regions] = run;
+    run += c[j];
   }
-  totals[r] = run;
+  if (part == kRegParts - 1) totals[r] = run;
 }
 
 // base[r] = rows of regions before r (base[n_regions] = all); one workgroup
@@ -391,14 +404,21 @@ __device__ __forceinline__ bool same_key(const KeyCols& p, int64_t i, const KeyC
 
 // ---- probe emitting (probe_row, build_row) pairs -----------------------------
 //
-// Tiled with a decoupled look-back, like the compaction: a tile of
-// kEmitTile probe rows counts its matches, one wave looks back across
-// earlier tiles for the tile's output offset, and the pairs are written
-// densely.  No output counter is shared (one per wave serialises every wave
-// on a single address).  Each lane owns kEmitItems consecutive rows, so the
-// pairs come out in probe-row order.  With unique build keys one walk finds each row's
-// match and keeps it in a register; with duplicates the chain is walked
-// twice (count, then emit).
+// Tiled with a decoupled look-back: a tile of kEmitTile probe rows counts its
+// matches, one wave looks back across earlier tiles for the tile's output
+// offset, and the pairs are written densely, in probe-row order.  No output
+// counter is shared (one per wave serialises every wave on a single address).
+// Where the probe side is preserved, unfiltered, and the build keys are unique,
+// every row yields one pair, whose place is its own row: no tile waits for
+// another.
+//
+// Bound by the random 16-byte requests to the table.  A wave takes rows in
+// groups of 64 (whole lines of keys and pairs a request), and the chains of a
+// lane's rows are walked together, one request each in flight a round (eight
+// consecutive rows a lane, each chain walked by itself: 558 us for 20M LEFT rows
+// against 500K, 400 now; 552 and 475 INNER).  With unique build keys one walk finds each row's
+// match and keeps it in a register; with duplicates the chain is walked twice
+// (count, then emit).
 //
 // kPreserve (LEFT / RIGHT / FULL: the probe side is the preserved side) emits
 // one (probe_row, kNullRow) pair for a probe row that finds no match, in its
@@ -406,12 +426,13 @@ __device__ __forceinline__ bool same_key(const KeyCols& p, int64_t i, const KeyC
 // (src/exec/join.rs:396-437).  A non-null `unmatched` (FULL) has one byte per
 // build row, 1 on entry; every build row that matches is cleared to 0 with a
 // plain byte store (all writers store the same value).
+constexpr int kEmitBlock = 512;  // 256: LEFT 425 us, INNER 498; 1024: a LEFT join 40 us slower, INNER 5 faster
 constexpr int kEmitItems = 8;
-constexpr int kEmitTile = kProbeBlock * kEmitItems;  // 2048 rows
+constexpr int kEmitTile = kEmitBlock * kEmitItems;  // 4096 rows
 constexpr uint32_t kNullRow = 0xFFFFFFFFu;
 
 template <typename KeyT, bool kPreserve, bool kVerify>
-__global__ __launch_bounds__(kProbeBlock) void join_probe_emit_kernel(
+__global__ __launch_bounds__(kEmitBlock) void join_probe_emit_kernel(
     const uint4* __restrict__ tbl, uint64_t mask, const uint32_t* __restrict__ nonunique,
     const KeyT* __restrict__ keys, const uint8_t* __restrict__ kvalid, int64_t n, DevFilter f,
     uint64_t* __restrict__ status, uint32_t* __restrict__ ticket, uint32_t* __restrict__ err,
@@ -419,89 +440,121 @@ __global__ __launch_bounds__(kProbeBlock) void join_probe_emit_kernel(
     uint32_t* __restrict__ out_build, const uint4* __restrict__ bloom, uint64_t bmask,
     uint8_t* __restrict__ unmatched, KeyCols pk, KeyCols bk) {
   __shared__ uint32_t sh_tile;
-  __shared__ uint32_t wsum[kProbeBlock / 64];
+  __shared__ uint32_t wsum[kEmitBlock / 64];
   __shared__ unsigned long long sh_base;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) sh_tile = atomicAdd(ticket, 1u);
-  __syncthreads();
-  const int64_t tile = sh_tile;
-  const int64_t tbase = tile * kEmitTile;
   const bool first_only = (*nonunique == 0u);
+  const bool one_each = kPreserve && first_only && f.n == 0;
+  int64_t tile = blockIdx.x;
+  if (!one_each) {
+    if (threadIdx.x == 0) sh_tile = atomicAdd(ticket, 1u);
+    __syncthreads();
+    tile = sh_tile;
+  }
+  const int64_t row0 = tile * kEmitTile + wave * (64 * kEmitItems) + lane;  // the lane's rows: row0 + 64 j
   uint32_t m[kEmitItems], bv[kEmitItems];
-  uint32_t mine = 0, pad = 0, live = 0;
+  uint32_t pad = 0, live = 0, walk = 0;
   int64_t kk[kEmitItems];
   uint64_t ss[kEmitItems];
   uint4 ee[kEmitItems];
-  // keys and the home slots of the lane's rows first, all in flight together,
-  // then each row's chain from its already-loaded home slot
 #pragma unroll
   for (int j = 0; j < kEmitItems; j++) {
-    const int64_t i = tbase + ((int64_t)threadIdx.x * kEmitItems + j);
+    const int64_t i = row0 + 64 * j;
+    kk[j] = (int64_t)keys[i < n ? i : n - 1];  // all in flight before the first is used
+  }
+#pragma unroll
+  for (int j = 0; j < kEmitItems; j++) {
+    const int64_t i = row0 + 64 * j;
     const bool lv = i < n && eval_filter(f, i);
     live |= (uint32_t)lv << j;
     const bool ok = lv && bit_valid(kvalid, i);
-    kk[j] = ok ? (int64_t)keys[i] : 0;
-    ss[j] = ok && bloom_maybe(bloom, bmask, kk[j]) ? fmix64((uint64_t)kk[j]) & mask : ~0ull;
-  }
-#pragma unroll
-  for (int j = 0; j < kEmitItems; j++) ee[j] = ss[j] != ~0ull ? tbl[ss[j]] : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-  for (int j = 0; j < kEmitItems; j++) {
-    const int64_t i = tbase + ((int64_t)threadIdx.x * kEmitItems + j);
+    ss[j] = fmix64((uint64_t)kk[j]) & mask;
+    walk |= (uint32_t)(ok && bloom_maybe(bloom, bmask, kk[j])) << j;
     m[j] = 0;
-    bv[j] = 0;
-    uint4 e = ee[j];
-    uint64_t sl = ss[j];
-    for (uint64_t step = 0; e.w != 0u && step <= mask; step++) {
-      if (slot_key(e) == kk[j] && (!kVerify || same_key(pk, i, bk, e.z))) {
-        m[j]++;
-        bv[j] = e.z;
-        if (unmatched) unmatched[e.z] = 0;
-        if (first_only) break;
-      }
-      sl = (sl + 1) & mask;
-      e = tbl[sl];
-    }
-    if (kPreserve && ((live >> j) & 1u) && m[j] == 0) {
-      m[j] = 1;
-      bv[j] = kNullRow;
-      pad |= 1u << j;
-    }
-    mine += m[j];
+    bv[j] = kNullRow;
   }
-  // lane prefix within the wave, wave prefix within the tile
-  uint32_t inc = mine;
+  for (uint64_t step = 0; walk != 0u && step <= mask; step++) {
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t v = __shfl_up(inc, d);
-    if (lane >= d) inc += v;
-  }
-  if (lane == 63) wsum[wave] = inc;
-  __syncthreads();
-  if (wave == 0) {
-    uint32_t tile_total = 0;
-    for (int w = 0; w < kProbeBlock / 64; w++) tile_total += wsum[w];
-    const uint64_t excl = lookback_wave(status, tile, tile_total, err);
-    if (lane == 0) {
-      sh_base = excl;
-      if (tile == (int64_t)gridDim.x - 1) *total_out = excl + tile_total;
+    for (int j = 0; j < kEmitItems; j++)
+      if ((walk >> j) & 1u) ee[j] = tbl[ss[j]];
+#pragma unroll
+    for (int j = 0; j < kEmitItems; j++) {
+      if (!((walk >> j) & 1u)) continue;
+      if (ee[j].w == 0u) {
+        walk &= ~(1u << j);
+        continue;
+      }
+      if (slot_key(ee[j]) == kk[j] && (!kVerify || same_key(pk, row0 + 64 * j, bk, ee[j].z))) {
+        m[j]++;
+        bv[j] = ee[j].z;
+        if (unmatched) unmatched[ee[j].z] = 0;
+        if (first_only) walk &= ~(1u << j);
+      }
+      ss[j] = (ss[j] + 1) & mask;
     }
   }
-  __syncthreads();
-  unsigned long long pos = sh_base + inc - mine;
-  for (int w = 0; w < wave; w++) pos += wsum[w];
+  if (kPreserve) {
+#pragma unroll
+    for (int j = 0; j < kEmitItems; j++)
+      if (((live >> j) & 1u) && m[j] == 0) {
+        m[j] = 1;
+        pad |= 1u << j;
+      }
+  }
+  // pairs before each row within the wave, wave prefix within the tile
+  uint32_t pre[kEmitItems], run = 0;
+  if (first_only) {
+#pragma unroll
+    for (int j = 0; j < kEmitItems; j++) {
+      const uint64_t b = __ballot(m[j] != 0u);
+      pre[j] = run + (uint32_t)__popcll(b & ((1ull << lane) - 1));
+      run += (uint32_t)__popcll(b);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kEmitItems; j++) {
+      uint32_t inc = m[j];
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t v = __shfl_up(inc, d);
+        if (lane >= d) inc += v;
+      }
+      pre[j] = run + inc - m[j];
+      run += __shfl(inc, 63);
+    }
+  }
+  unsigned long long base;
+  if (one_each) {
+    base = (unsigned long long)(row0 - lane);
+    if (tile == 0 && threadIdx.x == 0) *total_out = (unsigned long long)n;
+  } else {
+    if (lane == 0) wsum[wave] = run;
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t tile_total = 0;
+      for (int w = 0; w < kEmitBlock / 64; w++) tile_total += wsum[w];
+      const uint64_t excl = lookback_wave(status, tile, tile_total, err);
+      if (lane == 0) {
+        sh_base = excl;
+        if (tile == (int64_t)gridDim.x - 1) *total_out = excl + tile_total;
+      }
+    }
+    __syncthreads();
+    base = sh_base;
+    for (int w = 0; w < wave; w++) base += wsum[w];
+  }
 #pragma unroll
   for (int j = 0; j < kEmitItems; j++) {
     if (!m[j]) continue;
-    const int64_t i = tbase + ((int64_t)threadIdx.x * kEmitItems + j);
+    const int64_t i = row0 + 64 * j;
+    unsigned long long pos = base + pre[j];
     if (first_only || (pad >> j) & 1u) {
       if ((int64_t)pos < capacity) {
         out_probe[pos] = (uint32_t)i;
         out_build[pos] = bv[j];
       }
-      pos++;
     } else {
-      probe_chain(tbl, mask, (int64_t)keys[i], false, [&](uint32_t w) {
+      probe_chain(tbl, mask, kk[j], false, [&](uint32_t w) {
         if (kVerify && !same_key(pk, i, bk, w)) return;
         if ((int64_t)pos < capacity) {
           out_probe[pos] = (uint32_t)i;
@@ -697,7 +750,8 @@ extern "C" int bolt_join_build(bolt_stream_t stream, const bolt_column_t* build_
     if (e == hipSuccess) {
       join_region_hist_kernel<<<kRegGrid, kRegBlock, lds, s>>>(build_key->data, t->key_dtype, build_key->validity, n, per,
                                                                t->mask, n_regions, counts.ptr);
-      join_region_offsets_kernel<<<(n_regions + 255) / 256, 256, 0, s>>>(counts.ptr, kRegGrid, n_regions, totals.ptr);
+      join_region_offsets_kernel<<<(n_regions + kRegOffRegions - 1) / kRegOffRegions, kRegParts * kRegOffRegions, 0, s>>>(
+          counts.ptr, n_regions, totals.ptr);
       join_region_scan_kernel<<<1, kRegBlock, 0, s>>>(totals.ptr, n_regions, rbase.ptr);
       join_region_scatter_kernel<<<kRegGrid, kRegBlock, lds, s>>>(build_key->data, t->key_dtype, build_key->validity,
                                                                   cv, n, per, t->mask, n_regions, counts.ptr, rbase.ptr,
@@ -920,7 +974,7 @@ static int probe_emit(hipStream_t s, const bolt_join_table_t* t, const bolt_colu
     BOLT_TRY(status.alloc((size_t)tiles, s));
     BOLT_TRY(fill_u32(status.ptr, 0, (size_t)tiles * 2, s));
 #define EMIT_LAUNCH(KT, PRESERVE, VERIFY)                                                                        \
-  join_probe_emit_kernel<KT, PRESERVE, VERIFY><<<(unsigned)tiles, kProbeBlock, 0, s>>>(                          \
+  join_probe_emit_kernel<KT, PRESERVE, VERIFY><<<(unsigned)tiles, kEmitBlock, 0, s>>>(                           \
       t->tbl, t->mask, t->flags, static_cast<const KT*>(key.data), key.validity, key.length, f, status.ptr,      \
       misc.ptr, misc.ptr + 1, counter.ptr, capacity, out_probe, out_build, t->bloom, t->bloom_mask, unmatched,  \
       pk, bk)
