@@ -8,6 +8,9 @@
 // round-trip to the host between passes.  Here every aggregate of the query
 // is updated by the same pass:
 //
+//   copy    Only where a sample of the keys finds more groups than an LDS table
+//           holds and at most what 256 of them do: the rows are copied grouped
+//           by key hash, and pass A gives each part a table (no spills).
 //   pass A  LDS tier.  Each workgroup keeps an open-addressing table of up to
 //           a few thousand groups in LDS (keys + one 64-bit word per
 //           accumulator field) and updates it with LDS atomics.  Rows whose
@@ -1106,7 +1109,15 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     if (gfn && try_partition) {
       bool yes = false;
       BOLT_TRY(gb_part_wanted(s, ks, f, n, S, part_S, &yes));
-      if (yes) BOLT_TRY(gb_part_copy(s, ks, P, f, gs, glits, gcols, n, &pc, &yes));
+      if (yes) {
+        const int st = gb_part_copy(s, ks, P, f, gs, glits, gcols, n, &pc, &yes);
+        if (st == BOLT_ERR_MEMORY) {  // no room for the copy (nothing launched yet): the paths without one
+          pc.bufs.clear();
+          yes = false;
+        } else if (st != BOLT_OK) {
+          return st;
+        }
+      }
       hipFunction_t pfn = nullptr;
       if (yes && jit_get_keyed(gb_jit_key(pc.spec), [&] { return jit_gb_lds_source(pc.spec); }, &pfn) == BOLT_OK) {
         gfn = pfn;

@@ -219,6 +219,7 @@ int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys
  * the LDS tier's partial records merged into the table, 1 = rows also spilled
  * to the global table with atomics, 2 = the radix-partitioned tier; the rows
  * the LDS tier spilled, its partial records, and the partitions (tier 2).
+ * Inputs copied by key partitions first (each aggregated in LDS) are tier 0.
  * Any pointer may be NULL. */
 int bolt_groupby_last_plan(int32_t* tier, int64_t* spilled_rows, int64_t* partial_records, int32_t* partitions);
 /* Autotuner of the radix-partitioned tier's fan-out, the partition count
@@ -330,9 +331,10 @@ int bolt_join(bolt_stream_t stream, const bolt_column_t* left_keys, const bolt_c
 /* ------------------------------------------------------------------------
  * Radix sort — replaces sort_indices_on_gpu_radix{,_multi}
  * (src/exec/gpu_sort.rs:944,995) and run_radix_pipeline_i64 (:1493).
- * Stable LSD radix sort, one up-front histogram pass for all digits, then per
- * digit one onesweep pass (LDS ranking + decoupled look-back), no host round
- * trip between passes.  n < 2^30.
+ * Stable.  Up to 2^23 rows (2^25 where the top digits are uneven) buckets from
+ * a sample of the keys, sorted in LDS; above, two onesweep passes (LDS ranking
+ * + decoupled look-back) over the top varying digits and LDS bucket sorts;
+ * onesweep passes over every digit where a bucket does not fit.  n < 2^30.
  * ------------------------------------------------------------------------ */
 
 /* Sort (key, value) pairs by int64 key (ascending unless `descending`).
