@@ -963,6 +963,15 @@ __device__ __forceinline__ uint64_t load_raw(const void* d, int64_t i) {
   else return static_cast<const uint64_t*>(d)[2 * i + 1];
 }
 
+// The same past the caches, for a pass that reads the column once.
+template <int W>
+__device__ __forceinline__ uint64_t load_raw_once(const void* d, int64_t i) {
+  if constexpr (W == 1) return __builtin_nontemporal_load(static_cast<const uint8_t*>(d) + i);
+  else if constexpr (W == 4) return __builtin_nontemporal_load(static_cast<const uint32_t*>(d) + i);
+  else if constexpr (W == 8) return __builtin_nontemporal_load(static_cast<const uint64_t*>(d) + i);
+  else return __builtin_nontemporal_load(static_cast<const uint64_t*>(d) + 2 * i + 1);
+}
+
 // Ascending image of raw key bits (the transforms of radix_image).
 __device__ __forceinline__ uint64_t raw_image(uint64_t b, int dt) {
   switch (dt) {
@@ -1083,7 +1092,7 @@ __global__ __launch_bounds__(256) void topk_hist_sum_kernel(const uint32_t* __re
 // A bound from a sample: large inputs are read once, comparing each row's image
 // with a quantile of the sampled images a little above rank K, instead of
 // counting digits of every row in LDS (2 GiB of int64 keys: 0.57 ms to count
-// and guess, 0.43 to compare and collect; a plain read takes 0.33).  The
+// and guess, 0.40 to compare and collect; a plain read takes 0.33).  The
 // sample's images in sorted lists, as split_sample_kernel's.
 __global__ __launch_bounds__(kSampleList) void topk_sample_kernel(TopKey k, int64_t n, int S,
                                                                   uint64_t* __restrict__ lists) {
@@ -1153,7 +1162,9 @@ __global__ __launch_bounds__(256) void topk_collect_kernel(TopKey k, int64_t n, 
   // workgroup at the end (or per wave and kWaveBuf rows where many pass): an
   // atomic per wave and row group, all on one word, took 15 ns each, 1.28 ms
   // for 82,000 rows among 2^28.
-  constexpr int kWaveBuf = 1024;
+  // 64 bytes in flight per lane; 4 rows: int64 431 us, int32 about 430 (2^28 rows)
+  constexpr int kU = W >= 8 ? 8 : 16;
+  constexpr int kWaveBuf = 128 * kU;
   __shared__ uint32_t buf[4][kWaveBuf];
   __shared__ uint32_t wcnt[4];
   __shared__ unsigned long long wbase[4];
@@ -1162,16 +1173,16 @@ __global__ __launch_bounds__(256) void topk_collect_kernel(TopKey k, int64_t n, 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t have = 0;  // rows in buf[wave]
   uint64_t least = ~0ull;
-  for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < end; i0 += stride * kSelUnroll) {
-    uint64_t x[kSelUnroll];
+  for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < end; i0 += stride * kU) {
+    uint64_t x[kU];
 #pragma unroll
-    for (int u = 0; u < kSelUnroll; u++) {
+    for (int u = 0; u < kU; u++) {
       const int64_t i = i0 + u * stride;
-      x[u] = load_raw<W>(k.d, i < n ? i : n - 1);
+      x[u] = load_raw_once<W>(k.d, i < n ? i : n - 1);
     }
-    bool take[kSelUnroll];
+    bool take[kU];
 #pragma unroll
-    for (int u = 0; u < kSelUnroll; u++) {
+    for (int u = 0; u < kU; u++) {
       const int64_t i = i0 + u * stride;
       take[u] = false;
       if (i < n) {  // the validity bit, too, is read only for rows that exist
@@ -1181,13 +1192,13 @@ __global__ __launch_bounds__(256) void topk_collect_kernel(TopKey k, int64_t n, 
       }
     }
 #pragma unroll
-    for (int u = 0; u < kSelUnroll; u++) {
+    for (int u = 0; u < kU; u++) {
       const uint64_t m = __ballot(take[u]);
       if (m == 0) continue;
       if (take[u]) buf[wave][have + __popcll(m & ((1ull << lane) - 1))] = (uint32_t)(i0 + u * stride);
       have += (uint32_t)__popcll(m);
     }
-    if (have > kWaveBuf - 64 * kSelUnroll) {  // no room for another iteration's rows
+    if (have > kWaveBuf - 64 * kU) {  // no room for another iteration's rows
       unsigned long long base = 0;
       if (lane == 0) base = atomicAdd(count, (unsigned long long)have);
       base = __shfl(base, 0);
