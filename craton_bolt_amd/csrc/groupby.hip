@@ -106,21 +106,29 @@ __global__ __launch_bounds__(kGbBlock) void gb_lds_kernel(KeySpec ks, DevFilter 
 
 // ---- key partition: when the groups are too many for one LDS table -------------------
 //
-// Between what one workgroup's LDS table holds and what 256 of them hold, the
-// LDS tier alone spills most rows to global atomics on the table's words.
-// There the input is first copied, partitioned by the key's hash, and each of
-// 256 workgroups runs the LDS tier on one partition: no row spills, and every
-// group is complete in one workgroup.  A sample of the keys decides: it
-// estimates the group count, and a key frequent enough to leave its
-// partition's workgroup behind the others keeps the plain path, which
-// aggregates such keys in every workgroup.  10M rows of two int32 keys and two
-// float sums: 10,000 groups 1.41 -> 0.63 ms, 100,000 1.60 -> 0.96, 500,000 1.68
-// -> 1.02; 100M rows, 50,000 groups 8.6 -> 3.5 ms.  Below 2^21 rows the copy and
-// the sample's round trip cost what they save.
+// Between what one workgroup's LDS table holds and what 256 of them hold, the LDS
+// tier alone spills most rows to global atomics on the table's words. There the
+// input is first copied, partitioned by the key's hash, and each of 256 workgroups
+// runs the LDS tier on one partition: no row spills, and every group is complete in
+// one workgroup.  A sample of the keys proposes it: more groups than one table
+// holds, and no key frequent enough to leave its partition's workgroup behind the
+// others (the plain path aggregates such keys in every workgroup).  From 4096 keys
+// a million groups look like 0.6 to 2 million, and a few frequent keys hide a long
+// tail, so the first pass over the keys counts the groups (HyperLogLog, within
+// 2.3%) and stops the others on the device where they would fill the tables beyond
+// kGbPartLoad.  10M rows of two int32 keys and two float sums against the LDS tier
+// and global atomics alone: 10,000 groups 1.40 -> 0.56 ms, 100,000 1.60 -> 0.88,
+// 980,000 1.76 -> 1.09; 100M rows, 50,000 groups 8.5 -> 3.2 ms.  10M rows of 1.1M
+// groups, which the count sends back: 1.69 ms without the attempt, 1.77 with it.
+// Below 2^21 rows the copy and the sample's round trip cost what they save.
 
 constexpr int kGbSample = 4096;
 constexpr int kGbSampleSlots = 2 * kGbSample;
 constexpr int64_t kGbPartMinRows = (int64_t)1 << 21;
+// Share of the tables' slots that the counted groups may take.  Three standard
+// errors of the count more and the fullest partition's excess are below 0.7
+// full, where every key finds a slot within kPartProbes.
+constexpr double kGbPartLoad = 0.6;
 
 // One workgroup: distinct keys among kGbSample stratified rows that pass the
 // filter.  out = {rows with a regular key, distinct keys, most frequent key's
@@ -183,15 +191,36 @@ __global__ __launch_bounds__(1024) void gb_sample_kernel(KeySpec ks, DevFilter f
 
 // counts[c][p] -> first output row of chunk c's rows of partition p (rows of a
 // partition in chunk order), and ranges[p] = the partition's first row.  One
-// workgroup; thread (q, p) sums a quarter q of the chunks.
+// workgroup; thread (q, p) sums a quarter q of the chunks.  `hll` holds the keys'
+// registers: where the sum of 2^-register, in units of 2^-40, is below `least`
+// there are more groups than the tables take, every range is left empty (the
+// kernels behind then do nothing) and ranges[256 + 1] is 1.
+constexpr int kPartHllUnit = 40;
 __global__ __launch_bounds__(1024) void gb_part_offsets_kernel(uint32_t* __restrict__ counts, int chunks,
+                                                               const uint32_t* __restrict__ hll, uint64_t least,
                                                                uint32_t* __restrict__ ranges) {
   constexpr int P = 1 << kGbPartBits;
   static_assert(P == 256, "one thread per partition and quarter");
   __shared__ uint32_t part[4][P];
   __shared__ uint32_t start[P];
   __shared__ uint32_t wtot[4];
+  __shared__ uint64_t hsum[16];
   const int p = threadIdx.x & (P - 1), q = threadIdx.x >> 8, lane = threadIdx.x & 63;
+  uint64_t h = 0;
+  for (int i = threadIdx.x; i < kHllRegs; i += 1024) {
+    const uint32_t r = hll[i];
+    h += r <= kPartHllUnit ? 1ull << (kPartHllUnit - r) : 0ull;
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) h += __shfl_xor(h, m);
+  if (lane == 0) hsum[threadIdx.x >> 6] = h;
+  __syncthreads();
+  h = 0;
+  for (int w = 0; w < 16; w++) h += hsum[w];
+  if (h < least) {  // block-uniform
+    if (threadIdx.x <= P + 1) ranges[threadIdx.x] = threadIdx.x == P + 1 ? 1u : 0u;
+    return;
+  }
   const int per = (chunks + 3) / 4;
   const int c0 = q * per, c1 = c0 + per < chunks ? c0 + per : chunks;
   uint32_t sum = 0;
@@ -215,7 +244,10 @@ __global__ __launch_bounds__(1024) void gb_part_offsets_kernel(uint32_t* __restr
     for (int w = 0; w < (p >> 6); w++) inc += wtot[w];
     start[p] = inc - tot;
     ranges[p] = inc - tot;
-    if (p == P - 1) ranges[P] = inc;
+    if (p == P - 1) {
+      ranges[P] = inc;
+      ranges[P + 1] = 0;
+    }
   }
   __syncthreads();
   uint32_t at = start[p];
@@ -824,7 +856,7 @@ static int gb_jit_spec(const KeySpec& ks, const GPlan& P, const DevFilter& f, Gb
 
 // The key-partitioned copy of an input and where its partitions start.
 struct GbPartCopy {
-  DevBuf<uint32_t> counts, ranges;
+  DevBuf<uint32_t> counts, ranges, hll;
   std::vector<DevBuf<uint8_t>> bufs;
   KeySpec ks;          // the copied key (NULLs one byte per row)
   GbJitSpec spec;      // the LDS tier's kernel over the copies
@@ -844,6 +876,9 @@ static double sample_groups(double m, double d) {
   return lo;
 }
 
+// Groups that the partitions' tables of part_S slots take.
+static double part_groups_most(int part_S) { return kGbPartLoad * part_S * (1 << kGbPartBits); }
+
 // Whether the input goes through the key partition (synchronises).
 static int gb_part_wanted(hipStream_t s, const KeySpec& ks, const DevFilter& f, int64_t n, int S, int part_S,
                           bool* yes) {
@@ -859,18 +894,18 @@ static int gb_part_wanted(hipStream_t s, const KeySpec& ks, const DevFilter& f, 
   gb_sample_kernel<<<1, 1024, 0, s>>>(ks, f, n, out.ptr);
   BOLT_HIP(hipGetLastError());
   BOLT_TRY(read_back(s, {{h, out.ptr, 12}}));
-  // few sampled rows pass the filter: the plain path; more groups than half
-  // of what the LDS tables hold together would spill; a key above 0.4% of the
-  // rows (its share of 1/256) would make one workgroup the last
+  // few sampled rows pass the filter: the plain path; a key above 0.4% of the
+  // rows (its share of 1/256) would make one workgroup the last; twice the limit
+  // leaves the sample's error to the count
   const double est = sample_groups(h[0], h[1]);
-  *yes = h[0] >= kGbSample / 4 && est > 0.75 * S && est <= 0.5 * part_S * (1 << kGbPartBits) &&
-         h[2] <= 8 + h[0] / 256;
+  *yes = h[0] >= kGbSample / 4 && est > 0.75 * S && est <= 2 * part_groups_most(part_S) && h[2] <= 8 + h[0] / 256;
   return BOLT_OK;
 }
 
-// Copies the rows that pass the filter, partitioned by key hash.
-static int gb_part_copy(hipStream_t s, const KeySpec& ks, const GPlan& P, const DevFilter& f, const GbJitSpec& gs,
-                        JitLits& lits, JitCols& cols, int64_t n, GbPartCopy* out, bool* ok) {
+// Copies the rows that pass the filter, partitioned by key hash (nothing, with
+// ranges[257] set, where the groups are too many).
+static int gb_part_copy(hipStream_t s, const KeySpec& ks, const GbJitSpec& gs, JitLits& lits, JitCols& cols, int64_t n,
+                        int part_S, GbPartCopy* out, bool* ok) {
   *ok = false;
   std::vector<int> copied;
   for (const GbJitSpec::Agg& a : gs.aggs)
@@ -886,7 +921,9 @@ static int gb_part_copy(hipStream_t s, const KeySpec& ks, const GPlan& P, const 
   long long per = per_tiles * kGbPartTile, nn = n;
   const int np = 1 << kGbPartBits;
   BOLT_TRY(out->counts.alloc((size_t)chunks * np, s));
-  BOLT_TRY(out->ranges.alloc(np + 1, s));
+  BOLT_TRY(out->ranges.alloc(np + 2, s));
+  BOLT_TRY(out->hll.alloc(kHllRegs, s));
+  BOLT_TRY(fill_u32(out->hll.ptr, 0, kHllRegs, s));
   GbCopies dst;
   memset(&dst, 0, sizeof dst);
   auto buf = [&](size_t bytes, void** p) -> int {
@@ -941,11 +978,17 @@ static int gb_part_copy(hipStream_t s, const KeySpec& ks, const GPlan& P, const 
     if (a.col >= 0) a.col = at[a.col];
   sp.vbytes = any_valid;
   unsigned int* counts = out->counts.ptr;
+  unsigned int* hll = out->hll.ptr;
+  const unsigned int* rows_kept = out->ranges.ptr + np;
+  // the registers' sum at which hll_estimate gives the limit (its plain form,
+  // the one that holds at limits of tens of thousands and more)
+  const double m = kHllRegs, most = part_groups_most(part_S);
+  const uint64_t least = (uint64_t)std::ldexp(0.7213 / (1.0 + 1.079 / m) * m * m / most, kPartHllUnit);
   for (int mode = 0; mode < 2; mode++) {
     void* args[] = {&nn, &per, &mode, (void*)&ks.d0, (void*)&ks.v0, (void*)&ks.d1, (void*)&ks.v1, &lits, &cols,
-                    (void*)&counts, &dst};
+                    (void*)&counts, &dst, (void*)&hll, (void*)&rows_kept};
     BOLT_HIP(hipModuleLaunchKernel(fn, (unsigned)chunks, 1, 1, 1024, 1, 1, 0, s, args, nullptr));
-    if (mode == 0) gb_part_offsets_kernel<<<1, 1024, 0, s>>>(counts, chunks, out->ranges.ptr);
+    if (mode == 0) gb_part_offsets_kernel<<<1, 1024, 0, s>>>(counts, chunks, hll, least, out->ranges.ptr);
   }
   BOLT_HIP(hipGetLastError());
   *ok = true;
@@ -1110,7 +1153,7 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
       bool yes = false;
       BOLT_TRY(gb_part_wanted(s, ks, f, n, S, part_S, &yes));
       if (yes) {
-        const int st = gb_part_copy(s, ks, P, f, gs, glits, gcols, n, &pc, &yes);
+        const int st = gb_part_copy(s, ks, gs, glits, gcols, n, part_S, &pc, &yes);
         if (st == BOLT_ERR_MEMORY) {  // no room for the copy (nothing launched yet): the paths without one
           pc.bufs.clear();
           yes = false;
@@ -1170,13 +1213,17 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     prof_end(s);
     BOLT_HIP(hipGetLastError());
     std::vector<uint32_t> regs(kHllRegs + 4);
-    BOLT_TRY(read_back(s, {{regs.data(), hll.ptr, (kHllRegs + 4) * 4}}));
+    uint32_t declined = 0;
+    if (key_parts)
+      BOLT_TRY(read_back(s, {{regs.data(), hll.ptr, (kHllRegs + 4) * 4}, {&declined, ranges + (1 << kGbPartBits) + 1, 4}}));
+    else
+      BOLT_TRY(read_back(s, {{regs.data(), hll.ptr, (kHllRegs + 4) * 4}}));
     unsigned long long hc[2];
     memcpy(hc, regs.data() + kHllRegs, 16);
     n_parts = (int64_t)hc[0];
     n_spill = (int64_t)hc[1];
     est = hll_estimate(regs.data());
-    if (key_parts && n_spill > 0)  // more groups than the sample promised
+    if (key_parts && (declined || n_spill > 0))  // more groups than the tables take
       return groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags, false, out);
   } else {
     n_spill = n;  // every row goes to the global table

@@ -881,7 +881,7 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
          "        else {\n"
          "          const bool taken = cur" << rs << " != kEmpty;\n"
          "          const u32_t from = taken ? (home" << rs << " + 1 == (u32_t)S ? 0u : home" << rs << " + 1) : home" << rs << ";\n"
-         "          const int lim = gb_lds_probes(S, &sused[3]);\n"
+         "          const int lim = gb_lds_probes(S, &sused[3], ranges ? kPartProbes : kLdsProbes);\n"
          "          slot = gb_lds_probe(skeys, S, key" << rs << ", from, taken ? lim - 1 : lim, &sused[3]);\n"
          "          spill = slot < 0;\n"
          "        }\n"
@@ -957,7 +957,8 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
 // [c * per, (c + 1) * per)) in tiles of kGbPartTile rows; a row that passes the
 // filter goes to the partition of the top 8 bits of its key's hash (a row of
 // the NULL group to any, by its position).  mode 0: counts[c][p] = rows of the
-// chunk in partition p.  mode 1: `counts` holds where the chunk's rows of each
+// chunk in partition p, and the keys' HyperLogLog registers in `hll` (from the
+// hash bits below the partition's).  mode 1: `counts` holds where the chunk's rows of each
 // partition start, and the columns are copied there, in row order: a tile is
 // ranked per partition in LDS, and each column in turn is staged in LDS in
 // partition order and written as runs.  Bound by the copies' traffic: no
@@ -972,14 +973,18 @@ std::string jit_gb_partition_source(const GbJitSpec& sp, const std::vector<int>&
   o << "extern \"C\" __global__ void __launch_bounds__(1024) bolt_jit_kernel(\n"
        "    long long n, long long per, int mode, const void* __restrict__ k0p, const unsigned char* __restrict__ k0v,\n"
        "    const void* __restrict__ k1p, const unsigned char* __restrict__ k1v, bolt::JitLits lits,\n"
-       "    bolt::JitCols cols, unsigned int* __restrict__ counts, bolt::GbCopies dst) {\n"
+       "    bolt::JitCols cols, unsigned int* __restrict__ counts, bolt::GbCopies dst, unsigned int* __restrict__ hll,\n"
+       "    const unsigned int* __restrict__ rows_kept) {\n"
        "  using namespace bolt;\n"
+       "  if (mode && *rows_kept == 0) return;  // nothing to copy, or too many groups\n"
        "  __shared__ u64_t st[" << kGbPartTile << "];\n"
        "  __shared__ unsigned char sdig[" << kGbPartTile << "];\n"
        "  __shared__ u32_t cnt[" << P << "], pre[" << P << "], off[" << P << "], run[" << P << "], wtot[" << P / 64 << "];\n"
        "  const int t = threadIdx.x, lane = t & 63;\n";
   emit_gb_ptrs(o, sp);
-  o << "  const long long lo = (long long)blockIdx.x * per;\n"
+  o << "  u32_t* const shll = (u32_t*)st;  // mode 0 stages nothing\n"
+       "  if (mode == 0) for (int i = t; i < kHllRegs; i += 1024) shll[i] = 0;\n"
+       "  const long long lo = (long long)blockIdx.x * per;\n"
        "  if (n > lo + per) n = lo + per;\n"
        "  if (t < " << P << ") { cnt[t] = 0; off[t] = mode ? counts[(long long)blockIdx.x * " << P << " + t] : 0; }\n"
        "  __syncthreads();\n"
@@ -988,11 +993,14 @@ std::string jit_gb_partition_source(const GbJitSpec& sp, const std::vector<int>&
   emit_gb_rows(o, sp, R, 1024);
   for (int r = 0; r < R; r++) {
     const std::string rs = std::to_string(r);
-    o << "    const int p" << rs << " = kind" << rs << " == 0 ? -1 : (int)((kind" << rs << " == 2 ? (u64_t)i" << rs
-      << " * 0x9E3779B97F4A7C15ull : fmix64(key" << rs << ")) >> " << 64 - kGbPartBits << ");\n";
+    o << "    const u64_t h" << rs << " = kind" << rs << " == 2 ? (u64_t)i" << rs << " * 0x9E3779B97F4A7C15ull : fmix64(key"
+      << rs << ");\n"
+      << "    const int p" << rs << " = kind" << rs << " == 0 ? -1 : (int)(h" << rs << " >> " << 64 - kGbPartBits << ");\n";
   }
   o << "    if (mode == 0) {\n";
-  for (int r = 0; r < R; r++) o << "      if (p" << r << " >= 0) atomicAdd(&cnt[p" << r << "], 1u);\n";
+  for (int r = 0; r < R; r++)
+    o << "      if (p" << r << " >= 0) atomicAdd(&cnt[p" << r << "], 1u);\n"
+      << "      if (kind" << r << " == 1) hll_add_hash(shll, h" << r << " << " << kGbPartBits << ");\n";
   o << "      continue;\n    }\n";
   for (int r = 0; r < R; r++)
     o << "    const u32_t rank" << r << " = p" << r << " >= 0 ? atomicAdd(&cnt[p" << r << "], 1u) : 0u;\n";
@@ -1076,7 +1084,10 @@ std::string jit_gb_partition_source(const GbJitSpec& sp, const std::vector<int>&
   }
   o << "  }\n"
        "  __syncthreads();\n"
-       "  if (mode == 0 && t < " << P << ") counts[(long long)blockIdx.x * " << P << " + t] = cnt[t];\n"
+       "  if (mode) return;\n"
+       "  if (t < " << P << ") counts[(long long)blockIdx.x * " << P << " + t] = cnt[t];\n"
+       "  for (int i = t; i < kHllRegs; i += 1024)\n"
+       "    if (shll[i] > hll[i]) atomicMax(&hll[i], shll[i]);\n"
        "}\n";
   return o.str();
 }

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from craton_bolt_amd import _native as N
-from craton_bolt_amd.ops import Term
+from craton_bolt_amd.ops import Term, groupby_last_plan
 
 from gpu_util import dec_array
 from test_gpu_groupby import run_both
@@ -90,6 +90,43 @@ def test_more_groups_than_the_tables(gpu):
     print("[case] key partition overflow", flush=True)
     k = np.random.default_rng(7).permutation(n).astype(np.int64)
     run_both([(k, N.I64, None)], [(k.astype(np.float64), N.F64, None)], [(N.SUM, 0), (N.COUNT_STAR, 0)], [N.I64])
+
+
+# SUM(f64) and COUNT(*) are two words: 256 tables of 6440 slots, of which the
+# groups may take 0.6 (989,000).  At 300,000 and above a bound of 16 slots a
+# probe left keys without one, and the whole call ran again on the plain path.
+@pytest.mark.parametrize("kind", ["i64", "i32", "pair"])
+@pytest.mark.parametrize("groups", [300_000, 500_000, 700_000, 930_000])
+def test_every_group_finds_a_slot(gpu, monkeypatch, kind, groups):
+    monkeypatch.delenv("BOLT_GB_KEY_PARTITION")
+    n = 2_200_000
+    print(f"[case] key partition {kind} groups={groups}", flush=True)
+    rng = np.random.default_rng(groups)
+    g = rng.permutation(n) % groups
+    if kind == "pair":
+        keys, kdt = [((g % 900).astype(np.int32), N.I32, None), ((g // 900).astype(np.int32), N.I32, None)], [N.I32] * 2
+    elif kind == "i32":
+        keys, kdt = [((g * 7919 - 1).astype(np.int32), N.I32, None)], [N.I32]
+    else:
+        keys, kdt = [(rng.integers(-2 ** 63, 2 ** 63 - 1, groups)[g], N.I64, None)], [N.I64]
+    run_both(keys, [(rng.normal(size=n), N.F64, None)], [(N.SUM, 0), (N.COUNT_STAR, 0)], kdt)
+    assert groupby_last_plan() == {"tier": 0, "spilled_rows": 0, "partial_records": groups, "partitions": 0}
+
+
+@pytest.mark.parametrize("few", [0, 10_000])
+def test_too_many_groups_are_counted(gpu, monkeypatch, few):
+    """More groups than the tables take, by themselves or behind a few frequent ones (which a sample takes
+    for all): the count ends the partition, and the plain path answers."""
+    monkeypatch.delenv("BOLT_GB_KEY_PARTITION")
+    n, many = 2_400_000, 1_300_000
+    print(f"[case] key partition declined few={few}", flush=True)
+    rng = np.random.default_rng(8)
+    g = rng.permutation(n) % many
+    if few:
+        g = np.where(rng.random(n) < 0.3, rng.integers(0, few, n), g)
+    run_both([(g * 0x9E3779B97F4A7, N.I64, None)], [(rng.normal(size=n), N.F64, None)], [(N.SUM, 0), (N.COUNT_STAR, 0)],
+             [N.I64])
+    assert groupby_last_plan()["spilled_rows"] > 0
 
 
 @pytest.mark.parametrize("groups", [9_000, 300_000])
