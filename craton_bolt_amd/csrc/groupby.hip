@@ -1063,9 +1063,12 @@ static int order_groups(hipStream_t s, bolt_table* tbl, std::vector<bolt_column_
   return BOLT_OK;
 }
 
+// `parted` (may be null: no key partition) is set once the call has gone for the
+// key partition; kGbPlain: it does not hold the input, run again without.
+constexpr int kGbPlain = 1 << 20;  // no status of the API
 static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys, const bolt_column_t* inputs,
                        int32_t n_inputs, const bolt_agg_t* aggs, int32_t n_aggs, const bolt_filter_t* filter,
-                       uint32_t flags, bool try_partition, bolt_table_t** out) {
+                       uint32_t flags, bool* parted, bolt_table_t** out) {
   BOLT_CHECK_DEVICE();
   clear_error();
   *out = nullptr;
@@ -1149,18 +1152,11 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     const KeySpec* pks = &ks;
     JitCols* pcols = &gcols;
     const uint32_t* ranges = nullptr;
-    if (gfn && try_partition) {
+    if (gfn && parted) {
       bool yes = false;
       BOLT_TRY(gb_part_wanted(s, ks, f, n, S, part_S, &yes));
-      if (yes) {
-        const int st = gb_part_copy(s, ks, gs, glits, gcols, n, part_S, &pc, &yes);
-        if (st == BOLT_ERR_MEMORY) {  // no room for the copy (nothing launched yet): the paths without one
-          pc.bufs.clear();
-          yes = false;
-        } else if (st != BOLT_OK) {
-          return st;
-        }
-      }
+      *parted = yes;
+      if (yes) BOLT_TRY(gb_part_copy(s, ks, gs, glits, gcols, n, part_S, &pc, &yes));
       hipFunction_t pfn = nullptr;
       if (yes && jit_get_keyed(gb_jit_key(pc.spec), [&] { return jit_gb_lds_source(pc.spec); }, &pfn) == BOLT_OK) {
         gfn = pfn;
@@ -1168,6 +1164,8 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
         pks = &pc.ks;
         pcols = &pc.cols;
         ranges = pc.ranges.ptr;
+      } else {
+        pc.bufs.clear();
       }
       clear_error();
     }
@@ -1223,8 +1221,7 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     n_parts = (int64_t)hc[0];
     n_spill = (int64_t)hc[1];
     est = hll_estimate(regs.data());
-    if (key_parts && (declined || n_spill > 0))  // more groups than the tables take
-      return groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags, false, out);
+    if (key_parts && (declined || n_spill > 0)) return kGbPlain;  // more groups than the tables take
   } else {
     n_spill = n;  // every row goes to the global table
     est = (double)n;
@@ -1465,8 +1462,14 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
 extern "C" int bolt_groupby(bolt_stream_t stream, const bolt_column_t* keys, int32_t n_keys,
                             const bolt_column_t* inputs, int32_t n_inputs, const bolt_agg_t* aggs, int32_t n_aggs,
                             const bolt_filter_t* filter, uint32_t flags, bolt_table_t** out) {
-  return groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags,
-                     !(flags & BOLT_GROUPBY_FORCE_PARTITIONED), out);
+  bool parted = false;
+  int st = groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags,
+                       (flags & BOLT_GROUPBY_FORCE_PARTITIONED) ? nullptr : &parted, out);
+  // the attempt's buffers are free again: what fits without the key partition
+  // fits, wherever in the attempt the room ended
+  if (st == kGbPlain || (parted && st == BOLT_ERR_MEMORY))
+    st = groupby_run(stream, keys, n_keys, inputs, n_inputs, aggs, n_aggs, filter, flags, nullptr, out);
+  return st;
 }
 
 extern "C" int bolt_groupby_last_plan(int32_t* tier, int64_t* spilled_rows, int64_t* partial_records,

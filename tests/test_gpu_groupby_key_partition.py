@@ -3,6 +3,11 @@ size): every key form, NULL keys and inputs, filters, every aggregate, row
 counts around the partition's tiles and chunks, and inputs with more groups
 than the partitions' LDS tables hold (the plain path runs instead), against
 the oracle with test_gpu_groupby's comparisons and tolerances."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -127,6 +132,38 @@ def test_too_many_groups_are_counted(gpu, monkeypatch, few):
     run_both([(g * 0x9E3779B97F4A7, N.I64, None)], [(rng.normal(size=n), N.F64, None)], [(N.SUM, 0), (N.COUNT_STAR, 0)],
              [N.I64])
     assert groupby_last_plan()["spilled_rows"] > 0
+
+
+_PEAK = """
+import ctypes as C, os
+import numpy as np
+from craton_bolt_amd import _native as N
+from craton_bolt_amd.device import DeviceColumn
+from craton_bolt_amd.ops import execute_groupby
+def peak():
+    used, high = C.c_size_t(), C.c_size_t()
+    N.check_rt(N.lib().bolt_hip_pool_stats(C.byref(used), C.byref(high)))
+    return high.value
+n = 4_000_000
+g = np.random.default_rng(9).permutation(n) % 1_300_000
+k, v = DeviceColumn.from_numpy(g * 0x9E3779B97F4A7), DeviceColumn.from_numpy(np.ones(n))
+for how in ("0", "1"):
+    os.environ["BOLT_GB_KEY_PARTITION"] = how
+    assert execute_groupby([k], [v], [(N.SUM, 0), (N.COUNT_STAR, 0)])["n_groups"] == 1_300_000
+    print("peak", how, peak(), flush=True)
+"""
+
+
+def test_declined_attempt_holds_no_memory(gpu):
+    """A call whose attempt is given up needs no more device memory at once than the plain path alone (the
+    high-water mark of a process of its own: it never falls)."""
+    print("[case] key partition declined, peak memory", flush=True)
+    r = subprocess.run([sys.executable, "-u", "-c", _PEAK], cwd=Path(__file__).resolve().parent.parent, timeout=100,
+                       env=dict(os.environ), capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    plain, tried = (int(line.split()[2]) for line in r.stdout.splitlines() if line.startswith("peak"))
+    # a few hundred bytes go with the rows that the LDS tier happens to spill; the attempt's copies alone are 64 MB
+    assert tried <= plain + (1 << 20), (tried, plain)
 
 
 @pytest.mark.parametrize("groups", [9_000, 300_000])
