@@ -1143,23 +1143,18 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     GbJitSpec gs;
     JitLits glits;
     JitCols gcols;
-    if (jit_enabled() && gb_jit_spec(ks, P, f, &gs, &glits, &gcols) == BOLT_OK &&
-        jit_get_keyed(gb_jit_key(gs), [&] { return jit_gb_lds_source(gs); }, &gfn) != BOLT_OK)
-      gfn = nullptr;
-    clear_error();
+    const bool jit = jit_enabled() && gb_jit_spec(ks, P, f, &gs, &glits, &gcols) == BOLT_OK;
     // more groups than one LDS table holds: the key partition first
     GbPartCopy pc;
     const KeySpec* pks = &ks;
     JitCols* pcols = &gcols;
     const uint32_t* ranges = nullptr;
-    if (gfn && parted) {
+    if (jit && parted) {
       bool yes = false;
       BOLT_TRY(gb_part_wanted(s, ks, f, n, S, part_S, &yes));
       *parted = yes;
       if (yes) BOLT_TRY(gb_part_copy(s, ks, gs, glits, gcols, n, part_S, &pc, &yes));
-      hipFunction_t pfn = nullptr;
-      if (yes && jit_get_keyed(gb_jit_key(pc.spec), [&] { return jit_gb_lds_source(pc.spec); }, &pfn) == BOLT_OK) {
-        gfn = pfn;
+      if (yes && jit_get_keyed(gb_jit_key(pc.spec), [&] { return jit_gb_lds_source(pc.spec); }, &gfn) == BOLT_OK) {
         gs = pc.spec;
         pks = &pc.ks;
         pcols = &pc.cols;
@@ -1167,9 +1162,11 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
       } else {
         pc.bufs.clear();
       }
-      clear_error();
     }
     key_parts = ranges != nullptr;
+    if (jit && !key_parts && jit_get_keyed(gb_jit_key(gs), [&] { return jit_gb_lds_source(gs); }, &gfn) != BOLT_OK)
+      gfn = nullptr;
+    clear_error();
     if (key_parts) S = part_S;
     const size_t lds = (size_t)(S + 2) * 8 * (1 + W) + (kHllRegs + 4) * 4;
     const int64_t rows_per_iter = (int64_t)kGbBlock * (gfn ? gs.unroll : 1);

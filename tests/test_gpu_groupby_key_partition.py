@@ -3,6 +3,7 @@ size): every key form, NULL keys and inputs, filters, every aggregate, row
 counts around the partition's tiles and chunks, and inputs with more groups
 than the partitions' LDS tables hold (the plain path runs instead), against
 the oracle with test_gpu_groupby's comparisons and tolerances."""
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -164,6 +165,23 @@ def test_declined_attempt_holds_no_memory(gpu):
     plain, tried = (int(line.split()[2]) for line in r.stdout.splitlines() if line.startswith("peak"))
     # a few hundred bytes go with the rows that the LDS tier happens to spill; the attempt's copies alone are 64 MB
     assert tried <= plain + (1 << 20), (tried, plain)
+
+
+def test_compiles_what_it_runs(gpu):
+    """A query shape of its own: the partition's kernel and the LDS tier over the copies, not the plain tier's."""
+    def compiled():
+        c, h, s = C.c_int64(), C.c_int64(), C.c_int64()
+        N.lib().bolt_jit_cache_stats(C.byref(c), C.byref(h), C.byref(s))
+        return c.value + h.value
+
+    rng = np.random.default_rng(10)
+    keys, kdt = _key("f32", 5000, 900, rng)
+    x = rng.normal(size=5000)
+    print("[case] key partition compiles", flush=True)
+    before = compiled()
+    run_both(keys, [(x, N.F64, rng.random(5000) > 0.2)],  # NULLs: a bitmap there, bytes in the copy
+             [(N.MIN, 0), (N.COUNT, 0), (N.MAX, 0), (N.AVG, 0), (N.COUNT_STAR, 0)], kdt)
+    assert compiled() - before == 2
 
 
 @pytest.mark.parametrize("groups", [9_000, 300_000])
