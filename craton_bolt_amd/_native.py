@@ -273,6 +273,7 @@ _SIGS = {
     "bolt_groupby": (C.c_int, [C.c_void_p, C.POINTER(BoltColumn), C.c_int32, C.POINTER(BoltColumn), C.c_int32,
                                C.POINTER(BoltAgg), C.c_int32, C.POINTER(BoltFilter), C.c_uint32,
                                C.POINTER(C.c_void_p)]),
+    "bolt_sort_last_plan": (C.c_int, [C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
     "bolt_groupby_last_plan": (C.c_int, [C.POINTER(C.c_int32), C.POINTER(C.c_int64), C.POINTER(C.c_int64),
                                          C.POINTER(C.c_int32)]),
     "bolt_groupby_autotune_partitions": (C.c_int, [C.c_void_p, C.POINTER(BoltColumn), C.c_int32,

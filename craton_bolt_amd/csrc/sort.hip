@@ -50,18 +50,21 @@ constexpr uint32_t kSFlagAgg = 1u << 30;
 constexpr uint32_t kSFlagInc = 2u << 30;
 constexpr uint32_t kSValue = (1u << 30) - 1;
 
-// ---- histogram of every digit ---------------------------------------------------
+// ---- histogram of the digits -----------------------------------------------------
 
+// Digits p < passes whose bit is set in `digits`.  Bound by its LDS atomics, one a
+// key and digit.
 __global__ __launch_bounds__(kSortBlock) void radix_hist_kernel(const uint64_t* __restrict__ keys, int64_t n,
-                                                                int passes, uint32_t* __restrict__ hist,
-                                                                uint64_t in_xor) {
+                                                                int passes, uint32_t digits,
+                                                                uint32_t* __restrict__ hist, uint64_t in_xor) {
   __shared__ uint32_t h[kMaxPasses][kBins];
   for (int i = threadIdx.x; i < passes * kBins; i += kSortBlock) (&h[0][0])[i] = 0;
   __syncthreads();
   const int64_t stride = (int64_t)gridDim.x * kSortBlock;
   for (int64_t i = (int64_t)blockIdx.x * kSortBlock + threadIdx.x; i < n; i += stride) {
     uint64_t k = __builtin_nontemporal_load(keys + i) ^ in_xor;
-    for (int p = 0; p < passes; p++) atomicAdd(&h[p][(k >> (p * kRadixBits)) & (kBins - 1)], 1u);
+    for (int p = 0; p < passes; p++)
+      if ((digits >> p) & 1u) atomicAdd(&h[p][(k >> (p * kRadixBits)) & (kBins - 1)], 1u);
   }
   __syncthreads();
   for (int i = threadIdx.x; i < passes * kBins; i += kSortBlock) {
@@ -523,32 +526,51 @@ __global__ __launch_bounds__(kLocBlock) void local_sort_kernel(
 
 namespace bolt {
 
-// The splitter sort of 2 <= n <= kSplitMax pairs.  *done = false when a bucket
+// Buckets of at most 384 rows on average (512 in one pass and above 3 << 23
+// rows), most of which the first bucket kernel holds.
+static int split_code_bits(int64_t n) {
+  const bool one = n <= kSplitOnePass;
+  int cbits = one ? 6 : 9;  // 6: the splitters of one sorted list, no merge
+  while (((int64_t)(one ? 512 : 384) << cbits) < n && cbits < 16) cbits++;
+  return cbits;
+}
+static int split_samples(int64_t n) {
+  const int cbits = split_code_bits(n);
+  return cbits == 6 ? kSampleList : cbits <= 12 ? 4096 : 16384;
+}
+// Allocates the sample (and the room for its merge) and draws it; `vary`
+// workgroups more look for varying bits.
+static int split_sample(hipStream_t s, const uint64_t* keys, int64_t n, uint64_t in_xor, DevBuf<uint64_t>& sample,
+                        uint64_t* one_zero, int vary) {
+  const int S = split_samples(n);
+  BOLT_TRY(sample.alloc((size_t)2 * S, s));
+  split_sample_kernel<<<S / kSampleList + vary, kSampleList, 0, s>>>(keys, n, in_xor, S, sample.ptr, one_zero);
+  BOLT_HIP(hipGetLastError());
+  return BOLT_OK;
+}
+
+// The splitter sort of 2 <= n <= kSplitMax pairs (`sample` drawn, or empty).  *done = false when a bucket
 // of different keys exceeded the LDS sort (keys_out / vals_out then hold
 // nothing of use; the inputs are untouched).
 static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t* vals_in, int64_t n,
                                 uint64_t* keys_out, uint32_t* vals_out, uint64_t in_xor, uint64_t out_xor,
-                                bool* done) {
+                                DevBuf<uint64_t>& sample, bool* done) {
   *done = true;
   if (n <= kSplitWhole) {
     split_whole_kernel<<<1, 1024, 0, s>>>(keys_in, vals_in, keys_out, vals_out, (int)n, in_xor, out_xor);
     BOLT_HIP(hipGetLastError());
     return BOLT_OK;
   }
-  // Buckets of at most 384 rows on average (512 in one pass and above 3 << 23
-  // rows), most of which the first bucket kernel holds.
   const bool one = n <= kSplitOnePass;
-  int cbits = one ? 6 : 9;  // 6: the splitters of one sorted list, no merge
-  while (((int64_t)(one ? 512 : 384) << cbits) < n && cbits < 16) cbits++;
-  const int C = 1 << cbits;
+  const int cbits = split_code_bits(n), C = 1 << cbits;
   const int b1 = one ? 8 : cbits / 2;
-  const int S = cbits == 6 ? kSampleList : cbits <= 12 ? 4096 : 16384;
+  const int S = split_samples(n);
   const int64_t tiles = (n + kSortTile - 1) / kSortTile;
-  DevBuf<uint64_t> sample, ktmp;
+  DevBuf<uint64_t> ktmp;
   DevBuf<uint32_t> vtmp, words, start;
   DevBuf<uint16_t> codes;
   DevBuf<uint8_t> digits;
-  BOLT_TRY(sample.alloc((size_t)2 * S, s));
+  if (!sample.ptr) BOLT_TRY(split_sample(s, keys_in, n, in_xor, sample, nullptr, 0));
   BOLT_TRY(codes.alloc((size_t)n, s));
   // counts, scanned counts, tickets and error, then the look-back words of
   // each pass: one fill
@@ -561,7 +583,6 @@ static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const ui
   uint32_t* misc = offs + 514;
   uint32_t* status = words.ptr + head;
   const Splitters sp{S == kSampleList ? sample.ptr : sample.ptr + S, S, std::min(C, S), std::max(cbits - 14, 0)};
-  split_sample_kernel<<<S / kSampleList, kSampleList, 0, s>>>(keys_in, n, in_xor, S, sample.ptr);
   if (S > 4096) split_merge_kernel<16><<<S / 64, 64, 0, s>>>(sample.ptr, sample.ptr + S);
   else if (S > kSampleList) split_merge_kernel<4><<<S / 64, 64, 0, s>>>(sample.ptr, sample.ptr + S);
   const size_t lds = (size_t)(sp.G + 1) * 8;
@@ -598,9 +619,33 @@ static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const ui
   return BOLT_OK;
 }
 
-// Sort (keys_in, vals_in) ascending by the low `key_bits` bits of
-// (key ^ in_xor), stable, writing (key image ^ out_xor, value) to keys_out /
-// vals_out.  Inputs are not modified and must not alias the outputs.
+// The calling thread's last sort (bolt_sort_last_plan).
+static thread_local bolt_sort_plan_t t_sort_plan = BOLT_SORT_COPY;
+static thread_local int t_sort_passes = 0;
+static void set_sort_plan(bolt_sort_plan_t plan, int passes) {
+  t_sort_plan = plan;
+  t_sort_passes = passes;
+}
+
+// Whether keys of np varying bytes are sorted by a onesweep pass per byte, n
+// between kSplitOnePass and kSplitMax.  A pass costs 15 us at 150,000 rows, 30 at
+// 1M, 60 at 5M and 120 at 20M, whatever the values; the splitter sort's cost
+// hardly depends on the bytes, but grows with the rows that share a value.  By
+// bytes / by splitters in us: 2,500 values (two bytes) 123 / 161 at 150,000 rows,
+// 148 / 275 at 1M, 241 / 351 at 5M, 808 / 1393 at 20M; 2^17 values (three) 171 /
+// 302 at 1M, 302 / 647 at 5M; 2^24 (three) 145 / 140 at 150,000, 166 / 195 at 1M;
+// 2^32 (four) 157 / 144 at 150,000, 189 / 202 at 1M, 356 / 421 at 5M; 2^40 (five)
+// 203 / 198 at 1M.  Above 2^23 rows a pass is cheaper still against the splitters
+// (2^25 values, four bytes, 1059 / 1547 at 20M; a float, eight, 1520 / 1315).
+static bool sort_by_bytes(int64_t n, int np) {
+  if (n > kSplitFirst) return np <= 6;
+  return np <= 2 || (np == 3 && n >= (1 << 18)) || (np == 4 && n >= (1 << 19));
+}
+
+// Sort (keys_in, vals_in) ascending by key ^ in_xor, stable, writing
+// (key image ^ out_xor, value) to keys_out / vals_out.  The bits of the keys from
+// key_bits up are the same in every key.  Inputs are not modified and must not
+// alias the outputs.
 int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t* vals_in, int64_t n,
                          uint64_t* keys_out, uint32_t* vals_out, int key_bits, uint64_t in_xor, uint64_t out_xor) {
   if (n <= 0) return BOLT_OK;
@@ -608,42 +653,67 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
   const int passes = (key_bits + kRadixBits - 1) / kRadixBits;
   if (passes < 1 || passes > kMaxPasses) return set_error(BOLT_ERR_PLAN, "radix sort: bad key width %d", key_bits);
   const bool grouped = getenv("BOLT_SORT_LSD") == nullptr;
-  bool split_tried = false;
+  DevBuf<uint64_t> sample;
   auto split = [&](bool* done) -> int {
-    split_tried = true;
-    return split_sort_u64_pairs(s, keys_in, vals_in, n, keys_out, vals_out, in_xor, out_xor, done);
+    BOLT_TRY(split_sort_u64_pairs(s, keys_in, vals_in, n, keys_out, vals_out, in_xor, out_xor, sample, done));
+    if (*done) set_sort_plan(n <= kSplitWhole ? BOLT_SORT_WORKGROUP : BOLT_SORT_SAMPLE, 0);
+    return BOLT_OK;
   };
-  // Up to kSplitFirst rows the splitter sort costs no more than the digit
-  // histogram and its read-back; above, the histogram decides (30M uniform
-  // keys: 1.08 ms by digits, 1.84 ms by splitters; 1.75 ms before, with one
-  // large workgroup per bucket).
-  if (n <= kSplitFirst && grouped) {
+  // Up to kSplitFirst rows the splitter sort, unless a pass over the keys beside
+  // the sample (uniform keys 197 -> 206 us at 1M rows) finds few bytes that vary;
+  // above, the histogram of all bytes decides (30M uniform keys: 1.08 ms by
+  // digits, 1.84 ms by splitters).
+  std::vector<int> todo;  // varying bytes
+  bool known = false;
+  if (n > kSplitOnePass && n <= kSplitFirst && grouped) {
+    DevBuf<uint64_t> one_zero;
+    uint64_t b[2 * kVaryGrid], one = 0, zero = 0;
+    const int vary = (int)grid_for(n, kSampleList, kVaryRows, kVaryGrid);
+    BOLT_TRY(one_zero.alloc(2 * kVaryGrid, s));
+    BOLT_TRY(split_sample(s, keys_in, n, in_xor, sample, one_zero.ptr, vary));
+    BOLT_TRY(read_back(s, {{b, one_zero.ptr, (size_t)vary * 16}}));
+    for (int g = 0; g < vary; g++) {
+      one |= b[2 * g];
+      zero |= b[2 * g + 1];
+    }
+    for (int p = 0; p < passes; p++)
+      if (((one & zero) >> (p * kRadixBits)) & (kBins - 1)) todo.push_back(p);
+    known = true;
+  }
+  if (n <= kSplitFirst && grouped && !(known && sort_by_bytes(n, (int)todo.size()))) {
     bool done = false;
     BOLT_TRY(split(&done));
     if (done) return BOLT_OK;
     // a bucket too large for LDS: LSD passes from the input
   }
+  auto copy_all = [&]() -> int {  // equal keys
+    copy_pairs_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(keys_in, vals_in, keys_out, vals_out, n, in_xor ^ out_xor);
+    BOLT_HIP(hipGetLastError());
+    set_sort_plan(BOLT_SORT_COPY, 0);
+    return BOLT_OK;
+  };
+  if (known && todo.empty()) return copy_all();
   DevBuf<uint32_t> hist, offs, misc;
   BOLT_TRY(hist.alloc((size_t)passes * kBins, s));
   BOLT_TRY(offs.alloc((size_t)passes * kBins, s));
   BOLT_TRY(misc.alloc(4, s));
   BOLT_TRY(fill_u32(hist.ptr, 0, (size_t)passes * kBins, s));
-  radix_hist_kernel<<<grid_for(n, kSortBlock, 16, 2048), kSortBlock, 0, s>>>(keys_in, n, passes, hist.ptr, in_xor);
+  uint32_t digits = known ? 0u : ~0u;
+  for (int p : todo) digits |= 1u << p;
+  radix_hist_kernel<<<grid_for(n, kSortBlock, 16, 2048), kSortBlock, 0, s>>>(keys_in, n, passes, digits, hist.ptr,
+                                                                            in_xor);
   radix_scan_kernel<<<passes, kBins, 0, s>>>(hist.ptr, offs.ptr);
   BOLT_HIP(hipGetLastError());
   std::vector<uint32_t> h((size_t)passes * kBins);
-  BOLT_TRY(read_back(s, {{h.data(), hist.ptr, h.size() * 4}}));
-  std::vector<int> todo;
-  for (int p = 0; p < passes; p++) {
-    bool trivial = false;
-    for (int b = 0; b < kBins; b++)
-      if (h[(size_t)p * kBins + b] == (uint32_t)n) trivial = true;
-    if (!trivial) todo.push_back(p);
-  }
-  if (todo.empty()) {
-    copy_pairs_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(keys_in, vals_in, keys_out, vals_out, n, in_xor ^ out_xor);
-    BOLT_HIP(hipGetLastError());
-    return BOLT_OK;
+  if (!known) {
+    BOLT_TRY(read_back(s, {{h.data(), hist.ptr, h.size() * 4}}));
+    for (int p = 0; p < passes; p++) {
+      bool trivial = false;
+      for (int b = 0; b < kBins; b++)
+        if (h[(size_t)p * kBins + b] == (uint32_t)n) trivial = true;
+      if (!trivial) todo.push_back(p);
+    }
+    if (todo.empty()) return copy_all();
   }
   const int64_t tiles = (n + kSortTile - 1) / kSortTile;
   DevBuf<uint64_t> ktmp;
@@ -668,13 +738,14 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
     return BOLT_OK;
   };
   const int np = (int)todo.size();
-  if (n <= 2 * kSplitMax && grouped && !split_tried) {
+  if (n > kSplitFirst && n <= 2 * kSplitMax && grouped) {
     // largest bucket of the top two varying digits if they were independent
     double most = (double)n;
     for (int q = np - 1; q >= 0 && q >= np - 2; q--)
       most *= (double)*std::max_element(h.begin() + (size_t)todo[q] * kBins, h.begin() + (size_t)(todo[q] + 1) * kBins) /
               (double)n;
-    if (np >= 3 && most <= 0.8 * kSplitMid) {
+    // three bytes up to kSplitMax: their passes (929 us for 20M rows, 1043 here)
+    if (np >= (n <= kSplitMax ? 4 : 3) && most <= 0.8 * kSplitMid) {
       const int p1 = todo[np - 2], p2 = todo[np - 1];
       BOLT_TRY(pass(keys_in, vals_in, ktmp.ptr, vtmp.ptr, p1, in_xor, 0));
       BOLT_TRY(pass(ktmp.ptr, vtmp.ptr, keys_out, vals_out, p2, 0, out_xor));
@@ -689,10 +760,13 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
       uint32_t e[2] = {0, 0};
       BOLT_TRY(read_back(s, {{e, misc.ptr + 1, 8}}));
       if (e[0]) return set_error(BOLT_ERR_OTHER, "radix sort look-back timed out");
-      if (e[1] == 0) return BOLT_OK;
+      if (e[1] == 0) {
+        set_sort_plan(BOLT_SORT_DIGITS, 2);
+        return BOLT_OK;
+      }
     }
     bool done = false;
-    if (n <= kSplitMax) BOLT_TRY(split(&done));
+    if (n <= kSplitMax && !sort_by_bytes(n, np)) BOLT_TRY(split(&done));
     if (done) return BOLT_OK;
   }
   // hybrid: two global passes on the top varying digits, then LDS bucket sorts
@@ -719,11 +793,13 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
       uint32_t e2 = 0;
       BOLT_TRY(read_back(s, {{&e2, misc.ptr + 2, 4}}));
       if (e2) return set_error(BOLT_ERR_OTHER, "radix sort: bucket larger than the LDS sort");
+      set_sort_plan(BOLT_SORT_DIGITS, 2);
       return BOLT_OK;
     }
     // a bucket too large for LDS (skewed keys): plain LSD from the input
   }
   // LSD: one pass per varying digit, ping-pong so the last pass writes the output
+  set_sort_plan(BOLT_SORT_BYTES, np);
   const uint64_t* ksrc = keys_in;
   const uint32_t* vsrc = vals_in;
   for (int q = 0; q < np; q++) {
@@ -1476,6 +1552,12 @@ static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys,
     BOLT_TRY(read_back(s, {{&e, err.ptr, 4}}));
     *done = e == 0;
   }
+  return BOLT_OK;
+}
+
+extern "C" int bolt_sort_last_plan(int32_t* plan, int32_t* passes) {
+  if (plan) *plan = t_sort_plan;
+  if (passes) *passes = t_sort_passes;
   return BOLT_OK;
 }
 

@@ -18,8 +18,8 @@
 //     passes from the untouched input.
 //   * Up to 6,144 rows one workgroup sorts alone: one launch.
 // Uniform int64 keys, whole call, before (LSD or digit buckets) and now: 5,000
-// rows 214 -> 17 us, 20,000 232 -> 93, 100,000 234 -> 107, 1M 304 -> 202, 5M
-// 958 -> 425, 30M 1752 -> 1076 (by digits, with these bucket sorts).
+// rows 214 -> 17 us, 20,000 232 -> 93, 100,000 234 -> 107, 1M 304 -> 206, 5M
+// 958 -> 427, 30M 1752 -> 1076 (by digits, with these bucket sorts).
 #pragma once
 
 namespace bolt {
@@ -80,12 +80,48 @@ __device__ __forceinline__ void lds_bitonic(int size, F cmpx) {
 }
 
 // The sample: one row of each of S equal strata, at a scattered place within
-// it, sorted in lists of 1024.
+// it, sorted in lists of 1024.  The workgroups behind those of the lists, if any,
+// read all keys for the bits that vary: workgroup g's share of the keys has the
+// bits one_zero[2 g] set in some key, one_zero[2 g + 1] clear in some.
 constexpr int kSampleList = 1024;
+constexpr int kVaryRows = 8;      // keys in flight per lane
+constexpr int kVaryGrid = 256;
 __global__ __launch_bounds__(kSampleList) void split_sample_kernel(const uint64_t* __restrict__ keys, int64_t n,
                                                                    uint64_t in_xor, int S,
-                                                                   uint64_t* __restrict__ lists) {
+                                                                   uint64_t* __restrict__ lists,
+                                                                   uint64_t* __restrict__ one_zero) {
   __shared__ uint64_t k[kSampleList];
+  if ((int)blockIdx.x >= S / kSampleList) {
+    const int g = (int)blockIdx.x - S / kSampleList, grid = (int)gridDim.x - S / kSampleList;
+    const int64_t stride = (int64_t)grid * kSampleList;
+    uint64_t one = 0, zero = 0;
+    for (int64_t i0 = (int64_t)g * kSampleList + threadIdx.x; i0 < n; i0 += stride * kVaryRows) {
+      uint64_t x[kVaryRows];
+#pragma unroll
+      for (int u = 0; u < kVaryRows; u++) x[u] = keys[i0 + u * stride < n ? i0 + u * stride : i0];
+#pragma unroll
+      for (int u = 0; u < kVaryRows; u++) {
+        one |= x[u];
+        zero |= ~x[u];
+      }
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      one |= __shfl_xor(one, m);
+      zero |= __shfl_xor(zero, m);
+    }
+    if ((threadIdx.x & 63) == 0) {
+      k[threadIdx.x >> 6] = one;
+      k[64 + (threadIdx.x >> 6)] = zero;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      uint64_t r = 0;
+      for (int w = 0; w < kSampleList / 64; w++) r |= k[64 * threadIdx.x + w];
+      one_zero[2 * g + threadIdx.x] = r;
+    }
+    return;
+  }
   const int j = blockIdx.x * kSampleList + threadIdx.x;
   const int64_t lo = (int64_t)j * n / S, hi = (int64_t)(j + 1) * n / S;
   const uint32_t h = (uint32_t)j * 0x9E3779B1u;

@@ -728,6 +728,13 @@ def sort_pairs_i64(keys: DeviceBuffer, vals: DeviceBuffer, n: int, descending: b
     return ko, vo
 
 
+def sort_last_plan() -> tuple[str, int]:
+    """How the calling thread's last sort of pairs ran, and its passes by bytes (bolt_sort_last_plan)."""
+    plan, passes = C.c_int32(), C.c_int32()
+    N.check(N.lib().bolt_sort_last_plan(C.byref(plan), C.byref(passes)))
+    return ("copy", "bytes", "workgroup", "sample", "digits")[plan.value], passes.value
+
+
 def execute_sort(keys: list[DeviceColumn], descending: list[bool] | None = None,
                  nulls_first: list[bool] | None = None, stream: Stream | None = None) -> np.ndarray:
     """Stable row permutation for ORDER BY keys (numpy u32)."""

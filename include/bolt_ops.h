@@ -331,16 +331,29 @@ int bolt_join(bolt_stream_t stream, const bolt_column_t* left_keys, const bolt_c
 /* ------------------------------------------------------------------------
  * Radix sort — replaces sort_indices_on_gpu_radix{,_multi}
  * (src/exec/gpu_sort.rs:944,995) and run_radix_pipeline_i64 (:1493).
- * Stable.  Up to 2^23 rows (2^25 where the top digits are uneven) buckets from
- * a sample of the keys, sorted in LDS; above, two onesweep passes (LDS ranking
- * + decoupled look-back) over the top varying digits and LDS bucket sorts;
- * onesweep passes over every digit where a bucket does not fit.  n < 2^30.
+ * Stable.  Keys in which few bytes vary take one onesweep pass (LDS ranking +
+ * decoupled look-back) per byte.  Others: up to 2^23 rows (2^25 where the top
+ * bytes are uneven) buckets from a sample of the keys, sorted in LDS; above, two
+ * onesweep passes over the top varying bytes and LDS bucket sorts; passes over
+ * every byte where a bucket does not fit.  n < 2^30.
  * ------------------------------------------------------------------------ */
 
 /* Sort (key, value) pairs by int64 key (ascending unless `descending`).
  * keys_out / vals_out receive the sorted pairs; inputs are not modified. */
 int bolt_sort_pairs_i64(bolt_stream_t stream, const int64_t* keys_in, const uint32_t* vals_in,
                         int64_t n, int32_t descending, int64_t* keys_out, uint32_t* vals_out);
+
+/* How the calling thread's last sort of (key, value) pairs, direct or within
+ * another operator, ran, and its onesweep passes by bytes of the key.  Either
+ * pointer may be NULL. */
+typedef enum {
+  BOLT_SORT_COPY = 0,      /* all keys are equal */
+  BOLT_SORT_BYTES = 1,     /* a pass per varying byte */
+  BOLT_SORT_WORKGROUP = 2, /* by one workgroup */
+  BOLT_SORT_SAMPLE = 3,    /* buckets from a sample */
+  BOLT_SORT_DIGITS = 4     /* buckets from the top two varying bytes */
+} bolt_sort_plan_t;
+int bolt_sort_last_plan(int32_t* plan, int32_t* passes);
 
 /* ORDER BY: stable row permutation for a lexicographic multi-column key
  * (execute_sort, src/exec/sort.rs:161; key transforms of

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from craton_bolt_amd.device import DeviceBuffer, DeviceColumn
-from craton_bolt_amd.ops import sort_pairs_i64
+from craton_bolt_amd.ops import sort_last_plan, sort_pairs_i64
 
 pytestmark = pytest.mark.gpu
 
@@ -66,6 +66,34 @@ def test_split_sort_large(gpu, n, kind):
     order = np.argsort(key, kind="stable")
     assert np.array_equal(ko.to_numpy(np.int64, n), key[order])
     assert np.array_equal(vo.to_numpy(np.uint32, n), order.astype(np.uint32))
+
+
+_ANY = -1  # bytes that vary: all eight
+_MASK = {0: 0, 1: 1, 2: 0x1FF, 3: 0x1FFFF, 4: 0x1FFFFFF, 5: 0x1FFFFFFFF}
+
+
+@pytest.mark.parametrize("n,nbytes,shift,plan", [
+    (131_072, 1, 0, ("sample", 0)), (131_073, 0, 0, ("copy", 0)), (131_073, 1, 56, ("bytes", 1)),
+    (131_073, 2, 0, ("bytes", 2)), (131_073, 3, 0, ("sample", 0)), (262_144, 3, 8, ("bytes", 3)),
+    (524_287, 4, 0, ("sample", 0)), (524_288, 4, 24, ("bytes", 4)), (1 << 23, 5, 0, ("sample", 0)),
+    (1 << 23, 4, 0, ("bytes", 4)), (1 << 23, _ANY, 0, ("sample", 0)), ((1 << 23) + 1, 0, 0, ("copy", 0)),
+    ((1 << 23) + 1, 1, 0, ("bytes", 1)), ((1 << 23) + 1, 3, 0, ("bytes", 3)), ((1 << 23) + 1, 5, 0, ("bytes", 5)),
+    ((1 << 23) + 1, _ANY, 0, ("digits", 2))])
+def test_few_varying_bytes(gpu, n, nbytes, shift, plan):
+    """Keys in which few bytes vary take a pass per byte.  The top varying byte takes two values, so above 2^23
+    rows the top two bytes alone do not separate the rows."""
+    print(f"[case] sort n={n} bytes={nbytes} shift={shift}", flush=True)
+    rng = np.random.default_rng(n + nbytes)
+    key = rng.integers(I64.min, I64.max, n, endpoint=True)
+    if nbytes != _ANY:
+        key = (key & _MASK[nbytes]) << shift
+    rid = np.arange(n, dtype=np.uint32)
+    for desc in (False, True):
+        ko, vo = sort_pairs_i64(DeviceBuffer.from_numpy(key), DeviceBuffer.from_numpy(rid), n, desc)
+        assert sort_last_plan() == plan
+        order = np.argsort(~key if desc else key, kind="stable")
+        assert np.array_equal(ko.to_numpy(np.int64, n), key[order])
+        assert np.array_equal(vo.to_numpy(np.uint32, n), order.astype(np.uint32))
 
 
 @pytest.mark.parametrize("n", [2, 777, 40_000, 600_001])
