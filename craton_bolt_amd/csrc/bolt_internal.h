@@ -106,6 +106,9 @@ struct ReadPart {
 };
 int read_back(hipStream_t s, std::initializer_list<ReadPart> parts);
 
+// Distinct values behind a sample of m with d distinct ones (groupby.hip).
+double sample_groups(double m, double d);
+
 // Graph-capture-safe fill (a kernel, never hipMemsetAsync).
 int fill_u32(void* dst, uint32_t value, size_t n_words, hipStream_t s);
 int fill_u8(void* dst, uint8_t value, size_t n, hipStream_t s);

@@ -804,6 +804,19 @@ double bolt::hll_estimate(const uint32_t* regs) {
   return e;
 }
 
+// Groups that a sample of m keys with d distinct ones stands for, if they are
+// about equally frequent: the G with G (1 - exp(-m / G)) = d.
+double bolt::sample_groups(double m, double d) {
+  if (d >= m) return 1e18;
+  double lo = d, hi = 1e12;
+  for (int i = 0; i < 100; i++) {
+    const double g = std::sqrt(lo * hi);
+    if (g * -std::expm1(-m / g) < d) lo = g;
+    else hi = g;
+  }
+  return lo;
+}
+
 uint64_t bolt::next_pow2(uint64_t x) {
   uint64_t p = 1;
   while (p < x) p <<= 1;
@@ -862,19 +875,6 @@ struct GbPartCopy {
   GbJitSpec spec;      // the LDS tier's kernel over the copies
   JitCols cols;
 };
-
-// Groups that a sample of m keys with d distinct ones stands for, if they are
-// about equally frequent: the G with G (1 - exp(-m / G)) = d.
-static double sample_groups(double m, double d) {
-  if (d >= m) return 1e18;
-  double lo = d, hi = 1e12;
-  for (int i = 0; i < 100; i++) {
-    const double g = std::sqrt(lo * hi);
-    if (g * -std::expm1(-m / g) < d) lo = g;
-    else hi = g;
-  }
-  return lo;
-}
 
 // Groups that the partitions' tables of part_S slots take.
 static double part_groups_most(int part_S) { return kGbPartLoad * part_S * (1 << kGbPartBits); }

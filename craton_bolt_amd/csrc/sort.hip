@@ -538,23 +538,54 @@ static int split_samples(int64_t n) {
   const int cbits = split_code_bits(n);
   return cbits == 6 ? kSampleList : cbits <= 12 ? 4096 : 16384;
 }
-// Allocates the sample (and the room for its merge) and draws it; `vary`
-// workgroups more look for varying bits.
-static int split_sample(hipStream_t s, const uint64_t* keys, int64_t n, uint64_t in_xor, DevBuf<uint64_t>& sample,
+// A sort's sample: S keys in sorted lists, then as one list.
+struct SplitSample {
+  DevBuf<uint64_t> keys;  // [2 S]
+  const uint64_t* sorted = nullptr;
+};
+// Draws the sample; `vary` workgroups more look for varying bits.
+static int split_sample(hipStream_t s, const uint64_t* keys, int64_t n, uint64_t in_xor, SplitSample& sample,
                         uint64_t* one_zero, int vary) {
   const int S = split_samples(n);
-  BOLT_TRY(sample.alloc((size_t)2 * S, s));
-  split_sample_kernel<<<S / kSampleList + vary, kSampleList, 0, s>>>(keys, n, in_xor, S, sample.ptr, one_zero);
+  BOLT_TRY(sample.keys.alloc((size_t)2 * S, s));
+  split_sample_kernel<<<S / kSampleList + vary, kSampleList, 0, s>>>(keys, n, in_xor, S, sample.keys.ptr, one_zero);
   BOLT_HIP(hipGetLastError());
   return BOLT_OK;
 }
+// Draws it unless that is done, and merges its lists.
+static int split_sorted_sample(hipStream_t s, const uint64_t* keys, int64_t n, uint64_t in_xor, SplitSample& sample) {
+  if (sample.sorted) return BOLT_OK;
+  if (!sample.keys.ptr) BOLT_TRY(split_sample(s, keys, n, in_xor, sample, nullptr, 0));
+  const int S = split_samples(n);
+  uint64_t* lists = sample.keys.ptr;
+  if (S > 4096) split_merge_kernel<16><<<S / 64, 64, 0, s>>>(lists, lists + S);
+  else if (S > kSampleList) split_merge_kernel<4><<<S / 64, 64, 0, s>>>(lists, lists + S);
+  BOLT_HIP(hipGetLastError());
+  sample.sorted = S > kSampleList ? lists + S : lists;
+  return BOLT_OK;
+}
+// Rows that share a value, by the sample, if the values are about equally
+// frequent.
+static int split_rows_per_value(hipStream_t s, const uint64_t* keys, int64_t n, uint64_t in_xor, SplitSample& sample,
+                                double* rows) {
+  const int S = split_samples(n);
+  DevBuf<uint32_t> out;
+  uint32_t distinct = 0;
+  BOLT_TRY(out.alloc(1, s));
+  BOLT_TRY(split_sorted_sample(s, keys, n, in_xor, sample));
+  split_distinct_kernel<<<1, 1024, 0, s>>>(sample.sorted, S, out.ptr);
+  BOLT_HIP(hipGetLastError());
+  BOLT_TRY(read_back(s, {{&distinct, out.ptr, 4}}));
+  *rows = (double)n / sample_groups(S, distinct);
+  return BOLT_OK;
+}
 
-// The splitter sort of 2 <= n <= kSplitMax pairs (`sample` drawn, or empty).  *done = false when a bucket
+// The splitter sort of 2 <= n <= kSplitMax pairs (`sample` may be drawn).  *done = false when a bucket
 // of different keys exceeded the LDS sort (keys_out / vals_out then hold
 // nothing of use; the inputs are untouched).
 static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t* vals_in, int64_t n,
                                 uint64_t* keys_out, uint32_t* vals_out, uint64_t in_xor, uint64_t out_xor,
-                                DevBuf<uint64_t>& sample, bool* done) {
+                                SplitSample& sample, bool* done) {
   *done = true;
   if (n <= kSplitWhole) {
     split_whole_kernel<<<1, 1024, 0, s>>>(keys_in, vals_in, keys_out, vals_out, (int)n, in_xor, out_xor);
@@ -570,7 +601,7 @@ static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const ui
   DevBuf<uint32_t> vtmp, words, start;
   DevBuf<uint16_t> codes;
   DevBuf<uint8_t> digits;
-  if (!sample.ptr) BOLT_TRY(split_sample(s, keys_in, n, in_xor, sample, nullptr, 0));
+  BOLT_TRY(split_sorted_sample(s, keys_in, n, in_xor, sample));
   BOLT_TRY(codes.alloc((size_t)n, s));
   // counts, scanned counts, tickets and error, then the look-back words of
   // each pass: one fill
@@ -582,9 +613,7 @@ static int split_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const ui
   uint32_t* offs = words.ptr + 512;
   uint32_t* misc = offs + 514;
   uint32_t* status = words.ptr + head;
-  const Splitters sp{S == kSampleList ? sample.ptr : sample.ptr + S, S, std::min(C, S), std::max(cbits - 14, 0)};
-  if (S > 4096) split_merge_kernel<16><<<S / 64, 64, 0, s>>>(sample.ptr, sample.ptr + S);
-  else if (S > kSampleList) split_merge_kernel<4><<<S / 64, 64, 0, s>>>(sample.ptr, sample.ptr + S);
+  const Splitters sp{sample.sorted, S, std::min(C, S), std::max(cbits - 14, 0)};
   const size_t lds = (size_t)(sp.G + 1) * 8;
   BOLT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(split_code_kernel),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -653,7 +682,7 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
   const int passes = (key_bits + kRadixBits - 1) / kRadixBits;
   if (passes < 1 || passes > kMaxPasses) return set_error(BOLT_ERR_PLAN, "radix sort: bad key width %d", key_bits);
   const bool grouped = getenv("BOLT_SORT_LSD") == nullptr;
-  DevBuf<uint64_t> sample;
+  SplitSample sample;
   auto split = [&](bool* done) -> int {
     BOLT_TRY(split_sort_u64_pairs(s, keys_in, vals_in, n, keys_out, vals_out, in_xor, out_xor, sample, done));
     if (*done) set_sort_plan(n <= kSplitWhole ? BOLT_SORT_WORKGROUP : BOLT_SORT_SAMPLE, 0);
@@ -766,7 +795,15 @@ int radix_sort_u64_pairs(hipStream_t s, const uint64_t* keys_in, const uint32_t*
       }
     }
     bool done = false;
-    if (n <= kSplitMax && !sort_by_bytes(n, np)) BOLT_TRY(split(&done));
+    if (n <= kSplitMax && !sort_by_bytes(n, np)) {
+      // Up to a bucket's rows on one value leave the buckets to LDS networks; from
+      // there on values have buckets of their own.  20M floats in cents, by bytes
+      // 1470 us: one row a value 1413 by splitters, 3 rows 1564, 12 2175, 100 2078,
+      // 700 1609, 1000 1323; 33M, by bytes 2400: 1 2181, 3 2398, 100 3783, 1000 2638.
+      double rows = 0;
+      BOLT_TRY(split_rows_per_value(s, keys_in, n, in_xor, sample, &rows));
+      if (rows < 2.5 || rows > 800.0) BOLT_TRY(split(&done));
+    }
     if (done) return BOLT_OK;
   }
   // hybrid: two global passes on the top varying digits, then LDS bucket sorts

@@ -169,6 +169,22 @@ __global__ __launch_bounds__(64) void split_merge_kernel(const uint64_t* __restr
   sorted[r] = k;
 }
 
+// *out = the sample's distinct keys.
+__global__ __launch_bounds__(1024) void split_distinct_kernel(const uint64_t* __restrict__ sorted, int S,
+                                                              uint32_t* __restrict__ out) {
+  __shared__ uint32_t wsum[16];
+  uint32_t c = 0;
+  for (int i = threadIdx.x; i < S; i += 1024) c += i == 0 || sorted[i] != sorted[i - 1] ? 1u : 0u;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) c += __shfl_xor(c, m);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) c += wsum[w];
+    *out = c;
+  }
+}
+
 // Code of every key, and the counts of both digits of the codes (hist[0..255]:
 // the low b1 bits, hist[256..511]: the rest).  Bound by the LDS searches, 6 to
 // 14 dependent reads a key, four keys in flight per lane.

@@ -96,6 +96,23 @@ def test_few_varying_bytes(gpu, n, nbytes, shift, plan):
         assert np.array_equal(vo.to_numpy(np.uint32, n), order.astype(np.uint32))
 
 
+@pytest.mark.parametrize("rows,plan", [(1, ("sample", 0)), (10, ("bytes", 8)), (400, ("bytes", 8)),
+                                       (2000, ("sample", 0))])
+def test_values_shared_by_rows(gpu, rows, plan):
+    """Above 2^23 rows, floats whose exponents leave the top two bytes uneven: values of a few to a few hundred
+    rows take passes by bytes, the sample's buckets are left with the others."""
+    n = 9_000_001
+    print(f"[case] sort rows per value={rows}", flush=True)
+    rng = np.random.default_rng(rows)
+    key = (rng.integers(0, n // rows, n) / 100.0).view(np.int64)
+    rid = np.arange(n, dtype=np.uint32)
+    ko, vo = sort_pairs_i64(DeviceBuffer.from_numpy(key), DeviceBuffer.from_numpy(rid), n)
+    assert sort_last_plan() == plan
+    order = np.argsort(key, kind="stable")
+    assert np.array_equal(ko.to_numpy(np.int64, n), key[order])
+    assert np.array_equal(vo.to_numpy(np.uint32, n), order.astype(np.uint32))
+
+
 @pytest.mark.parametrize("n", [2, 777, 40_000, 600_001])
 @pytest.mark.parametrize("shape", ["fits", "cut", "ties", "long_ties", "constant"])
 def test_order_by_packed(gpu, n, shape):
