@@ -901,15 +901,17 @@ __global__ void order_key_kernel(const void* __restrict__ d, const uint8_t* __re
 
 // ---- multi-column ORDER BY as one sort ---------------------------------------------
 //
-// Every ORDER BY key is one or two fields (its NULL rank, its value; a
-// Decimal128 value is its signed high word, then its low word), each an
-// unsigned image that ascends along the order.  The fields' images, less their
-// smallest value, are packed most significant first into one 64-bit key, so a
-// single sort orders all columns: 0.76 ms for a nullable date and a float over
-// 5M rows, where one sort per field, each reading its column through the
-// permutation so far, took 1.25 ms (and 1.60 ms with LSD passes).  When the
-// fields need more than 64 bits the last one that fits is cut, and runs of rows
-// that agree on all 64 bits are put in order by the full columns afterwards.
+// Every ORDER BY key is one or two fields (its NULL rank, its value; a Decimal128
+// value is its signed high word, then its low word), each an unsigned image that
+// ascends along the order.  The fields' images, less their smallest value, are
+// packed most significant first into one 64-bit key, so a single sort orders all
+// columns: 0.71 ms for a nullable date and a float over 5M rows, where one sort
+// per field, each reading its column through the permutation so far, took 1.60 ms.
+// When the fields need more than 64 bits the last one that fits is cut.  Rows that
+// agree on all 64 bits are then put in order run by run where the runs are short
+// and few (tie_order_kernel).  Elsewhere the keys are replaced by their rank
+// (rank_pack_kernel), which leaves room for the next bits, and sorted again: a
+// sort per 64 bits or so, not per field.
 constexpr int kMaxFields = 16;
 enum { kFieldValue = 0, kFieldNull = 1, kFieldDecHigh = 2 };
 struct OrderField {
@@ -917,8 +919,8 @@ struct OrderField {
   const uint8_t* v;
   uint64_t min;      // smallest image of a valid row
   int32_t dt, kind, bits, desc, nulls_first;
-  int32_t width;     // bits of the packed key
-  int32_t drop;      // low bits of the image left out of it
+  int32_t width;     // bits in the packed key
+  int32_t drop;      // the image's bits below those
 };
 struct OrderFields {
   OrderField f[kMaxFields];
@@ -977,6 +979,13 @@ __global__ __launch_bounds__(256) void field_range_kernel(OrderFields of, int64_
   }
 }
 
+// The bits of field f (width > 0) that the packed key holds.
+__device__ __forceinline__ uint64_t field_bits(const OrderField& f, int64_t row) {
+  if (f.kind == kFieldNull) return null_rank(f, row);
+  const uint64_t x = bit_valid(f.v, row) ? (field_image(f, row) - f.min) >> f.drop : 0ull;
+  return f.width < 64 ? x & ((1ull << f.width) - 1) : x;
+}
+
 // key[i] = the packed fields of row i, rows[i] = i.
 __global__ __launch_bounds__(256) void pack_fields_kernel(OrderFields of, int64_t n, uint64_t* __restrict__ key,
                                                           uint32_t* __restrict__ rows) {
@@ -988,12 +997,7 @@ __global__ __launch_bounds__(256) void pack_fields_kernel(OrderFields of, int64_
       if (f.width == 0) continue;  // constant, or beyond the packed bits
       uint64_t x[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int64_t i = i0 + u * stride < n ? i0 + u * stride : i0;
-        x[u] = f.kind == kFieldNull ? null_rank(f, i)
-               : bit_valid(f.v, i)  ? (field_image(f, i) - f.min) >> f.drop
-                                    : 0ull;
-      }
+      for (int u = 0; u < 4; u++) x[u] = field_bits(f, i0 + u * stride < n ? i0 + u * stride : i0);
 #pragma unroll
       for (int u = 0; u < 4; u++) k[u] = f.width < 64 ? (k[u] << f.width) | x[u] : x[u];
     }
@@ -1008,10 +1012,56 @@ __global__ __launch_bounds__(256) void pack_fields_kernel(OrderFields of, int64_
   }
 }
 
+// Sorted keys that packed rows share.  Workgroup g looks at rows [g * per,
+// (g + 1) * per): heads[g] = the runs of equal keys that start there, work[g] =
+// the sum of the squares of the lengths of those of two to kTieRun rows, which is
+// what tie_order_kernel's insertion sorts cost; a longer run makes it kTieNever.
+constexpr int kTieRun = 64;
+constexpr int kTieGrid = 1024;
+// Work a row up to which runs are put in order one by one: about three rows a
+// value.  Two floats over 5M rows, by runs / by ranks in us: 1 row a value of the
+// first 647 / 1117, 2 924 / 1188, 4 1322 / 1325, 8 2222 / 1519, 20 5211 / 1549 (a
+// sort per field 1660); 500,000 rows: 2 360 / 461, 4 490 / 502, 8 723 / 523.
+constexpr double kTieWork = 4.0;
+constexpr unsigned long long kTieNever = 1ull << 50;  // kTieGrid of them fit 64 bits
+__global__ __launch_bounds__(256) void tie_count_kernel(const uint64_t* __restrict__ key, int64_t n, int64_t per,
+                                                        uint32_t* __restrict__ heads,
+                                                        unsigned long long* __restrict__ work) {
+  const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < n ? lo + per : n;
+  uint32_t h = 0;
+  unsigned long long w = 0;
+  for (int64_t i = lo + threadIdx.x; i < hi; i += 256) {
+    const uint64_t k = key[i];
+    if (i > 0 && key[i - 1] == k) continue;
+    h++;
+    int len = 1;
+    while (len <= kTieRun && i + len < n && key[i + len] == k) len++;
+    if (len > kTieRun) w = kTieNever;
+    else if (len > 1 && w < kTieNever) w += (unsigned long long)(len * len);
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    h += __shfl_xor(h, m);
+    w += __shfl_xor(w, m);
+  }
+  __shared__ uint32_t sh[4];
+  __shared__ unsigned long long sw[4];
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = h;
+    sw[threadIdx.x >> 6] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    heads[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+    w = sw[0] + sw[1] + sw[2] + sw[3];
+    work[blockIdx.x] = w < kTieNever ? w : kTieNever;
+  }
+}
+
 // Rows that agree on the packed key, in row order: the first of each run sorts
 // it by the fields that the key does not hold whole (an insertion sort, which
-// keeps equal rows in row order).  A run above kTieRun rows sets *err.
-constexpr int kTieRun = 64;
+// keeps equal rows in row order).  Does nothing, and sets res[0], where
+// tie_count_kernel found more than `limit` work; res[1] = the runs.
 __device__ __forceinline__ int cmp_rows(const OrderFields& of, int first, uint32_t a, uint32_t b) {
   for (int q = first; q < of.n; q++) {
     const OrderField& f = of.f[q];
@@ -1029,17 +1079,39 @@ __device__ __forceinline__ int cmp_rows(const OrderFields& of, int first, uint32
 }
 __global__ __launch_bounds__(256) void tie_order_kernel(OrderFields of, int first, const uint64_t* __restrict__ key,
                                                         int64_t n, uint32_t* __restrict__ rows,
-                                                        uint32_t* __restrict__ err) {
+                                                        const uint32_t* __restrict__ heads,
+                                                        const unsigned long long* __restrict__ work, int chunks,
+                                                        unsigned long long limit, uint32_t* __restrict__ res) {
+  __shared__ uint32_t sh[4];
+  __shared__ unsigned long long sw[4];
+  uint32_t h = 0;
+  unsigned long long w = 0;
+  for (int c = threadIdx.x; c < chunks; c += 256) {
+    h += heads[c];
+    w += work[c];
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    h += __shfl_xor(h, m);
+    w += __shfl_xor(w, m);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = h;
+    sw[threadIdx.x >> 6] = w;
+  }
+  __syncthreads();
+  w = sw[0] + sw[1] + sw[2] + sw[3];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    res[0] = w > limit ? 1u : 0u;
+    res[1] = sh[0] + sh[1] + sh[2] + sh[3];
+  }
+  if (w == 0 || w > limit) return;  // block-uniform
   const int64_t stride = (int64_t)gridDim.x * 256;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i + 1 < n; i += stride) {
     const uint64_t k = key[i];
     if (key[i + 1] != k || (i > 0 && key[i - 1] == k)) continue;
     int len = 2;
-    while (len <= kTieRun && i + len < n && key[i + len] == k) len++;
-    if (len > kTieRun) {
-      *err = 1u;
-      continue;
-    }
+    while (i + len < n && key[i + len] == k) len++;
     for (int x = 1; x < len; x++) {
       const uint32_t r = rows[i + x];
       int y = x - 1;
@@ -1049,6 +1121,41 @@ __global__ __launch_bounds__(256) void tie_order_kernel(OrderFields of, int firs
       }
       rows[i + y + 1] = r;
     }
+  }
+}
+
+// next[i] = the rank of key[i] among the distinct keys, then the fields' next
+// bits of row rows[i].  Workgroups as tie_count_kernel's.
+__global__ __launch_bounds__(256) void rank_pack_kernel(OrderFields of, const uint64_t* __restrict__ key, int64_t n,
+                                                        int64_t per, const uint32_t* __restrict__ heads,
+                                                        const uint32_t* __restrict__ rows,
+                                                        uint64_t* __restrict__ next) {
+  __shared__ uint32_t sh[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t before = 0;  // runs before this workgroup's rows
+  for (int c = threadIdx.x; c < (int)blockIdx.x; c += 256) before += heads[c];
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m);
+  if (lane == 0) sh[wave] = before;
+  __syncthreads();
+  before = sh[0] + sh[1] + sh[2] + sh[3];
+  const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < n ? lo + per : n;
+  for (int64_t base = lo; base < hi; base += 256) {
+    const int64_t i = base + threadIdx.x;
+    const bool head = i < hi && (i == 0 || key[i] != key[i - 1]);
+    const uint64_t b = __ballot(head);
+    __syncthreads();  // sh is read
+    if (lane == 0) sh[wave] = (uint32_t)__popcll(b);
+    __syncthreads();
+    uint32_t rank = before + (uint32_t)__popcll(b & (~0ull >> (63 - lane)));  // runs up to this row's
+    for (int w = 0; w < wave; w++) rank += sh[w];
+    before += sh[0] + sh[1] + sh[2] + sh[3];
+    if (i >= hi) continue;
+    uint64_t k = rank - 1;
+    const int64_t row = rows[i];
+    for (int q = 0; q < of.n; q++)
+      if (of.f[q].width) k = of.f[q].width < 64 ? (k << of.f[q].width) | field_bits(of.f[q], row) : field_bits(of.f[q], row);
+    next[i] = k;
   }
 }
 
@@ -1508,9 +1615,8 @@ extern "C" int bolt_sort_pairs_i64(bolt_stream_t stream, const int64_t* keys_in,
   return BOLT_OK;
 }
 
-// ORDER BY as one sort of packed keys.  *done = false when it does not apply
-// (too many fields, or a long run of rows that agree on the packed bits only):
-// the caller then sorts field by field.
+// ORDER BY by packed keys.  *done = false when there are too many fields: the
+// caller then sorts field by field.
 static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys, const int32_t* descending,
                        const int32_t* nulls_first, int64_t n, uint64_t* k0, uint64_t* k1, uint32_t* p0,
                        uint32_t* out_rows, bool* done) {
@@ -1529,11 +1635,11 @@ static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys,
     f.nulls_first = nulls_first ? nulls_first[k] : 1;
     if (c.validity) {
       f.kind = kFieldNull;
-      f.width = f.bits = 1;
+      f.bits = 1;
       of.f[of.n++] = f;
       total += 1;
     }
-    f.bits = f.width = c.dtype == BOLT_BOOL ? 1 : c.dtype == BOLT_DEC128 ? 64 : dtype_size(c.dtype) * 8;
+    f.bits = c.dtype == BOLT_BOOL ? 1 : c.dtype == BOLT_DEC128 ? 64 : dtype_size(c.dtype) * 8;
     if (c.dtype == BOLT_DEC128) {
       f.kind = kFieldDecHigh;
       of.f[of.n++] = f;
@@ -1541,9 +1647,10 @@ static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys,
     }
     f.kind = kFieldValue;
     of.f[of.n++] = f;
-    total += f.width;
+    total += f.bits;
   }
-  int cut = of.n;  // first field that the packed key does not hold whole
+  int rest[kMaxFields];  // bits of each field that no key has held yet
+  for (int q = 0; q < of.n; q++) rest[q] = of.f[q].bits;
   if (total > 64) {
     // the fields' own ranges: a date, a count or the high word of a decimal
     // needs far fewer bits than its type
@@ -1554,42 +1661,58 @@ static int sort_packed(hipStream_t s, const bolt_column_t* keys, int32_t n_keys,
     field_range_kernel<<<dim3(grid_for(n, 256, 4, 1024), of.n), 256, 0, s>>>(of, n, range.ptr);
     BOLT_HIP(hipGetLastError());
     BOLT_TRY(read_back(s, {{h, range.ptr, sizeof h}}));
-    int left = 64;
-    total = 0;
     for (int q = 0; q < of.n; q++) {
       OrderField& f = of.f[q];
-      if (f.kind != kFieldNull) {
-        const uint64_t lo = ~(uint64_t)h[2 * q], hi = h[2 * q + 1];
-        f.min = lo <= hi ? lo : 0;  // no valid row: every image is skipped
-        const uint64_t r = lo <= hi ? hi - lo : 0;
-        f.width = r ? 64 - __builtin_clzll(r) : 0;
-      }
-      if (cut < of.n) {
-        f.width = 0;
-      } else if (f.width > left) {
-        cut = q;
-        f.drop = f.width - left;
-        f.width = left;
-      }
-      left -= f.width;
-      total += f.width;
+      if (f.kind == kFieldNull) continue;
+      const uint64_t lo = ~(uint64_t)h[2 * q], hi = h[2 * q + 1];
+      f.min = lo <= hi ? lo : 0;  // no valid row: every image is skipped
+      const uint64_t r = lo <= hi ? hi - lo : 0;
+      rest[q] = r ? 64 - __builtin_clzll(r) : 0;
     }
   }
+  // the next `left` bits of the fields to the next key; how many there were
+  auto take = [&](int left) -> int {
+    int taken = 0;
+    for (int q = 0; q < of.n; q++) {
+      OrderField& f = of.f[q];
+      f.width = std::min(rest[q], left - taken);
+      f.drop = rest[q] -= f.width;
+      taken += f.width;
+    }
+    return taken;
+  };
+  total = take(64);
   pack_fields_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(of, n, k0, p0);
   BOLT_HIP(hipGetLastError());
   BOLT_TRY(radix_sort_u64_pairs(s, k0, p0, n, k1, out_rows, std::max(total, 1), 0, 0));
   *done = true;
-  if (cut < of.n) {
-    DevBuf<uint32_t> err;
-    uint32_t e = 0;
-    BOLT_TRY(err.alloc(1, s));
-    BOLT_TRY(fill_u32(err.ptr, 0, 1, s));
-    tie_order_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(of, cut, k1, n, out_rows, err.ptr);
+  const int64_t per = (n + kTieGrid - 1) / kTieGrid;
+  const int chunks = (int)((n + per - 1) / per);
+  DevBuf<uint32_t> heads;
+  DevBuf<unsigned long long> work;
+  for (;;) {
+    int first = 0;
+    while (first < of.n && rest[first] == 0) first++;
+    if (first == of.n) return BOLT_OK;
+    if (!heads.ptr) {
+      BOLT_TRY(heads.alloc(kTieGrid + 2, s));
+      BOLT_TRY(work.alloc(kTieGrid, s));
+    }
+    uint32_t* res = heads.ptr + kTieGrid;
+    uint32_t h[2];
+    tie_count_kernel<<<chunks, 256, 0, s>>>(k1, n, per, heads.ptr, work.ptr);
+    tie_order_kernel<<<grid_for(n, 256, 4), 256, 0, s>>>(of, first, k1, n, out_rows, heads.ptr, work.ptr, chunks,
+                                                        (unsigned long long)(kTieWork * (double)n), res);
     BOLT_HIP(hipGetLastError());
-    BOLT_TRY(read_back(s, {{&e, err.ptr, 4}}));
-    *done = e == 0;
+    BOLT_TRY(read_back(s, {{h, res, 8}}));
+    if (h[0] == 0) return BOLT_OK;
+    const int rank_bits = h[1] > 1 ? 32 - __builtin_clz(h[1] - 1) : 0;
+    total = take(64 - rank_bits);
+    rank_pack_kernel<<<chunks, 256, 0, s>>>(of, k1, n, per, heads.ptr, out_rows, k0);
+    BOLT_HIP(hipGetLastError());
+    BOLT_TRY(radix_sort_u64_pairs(s, k0, out_rows, n, k1, p0, std::max(rank_bits + total, 1), 0, 0));
+    BOLT_HIP(hipMemcpyAsync(out_rows, p0, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
   }
-  return BOLT_OK;
 }
 
 extern "C" int bolt_sort_last_plan(int32_t* plan, int32_t* passes) {

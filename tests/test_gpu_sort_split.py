@@ -114,11 +114,12 @@ def test_values_shared_by_rows(gpu, rows, plan):
 
 
 @pytest.mark.parametrize("n", [2, 777, 40_000, 600_001])
-@pytest.mark.parametrize("shape", ["fits", "cut", "ties", "long_ties", "constant"])
+@pytest.mark.parametrize("shape", ["fits", "cut", "pairs", "ties", "long_ties", "one_run", "deep", "constant"])
 def test_order_by_packed(gpu, n, shape):
-    """ORDER BY as one sort of packed keys: all fields fit in 64 bits, the last
-    one is cut, short runs agree on all packed bits, runs too long to be fixed
-    in place (field by field instead), and fields without a range."""
+    """ORDER BY by packed keys: all fields fit in 64 bits, the last one is cut,
+    runs that agree on all packed bits, few and short (put in order in place),
+    many, long, one of them too long (ranks and the next bits instead), several
+    times over, and fields without a range."""
     import oracle as O
     from craton_bolt_amd import _native as N
     from craton_bolt_amd.ops import execute_sort
@@ -139,6 +140,15 @@ def test_order_by_packed(gpu, n, shape):
     elif shape == "ties":  # the second key differs only below the packed bits
         cols = [both(wide[rng.integers(0, max(n // 8, 1), n)], N.F64, None),
                 both(1.0 + rng.integers(0, 4, n) * 2.0 ** -52, N.F64, vb)]
+    elif shape == "pairs":
+        cols = [both(wide[rng.permutation(n) // 2], N.F64, va), both(wide[::-1].copy(), N.F64, vb)]
+    elif shape == "one_run":  # 64 rows are put in order in place, 65 are not
+        k = np.arange(n, dtype=np.int64) * (2 ** 62 // n)
+        k[rng.permutation(n)[:65]] = 5
+        cols = [both(k[rng.permutation(n)], N.I64, None), both(rng.integers(-2 ** 62, 2 ** 62, n), N.I64, vb)]
+    elif shape == "deep":  # few values over all bits of every key
+        few = rng.integers(-2 ** 63, 2 ** 63 - 1, 5)
+        cols = [both(few[rng.integers(0, 5, n)], N.I64, v) for v in (va, None, vb)] + [both(wide, N.F64, None)]
     elif shape == "long_ties":
         cols = [both(np.where(rng.random(n) < 0.5, 1e-300, -1e300), N.F64, va),
                 both(np.where(rng.random(n) < 0.5, 1e-200, -1e200), N.F64, vb)]
@@ -150,3 +160,18 @@ def test_order_by_packed(gpu, n, shape):
         got = execute_sort([x for x, _ in cols], desc, nf)
         want = O.sort_indices([h for _, h in cols], desc, nf)
         assert np.array_equal(got, want)
+
+
+def test_order_by_few_values_first(gpu):
+    """A float of two values, then a float: the second sort's key is the first's rank and the next bits (61 of
+    them), where sorting field by field ended with the two values alone, in two bytes."""
+    from craton_bolt_amd import _native as N
+    from craton_bolt_amd.ops import execute_sort
+
+    n = 600_001
+    print("[case] packed order, few values first", flush=True)
+    rng = np.random.default_rng(11)
+    a, x = rng.integers(0, 2, n).astype(np.float64), rng.random(n)
+    got = execute_sort([DeviceColumn.from_numpy(a, N.F64), DeviceColumn.from_numpy(x, N.F64)], [False, True], [True, True])
+    assert sort_last_plan() == ("sample", 0)
+    assert np.array_equal(got, np.lexsort((-x, a)))
