@@ -13,7 +13,8 @@ import numpy as np
 import pytest
 
 from craton_bolt_amd import _native as N
-from craton_bolt_amd.ops import Term, groupby_last_plan
+from craton_bolt_amd.device import DeviceColumn
+from craton_bolt_amd.ops import Term, execute_groupby, groupby_last_plan
 
 from gpu_util import dec_array
 from test_gpu_groupby import run_both
@@ -45,6 +46,11 @@ def _key(kind, n, groups, rng):
         return [(g.astype(np.float32), N.F32, None)], [N.F32]
     if kind == "dec":
         return [(dec_array([int(x) - 5 for x in g]), N.DEC128, None)], [N.DEC128]
+    if kind in ("null_i64", "clash_i64"):  # clash: the NULL group beside a key of its packed value
+        k = g * 0x9E3779B97F4A7 - 1
+        if kind == "clash_i64":
+            k[g == 2] = 2 ** 63 - 1
+        return [(k.astype(np.int64), N.I64, rng.random(n) > 0.3)], [N.I64]
     if kind == "null_i32":
         return [(g.astype(np.int32), N.I32, rng.random(n) > 0.3)], [N.I32]
     a, b = (g % 50).astype(np.int32), (g // 50).astype(np.int32)
@@ -54,7 +60,8 @@ def _key(kind, n, groups, rng):
 
 
 @pytest.mark.parametrize("n", [1, 4095, 4097, 100_003])
-@pytest.mark.parametrize("kind", ["i64", "i32", "date", "f64", "f32", "null_i32", "pair", "null_pair"])
+@pytest.mark.parametrize("kind", ["i64", "i32", "date", "f64", "f32", "null_i32", "null_i64", "clash_i64", "pair",
+                                  "null_pair"])
 def test_key_forms(gpu, n, kind):
     print(f"[case] key partition {kind} n={n}", flush=True)
     rng = np.random.default_rng(n)
@@ -63,6 +70,30 @@ def test_key_forms(gpu, n, kind):
     x = rng.normal(size=n)
     run_both(keys, [(v, N.I64, None), (x, N.F64, rng.random(n) > 0.2)],
              [(N.SUM, 0), (N.COUNT_STAR, 0), (N.MIN, 0), (N.MAX, 1), (N.SUM, 1), (N.COUNT, 1)], kdt)
+
+
+@pytest.mark.parametrize("nullable", [False, True])
+@pytest.mark.parametrize("n", [1, 4097, 100_003])
+def test_decimal_keys(gpu, n, nullable):
+    """The copy keeps the low word of a Decimal128 key, the extraction widens it again (-5 to 11,000, -1 and 0
+    among them; NULL rows hold high words of any value): as the same keys in 64 bits."""
+    print(f"[case] key partition dec n={n} nullable={nullable}", flush=True)
+    rng = np.random.default_rng(n)
+    (dec, _, _), = _key("dec", n, max(2, n // 9), rng)[0]
+    valid = rng.random(n) > 0.3 if nullable else None
+    v = rng.integers(-1000, 1000, n).astype(np.int64)
+    aggs = [(N.SUM, 0), (N.COUNT_STAR, 0), (N.MAX, 0)]
+    want, _ = run_both([(dec[:, 0].copy(), N.I64, valid)], [(v, N.I64, None)], aggs, [N.I64])
+    if nullable:
+        dec[~valid, 1] = 77
+    got = execute_groupby([DeviceColumn.from_numpy(dec, N.DEC128, valid)], [DeviceColumn.from_numpy(v)], aggs)
+    assert got["n_groups"] == want["n_groups"]
+    (gk, gv), (wk, wv) = got["keys"][0], want["keys"][0]
+    live = np.ones(len(wk), bool) if wv is None else wv
+    assert (gv is None) == (wv is None) and (gv is None or np.array_equal(gv, wv))
+    assert np.array_equal(gk[live, 0], wk[live]) and np.array_equal(gk[live, 1], wk[live] >> 63)
+    for (g, _), (w, _) in zip(got["aggs"], want["aggs"]):
+        assert np.array_equal(g, w)
 
 
 @pytest.mark.parametrize("n", [60_001])

@@ -7,9 +7,10 @@ import pytest
 
 import oracle as O
 from craton_bolt_amd import _native as N
+from craton_bolt_amd.device import DeviceColumn
 from craton_bolt_amd.ops import execute_sort_limit
 
-from gpu_util import both, dec_array
+from gpu_util import both
 
 pytestmark = pytest.mark.gpu
 
@@ -24,12 +25,14 @@ def _check(cols, desc, nf, limit, offset):
     assert np.array_equal(got, O.sort_limit([h for _, h in cols], desc, nf, limit, offset))
 
 
-@pytest.mark.parametrize("kind", ["i64", "i32", "f64", "f32", "dec", "bool", "days", "skewed", "constant", "nulls"])
+@pytest.mark.parametrize("kind", ["i64", "i32", "f64", "f32", "dec", "bool", "flag", "days", "skewed", "constant", "nulls",
+                                  "f64_nulls", "f32_nulls", "dec_nulls", "bool_nulls"])
 @pytest.mark.parametrize("limit,offset", [(1, 0), (100, 0), (1500, 400), (15_000, 3)])
 def test_kinds(gpu, kind, limit, offset):
     print(f"[case] sampled limit {kind} {limit} {offset}", flush=True)
     n = 1_100_003
     rng = np.random.default_rng(limit)
+    valid = rng.random(n) > 0.001 if kind.endswith("nulls") else None
     if kind == "i64":
         col = both(rng.integers(-(1 << 62), 1 << 62, n), N.I64)
     elif kind == "i32":
@@ -39,12 +42,18 @@ def test_kinds(gpu, kind, limit, offset):
         v[rng.integers(0, n, 60)] = np.nan
         v[rng.integers(0, n, 60)] = -np.inf
         col = both(v, N.F64)
-    elif kind == "f32":
-        col = both(rng.standard_normal(n).astype(np.float32), N.F32)
-    elif kind == "dec":
+    elif kind.startswith("f32"):
+        col = both(rng.standard_normal(n).astype(np.float32), N.F32, valid)
+    elif kind == "f64_nulls":
+        col = both(rng.standard_normal(n), N.F64, valid)
+    elif kind.startswith("dec"):
         lo = rng.integers(-(1 << 62), 1 << 62, n)
-        col = both(np.stack([lo, rng.integers(-3, 3, n)], 1), N.DEC128)
-    elif kind == "bool":
+        col = both(np.stack([lo, rng.integers(-3, 3, n) if kind == "dec" else rng.integers(-(1 << 40), 1 << 40, n)], 1),
+                   N.DEC128, valid)
+    elif kind.startswith("bool"):  # one in 200: the bound of 1900 rows holds them, the others' bounds decline
+        flag = rng.random(n) < 0.005
+        col = (DeviceColumn.from_numpy(flag.astype(np.uint8), N.BOOL, valid), both(flag.astype(np.int32), N.I32, valid)[1])
+    elif kind == "flag":
         col = both((rng.random(n) < 0.0001).astype(np.int32), N.I32)
     elif kind == "days":
         col = both(rng.integers(0, 2500, n).astype(np.int32), N.DATE32)
@@ -53,7 +62,7 @@ def test_kinds(gpu, kind, limit, offset):
     elif kind == "constant":
         col = both(np.full(n, 5, np.int64), N.I64)
     else:
-        col = both(rng.integers(0, 1 << 40, n), N.I64, rng.random(n) > 0.001)
+        col = both(rng.integers(0, 1 << 40, n), N.I64, valid)
     for desc in (False, True):
         _check([col], [desc], [desc], limit, offset)
 
