@@ -1378,10 +1378,11 @@ static int groupby_run(bolt_stream_t stream, const bolt_column_t* keys, int32_t 
     }
     hipError_t le = hipGetLastError();
     uint32_t eh[4] = {0, 0, 0, 0}, terr[4] = {0, 0, 0, 0};
-    st = le == hipSuccess ? read_back(s, {{eh, emisc, 16}, {terr, t.err, 16}}) : BOLT_ERR_DEVICE;
+    st = le == hipSuccess ? read_back(s, {{eh, emisc, 16}, {terr, t.err, 16}})
+                          : set_error(BOLT_ERR_DEVICE, "GROUP BY extraction failed: %s", hipGetErrorString(le));
     if (st != BOLT_OK) {
       bolt_table_release(tbl);
-      return set_error(BOLT_ERR_DEVICE, "GROUP BY extraction failed: %s", hipGetErrorString(le));
+      return st;
     }
     if (terr[0]) {  // the global table overflowed: discard this result and rerun larger
       bolt_table_release(tbl);
