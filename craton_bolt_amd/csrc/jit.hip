@@ -953,16 +953,17 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
   return o.str();
 }
 
-// Key partition of a GROUP BY's input.  Workgroup c walks chunk c (rows
-// [c * per, (c + 1) * per)) in tiles of kGbPartTile rows; a row that passes the
-// filter goes to the partition of the top 8 bits of its key's hash (a row of
-// the NULL group to any, by its position).  mode 0: counts[c][p] = rows of the
-// chunk in partition p, and the keys' HyperLogLog registers in `hll` (from the
-// hash bits below the partition's).  mode 1: `counts` holds where the chunk's rows of each
-// partition start, and the columns are copied there, in row order: a tile is
-// ranked per partition in LDS, and each column in turn is staged in LDS in
-// partition order and written as runs.  Bound by the copies' traffic: no
-// atomics outside LDS, no look-back, and the layout does not depend on timing.
+// Key partition of a GROUP BY's input.  Workgroup c walks chunk c (rows [c * per,
+// (c + 1) * per)) in tiles of kGbPartTile rows; a row that passes the filter goes
+// to the partition of the top 8 bits of its key's hash (a row of the NULL group to
+// any, by its position).  mode 0: counts[c][p] = rows of the chunk in partition p,
+// and the keys' HyperLogLog registers in `hll` (from the hash bits below the
+// partition's).  mode 1: `counts` holds where the chunk's rows of each partition
+// start, and the columns are copied there, tile by tile: a tile is ranked per
+// partition in LDS, and each column in turn is staged in LDS in partition order
+// and written as runs.  Bound by the copies' traffic: no atomics outside LDS, no
+// look-back.  Where a tile's rows of a partition lie is fixed; their order there
+// is that of the LDS atomics.
 std::string jit_gb_partition_source(const GbJitSpec& sp, const std::vector<int>& copied) {
   std::ostringstream o;
   const int R = kGbPartTile / 1024;
