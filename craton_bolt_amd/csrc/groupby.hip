@@ -129,6 +129,13 @@ constexpr int64_t kGbPartMinRows = (int64_t)1 << 21;
 // errors of the count more and the fullest partition's excess are below 0.7
 // full, where every key finds a slot within kPartProbes.
 constexpr double kGbPartLoad = 0.6;
+// How full the plain path's LDS tables are where the partition begins to pay.  The
+// rows that they spill there are few, against a copy of all rows: two float sums
+// by an int32 key, plain / partitioned in us, 10M rows 0.8 full 501 / 423, 1.0
+// full 709 / 424; 50M rows 0.8 full 624 / 1308, 0.9 836 / 1311, 1.0 1783 / 1331,
+// 1.1 2070 / 1321 (by two int32 keys 667 / 1615, 717 / 1585, 1556 / 1583, 2037 /
+// 1596).
+constexpr double gb_part_full(int64_t n) { return n <= (int64_t)1 << 24 ? 0.75 : 1.0; }
 
 // One workgroup: distinct keys among kGbSample stratified rows that pass the
 // filter.  out = {rows with a regular key, distinct keys, most frequent key's
@@ -895,10 +902,11 @@ static int gb_part_wanted(hipStream_t s, const KeySpec& ks, const DevFilter& f, 
   BOLT_HIP(hipGetLastError());
   BOLT_TRY(read_back(s, {{h, out.ptr, 12}}));
   // few sampled rows pass the filter: the plain path; a key above 0.4% of the
-  // rows (its share of 1/256) would make one workgroup the last; twice the limit
-  // leaves the sample's error to the count
+  // rows (its share of 1/256) would make one workgroup the last; above 1.2 times
+  // the limit an attempt, which costs 110 us where the count ends it, rarely holds
   const double est = sample_groups(h[0], h[1]);
-  *yes = h[0] >= kGbSample / 4 && est > 0.75 * S && est <= 2 * part_groups_most(part_S) && h[2] <= 8 + h[0] / 256;
+  *yes = h[0] >= kGbSample / 4 && est > gb_part_full(n) * S && est <= 1.2 * part_groups_most(part_S) &&
+         h[2] <= 8 + h[0] / 256;
   return BOLT_OK;
 }
 

@@ -836,6 +836,7 @@ std::string jit_gb_lds_source(const GbJitSpec& sp) {
        "    const void* __restrict__ k1p, const unsigned char* __restrict__ k1v, bolt::JitLits lits,\n"
        "    bolt::JitCols cols, bolt::PartOut out, const unsigned int* __restrict__ ranges) {\n"
        "  using namespace bolt;\n"
+       "  if (ranges && ranges[" << (1 << kGbPartBits) << "] == 0) return;  // no rows, or too many groups\n"
        "  extern __shared__ u64_t sm[];\n"
        "  const int SS = S + 2;\n"
        "  u64_t* skeys = sm;\n"

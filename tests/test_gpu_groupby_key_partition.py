@@ -134,8 +134,7 @@ def test_more_groups_than_the_tables(gpu):
 # probe left keys without one, and the whole call ran again on the plain path.
 @pytest.mark.parametrize("kind", ["i64", "i32", "pair"])
 @pytest.mark.parametrize("groups", [300_000, 500_000, 700_000, 930_000])
-def test_every_group_finds_a_slot(gpu, monkeypatch, kind, groups):
-    monkeypatch.delenv("BOLT_GB_KEY_PARTITION")
+def test_every_group_finds_a_slot(gpu, kind, groups):
     n = 2_200_000
     print(f"[case] key partition {kind} groups={groups}", flush=True)
     rng = np.random.default_rng(groups)
@@ -151,10 +150,9 @@ def test_every_group_finds_a_slot(gpu, monkeypatch, kind, groups):
 
 
 @pytest.mark.parametrize("few", [0, 10_000])
-def test_too_many_groups_are_counted(gpu, monkeypatch, few):
+def test_too_many_groups_are_counted(gpu, few):
     """More groups than the tables take, by themselves or behind a few frequent ones (which a sample takes
     for all): the count ends the partition, and the plain path answers."""
-    monkeypatch.delenv("BOLT_GB_KEY_PARTITION")
     n, many = 2_400_000, 1_300_000
     print(f"[case] key partition declined few={few}", flush=True)
     rng = np.random.default_rng(8)
@@ -164,6 +162,22 @@ def test_too_many_groups_are_counted(gpu, monkeypatch, few):
     run_both([(g * 0x9E3779B97F4A7, N.I64, None)], [(rng.normal(size=n), N.F64, None)], [(N.SUM, 0), (N.COUNT_STAR, 0)],
              [N.I64])
     assert groupby_last_plan()["spilled_rows"] > 0
+
+
+@pytest.mark.parametrize("n,groups,parted", [((1 << 24) + 1, 3300, False), ((1 << 24) + 1, 4300, True),
+                                             (2_200_000, 3300, True)])
+def test_nearly_full_tables(gpu, monkeypatch, n, groups, parted):
+    """Two words leave the plain path's tables 3752 slots: above 2^24 rows the partition begins where the groups
+    fill them.  It has one partial record per group, the plain path one per workgroup and group."""
+    monkeypatch.delenv("BOLT_GB_KEY_PARTITION")
+    print(f"[case] key partition n={n} groups={groups}", flush=True)
+    k = np.random.default_rng(groups).integers(0, groups, n).astype(np.int32)
+    v = (np.arange(n) % 1000).astype(np.float64)  # sums below 2^53 are exact in any order
+    got = execute_groupby([DeviceColumn.from_numpy(k)], [DeviceColumn.from_numpy(v)], [(N.SUM, 0), (N.COUNT_STAR, 0)])
+    assert (groupby_last_plan()["partial_records"] == groups) == parted
+    assert np.array_equal(got["keys"][0][0], np.arange(groups))
+    assert np.array_equal(got["aggs"][0][0], np.bincount(k, v, groups))
+    assert np.array_equal(got["aggs"][1][0], np.bincount(k, minlength=groups))
 
 
 _PEAK = """
