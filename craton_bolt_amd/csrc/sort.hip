@@ -905,7 +905,7 @@ __global__ void order_key_kernel(const void* __restrict__ d, const uint8_t* __re
 // value is its signed high word, then its low word), each an unsigned image that
 // ascends along the order.  The fields' images, less their smallest value, are
 // packed most significant first into one 64-bit key, so a single sort orders all
-// columns: 0.73 ms for a nullable date and a float over 5M rows, where one sort
+// columns: 0.74 ms for a nullable date and a float over 5M rows, where one sort
 // per field, each reading its column through the permutation so far, took 1.60 ms.
 // When the fields need more than 64 bits the last one that fits is cut.  Rows that
 // agree on all 64 bits are then put in order run by run where the runs are short
