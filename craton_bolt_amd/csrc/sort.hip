@@ -13,9 +13,10 @@
 //     earlier tiles per digit for its global offsets (decoupled look-back,
 //     one digit per thread), reorders the tile by digit in LDS and writes
 //     runs of equal digits with coalesced stores;
-//   * up to 2^23 rows, and up to 2^25 where the top digits are uneven, the
-//     buckets come from a sample of the keys instead (sort_split.h);
-//   * passes whose digit is constant over the whole input are skipped;
+//   * passes whose digit is constant over the whole input are skipped; keys in
+//     which few digits vary take a pass per digit (sort_by_bytes);
+//   * others, up to 2^23 rows, and up to 2^25 where the top digits are uneven,
+//     get buckets from a sample of the keys instead (sort_split.h);
 //   * for larger inputs with three or more varying digits the sort is hybrid
 //     (MSD-grouped, LSD-finished): only the two most significant varying
 //     digits get global onesweep passes; they leave up to 65536 contiguous

@@ -25,7 +25,7 @@
 namespace bolt {
 
 constexpr int64_t kSplitMax = (int64_t)1 << 25;    // above: the digit hybrid (its buckets are 16 bits of digits)
-constexpr int64_t kSplitFirst = (int64_t)1 << 23;  // up to here without a look at the keys' digits
+constexpr int64_t kSplitFirst = (int64_t)1 << 23;  // above: a histogram of the keys' bytes first
 constexpr int64_t kSplitOnePass = (int64_t)1 << 17;  // up to here 256 buckets of 512 rows on average
 constexpr int kCodeBlock = 1024;
 
